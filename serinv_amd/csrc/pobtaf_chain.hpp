@@ -71,9 +71,8 @@ struct PobtafChain {
 };
 
 // Timeline events of the fused chain step g (diagnostic builds of a run):
-//   0 step start, 1 factorization done, 2 PX(g)/PD(g+1) staged,
-//   3 column blocks 0-2 and Linv(g) done, 4 L(g+1,g) complete, 5 step end,
-//   6 PX(g) published (by its helper), 7 L(g+2,g) published (by its helper).
+//   0 step start, 1 factorization done, 2 Linv(g) released, PX(g)/PD(g+1)
+//   staged, 3 L(g+1,g) complete, 5 step end, 6 PX(g) published (by its helper), 7 L(g+2,g) published (by its helper).
 constexpr int CHAIN_TRACE_EV = 8;
 __device__ __forceinline__ void chain_trace(const PobtafChain& P, int g, int e) {
   if (P.trace && threadIdx.x == 0)
@@ -657,11 +656,10 @@ __device__ __forceinline__ void chain_run(const PobtafChain& P, double* S, doubl
     const int* f_px = P.hflags + t_px(P, g);
     const int* f_pd = pre ? P.hflags + t_pd(P, g + 1) : f_px;
     // Full tiles: the inverse Linv(g) is formed by 16-row block rows while
-    // the tile is factored.  Block row I needs only panels 0 .. I, so waves
-    // 1-3 form block rows 0, 1, 2 while wave 0 factors panels 1, 2, 3
-    // (X_II by forward substitution, X_IJ = -X_II sum_K L_IK X_KJ on MFMA);
-    // block row 3 follows the factorization.  A wave that needs X_22 or X_33
-    // before another wave's copy is visible forms its own copy in Ws.
+    // the tile is factored.  Its diagonal blocks X_II come with the panels;
+    // the rest of block row I needs only panels 0 .. I, so waves 2 and 3
+    // form X_IJ = -X_II sum_K L_IK X_KJ (MFMA) of block rows 1 and 2 while
+    // wave 0 factors panels 2 and 3; block row 3 follows the factorization.
     // PX(g) and PD(g+1) are normally published while the tile is factored.
     // Wave 1 checks their flags while wave 0 factors the last panel and, if
     // both are set, acquires; every thread then loads its parts of the two
@@ -670,13 +668,8 @@ __device__ __forceinline__ void chain_run(const PobtafChain& P, double* S, doubl
     {
       const int64_t row0 = (int64_t)(g / P.nt) * P.b + (int64_t)(g % P.nt) * CT;
       if (m == CT) {
-        lds_potrf_t<CT>(S2, CT, P.info, row0, [&](int p) {
-          if (p == 0 && wave == 3) wave_diag_inv16(S2, X2, 0);
-          if (p == 16 && wave == 2) {
-            wave_diag_inv16(S2, X2, 16);
-            __builtin_amdgcn_wave_barrier();
-            wave_trtri_offdiag(S2, X2, &X2[16][16], TT_LD, 1, 0);
-          }
+        lds_potrf_t<CT>(S2, X2, CT, P.info, row0, [&](int p) {
+          if (p == 16 && wave == 2) wave_trtri_offdiag(S2, X2, &X2[16][16], TT_LD, 1, 0);
           if (p == 32) {
             if (wave == 1) {
               int ok = sub ? (__hip_atomic_load(f_px, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) &
@@ -686,19 +679,15 @@ __device__ __forceinline__ void chain_run(const PobtafChain& P, double* S, doubl
               if (ok) __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
               if (lane == 0) s_early = ok;
             } else if (wave == 2) {
-              wave_diag_inv16(S2, X2, 32);
-              __builtin_amdgcn_wave_barrier();
               wave_trtri_offdiag(S2, X2, &X2[32][32], TT_LD, 2, 1);
             } else {
-              wave_diag_inv16_to(S2, 32, Ws, WS_LD);
-              __builtin_amdgcn_wave_barrier();
-              wave_trtri_offdiag(S2, X2, Ws, WS_LD, 2, 0);
+              wave_trtri_offdiag(S2, X2, &X2[32][32], TT_LD, 2, 0);
             }
           }
         });
       } else {
         if (tid == 0) s_early = 0;
-        lds_potrf_t<0>(S2, m, P.info, row0);
+        lds_potrf_t<0>(S2, X2, m, P.info, row0);
       }
     }
     const int early = s_early;
@@ -737,15 +726,8 @@ __device__ __forceinline__ void chain_run(const PobtafChain& P, double* S, doubl
       seen = __hip_atomic_load(f_px, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) &
              __hip_atomic_load(f_pd, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     if (m == CT) {
-      // block row 3: X_33 on waves 0-2 (wave 0's copy is the result), then
-      // X_32, X_31, X_30
-      if (wave < 3) {
-        double* xi = (wave == 0) ? &X2[48][48] : Ws + 16 * wave * WS_LD;
-        const int ldi = (wave == 0) ? TT_LD : WS_LD;
-        wave_diag_inv16_to(S2, 48, xi, ldi);
-        __builtin_amdgcn_wave_barrier();
-        wave_trtri_offdiag(S2, X2, xi, ldi, 3, 2 - wave);
-      }
+      // block row 3: X_32, X_31, X_30
+      if (wave < 3) wave_trtri_offdiag(S2, X2, &X2[48][48], TT_LD, 3, 2 - wave);
       __syncthreads();
     } else {
       lds_trtri<false>(S2, X2, W2, m);
@@ -828,20 +810,96 @@ __device__ __forceinline__ void chain_run(const PobtafChain& P, double* S, doubl
 }
 
 
-// Column block J of L(g+1,g) = PX(g) Linv(g)^T (rows 0..63, K < 16J + 16),
-// with a compile-time trip count so that the LDS operand loads are
-// scheduled ahead of the products.  ACC f64x4: FP64 MFMA; f32x4: FP32.
-template <int J, typename ACC>
-__device__ __forceinline__ void chain_colblock(const double* Ps, const double (*X2)[TT_LD],
-                                               ACC (&cb)[4]) {
+// Rows r0 .. r0 + 15 of Ps (64 x 64, K-contiguous) <- Ps Linv^T, by the calling
+// wave, in place: column block J takes K < 16 J + 16 (Linv is lower
+// triangular), 40 MFMA steps on four accumulators, each operand of Ps read
+// once.  ACC f64x4: FP64 MFMA; f32x4: FP32 products.
+template <typename ACC>
+__device__ __forceinline__ void chain_trsm_rows(double* Ps, const double (*X2)[TT_LD], int r0) {
   const int lane = threadIdx.x & 63, li = lane & 15, lk = lane >> 4;
+  ACC c[4];
 #pragma unroll
-  for (int rb = 0; rb < 4; ++rb) cb[rb] = ACC{0, 0, 0, 0};
+  for (int J = 0; J < 4; ++J) c[J] = ACC{0, 0, 0, 0};
+  const double* pa = Ps + (r0 + li) * TT_LD + lk;
+  const double* pb = &X2[li][lk];
 #pragma unroll
-  for (int kk = 0; kk < 16 * J + 16; kk += 4) {
-    const double bv = X2[16 * J + li][kk + lk];
+  for (int kk = 0; kk < CT; kk += 4) {
+    const double av = pa[kk];
 #pragma unroll
-    for (int rb = 0; rb < 4; ++rb) cb[rb] = mfma_acc(Ps[(16 * rb + li) * TT_LD + kk + lk], bv, cb[rb]);
+    for (int J = kk / 16; J < 4; ++J) c[J] = mfma_acc(av, pb[16 * J * TT_LD + kk], c[J]);
+  }
+  __builtin_amdgcn_wave_barrier();
+#pragma unroll
+  for (int J = 0; J < 4; ++J)
+#pragma unroll
+    for (int r = 0; r < 4; ++r)
+      Ps[(r0 + acc_row(c[J], lane, r)) * TT_LD + 16 * J + acc_col(lane)] = (double)c[J][r];
+}
+
+// The ten lower 16 x 16 blocks of a 64-tile dealt to the four waves (3, 3, 2,
+// 2): block i of the calling wave, i < chain_nblk().
+__device__ __forceinline__ int chain_nblk(int wave) { return wave < 2 ? 3 : 2; }
+__device__ __forceinline__ void chain_blk(int wave, int i, int& rb, int& cb) {
+  rb = wave == 0 ? (i > 0 ? 1 : 0) : (wave == 1 ? 2 : 3);
+  cb = wave == 0 ? (i == 2 ? 1 : 0) : (wave == 3 ? i + 2 : i);
+}
+
+// The calling wave's blocks of tile t (full tile), in the accumulator layout
+// of ACC.
+template <typename ACC>
+__device__ __forceinline__ void chain_pd_load(const CTile& t, int wave, f64x4 (&pd)[3]) {
+  const int lane = threadIdx.x & 63;
+#pragma unroll
+  for (int i = 0; i < 3; ++i) {
+    if (i >= chain_nblk(wave)) break;
+    int rb, cb;
+    chain_blk(wave, i, rb, cb);
+#pragma unroll
+    for (int r = 0; r < 4; ++r)
+      pd[i][r] = t.p[(int64_t)(16 * rb + acc_row(ACC{}, lane, r)) * t.ld + 16 * cb + acc_col(lane)];
+  }
+}
+
+// The calling wave's blocks of Sn <- pd - Ps Ps^T.
+template <typename ACC>
+__device__ __forceinline__ void chain_syrk(const double* Ps, const f64x4 (&pd)[3], int wave,
+                                           double* Sn) {
+  const int lane = threadIdx.x & 63, li = lane & 15, lk = lane >> 4;
+  const int nblk = chain_nblk(wave);
+  ACC acc[3];
+  const double* pa[3];
+  const double* pb[3];
+#pragma unroll
+  for (int i = 0; i < 3; ++i) {
+    int rb, cb;
+    chain_blk(wave, i, rb, cb);
+    pa[i] = Ps + (16 * rb + li) * TT_LD + lk;
+    pb[i] = Ps + (16 * cb + li) * TT_LD + lk;
+    acc[i] = ACC{0, 0, 0, 0};
+    if constexpr (sizeof(ACC) == sizeof(f64x4)) acc[i] = pd[i];
+  }
+  if (nblk == 3) {
+#pragma unroll
+    for (int kk = 0; kk < CT; kk += 4)
+#pragma unroll
+      for (int i = 0; i < 3; ++i) acc[i] = mfma_acc(-pa[i][kk], pb[i][kk], acc[i]);
+  } else {
+#pragma unroll
+    for (int kk = 0; kk < CT; kk += 4)
+#pragma unroll
+      for (int i = 0; i < 2; ++i) acc[i] = mfma_acc(-pa[i][kk], pb[i][kk], acc[i]);
+  }
+#pragma unroll
+  for (int i = 0; i < 3; ++i) {
+    if (i >= nblk) break;
+    int rb, cb;
+    chain_blk(wave, i, rb, cb);
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      double v = (double)acc[i][r];
+      if constexpr (sizeof(ACC) != sizeof(f64x4)) v += pd[i][r];
+      Sn[(16 * rb + acc_row(acc[i], lane, r)) * TT_LD + 16 * cb + acc_col(lane)] = v;
+    }
   }
 }
 
@@ -849,32 +907,25 @@ __device__ __forceinline__ void chain_colblock(const double* Ps, const double (*
 // Chain schedule for matrices whose diagonal tiles are all full (b % 64 ==
 // 0).  Step g starts with D(g,g) fully updated in S and:
 //   1. factors it (wave 0 factors the 16-column panels; waves 1-3 update the
-//      trailing columns and form block rows 0-2 of Linv(g) beside them);
-//   2. with PX(g) staged in Ps, waves 1-3 form column blocks 0-2 of
-//      L(g+1,g) = PX(g) Linv(g)^T (column block J needs only block row J of
-//      Linv, already formed), while wave 0 forms X_33 = L(g,g)[48:64,48:64]^{-1};
-//   3. forms column block 3 by substitution (every wave 16 rows):
-//        L(g+1,g)[:, 48:64] = (PX(g)[:, 48:64] - L(g+1,g)[:, 0:48] L(g,g)[48:64, 0:48]^T) X_33^T,
-//      and waves 1-3 then form X_30, X_31, X_32, the rest of Linv's block row 3;
-//   4. D(g+1,g+1) = PD(g+1) - L(g+1,g) L(g+1,g)^T on waves 0, 2, 3 (the lower
-//      quadrants) into the other D buffer.
-// Wave 1 stores Linv(g) after step 3 and releases it during step 4, where
-// it has no quadrant; L(g+1,g) is released at the start of step g+1, whose
-// first panel only wave 0 works on.  In the mixed mode the products
-// (column blocks, the column-block-3 update and its X_33 product, the syrk)
-// round their operands to FP32 and accumulate in FP32; the differences and
-// the PD(g+1) term stay FP64.
+//      trailing columns and form block rows 1 and 2 of Linv(g) beside them;
+//      the diagonal blocks of Linv(g) come with the panels);
+//   2. completes Linv(g) (block row 3), stores it and releases it: the helpers
+//      wait for it first;
+//   3. with PX(g) staged in Ps, L(g+1,g) = PX(g) Linv(g)^T, 16 rows per wave;
+//   4. D(g+1,g+1) = PD(g+1) - L(g+1,g) L(g+1,g)^T on its lower 16 x 16
+//      blocks, into the other D buffer.
+// L(g+1,g) is released at the start of step g+1, whose first panel only wave
+// 0 works on.  In the mixed mode the products of steps 3 and 4 round their
+// operands to FP32 and accumulate in FP32; the PD(g+1) term stays FP64.
 // LDS: two D buffers [64][65] (D(g,g) -> L(g,g), and D(g+1,g+1)), Xs
-// [64][65] (Linv(g)), Ws [64][17] (scratch), Ps [64][65] (PX(g) -> L(g+1,g),
-// row-major = K-contiguous).
+// [64][65] (Linv(g)), Ps [64][65] (PX(g) -> L(g+1,g), row-major =
+// K-contiguous).
 template <int TAG>
 __device__ __forceinline__ void chain_run_fused(const PobtafChain& P, double* Sa, double* Sb,
-                                                double* Xs, double* Ws, double* Ps) {
+                                                double* Xs, double* Ps) {
   const int tid = threadIdx.x;
   double (*X2)[TT_LD] = reinterpret_cast<double (*)[TT_LD]>(Xs);
-  const int lane = tid & 63, wave = tid >> 6;
-  const int wm = (wave >> 1) * 32, wn = (wave & 1) * 32;
-  const int li = lane & 15, lk = lane >> 4;
+  const int lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int rs = tid >> 5, c2 = (tid & 31) * 2;
   constexpr int PUB = 64;  // wave 1, lane 0: runs the releases
   for (int idx = tid; idx < CT * TT_LD; idx += CH_THREADS) Xs[idx] = 0.0;
@@ -884,9 +935,8 @@ __device__ __forceinline__ void chain_run_fused(const PobtafChain& P, double* Sa
     cacc_to_lds(acc, Sa, TT_LD);
   }
   __syncthreads();
-  f64x4 pd_next[2][2];
   __shared__ int s_early;
-  int pending = -1;  // step whose Linv and L(g+1,g) stores wait for their release
+  int pending = -1;  // step whose L(g+1,g) stores wait for their release
   double* S = Sa;
   double* Sn = Sb;
   for (int g = 0; g < P.NT; ++g) {
@@ -904,16 +954,11 @@ __device__ __forceinline__ void chain_run_fused(const PobtafChain& P, double* Sa
     }
     pending = -1;
     chain_trace(P, g, 0);
-    // 1. factorization with Linv block rows 0-2 beside it; PX(g) and
+    // 1. factorization with Linv block rows 1 and 2 beside it; PX(g) and
     //    PD(g+1) flags checked by wave 1 during the last panel
     const int64_t row0 = (int64_t)(g / P.nt) * P.b + (int64_t)(g % P.nt) * CT;
-    lds_potrf_t<CT>(S2, CT, P.info, row0, [&](int p) {
-      if (p == 0 && wave == 3) wave_diag_inv16(S2, X2, 0);
-      if (p == 16 && wave == 2) {
-        wave_diag_inv16(S2, X2, 16);
-        __builtin_amdgcn_wave_barrier();
-        wave_trtri_offdiag(S2, X2, &X2[16][16], TT_LD, 1, 0);
-      }
+    lds_potrf_t<CT>(S2, X2, CT, P.info, row0, [&](int p) {
+      if (p == 16 && wave == 2) wave_trtri_offdiag(S2, X2, &X2[16][16], TT_LD, 1, 0);
       if (p == 32) {
         if (wave == 1) {
           int ok = sub ? (__hip_atomic_load(f_px, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) &
@@ -922,21 +967,49 @@ __device__ __forceinline__ void chain_run_fused(const PobtafChain& P, double* Sa
           ok = __builtin_amdgcn_readfirstlane(ok);
           if (ok) __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
           if (lane == 0) s_early = ok;
-        } else if (wave == 2) {
-          wave_diag_inv16(S2, X2, 32);
-          __builtin_amdgcn_wave_barrier();
-          wave_trtri_offdiag(S2, X2, &X2[32][32], TT_LD, 2, 1);
         } else {
-          wave_diag_inv16_to(S2, 32, Ws, WS_LD);
-          __builtin_amdgcn_wave_barrier();
-          wave_trtri_offdiag(S2, X2, Ws, WS_LD, 2, 0);
+          wave_trtri_offdiag(S2, X2, &X2[32][32], TT_LD, 2, wave == 2 ? 1 : 0);
         }
       }
     });
     const int early = s_early;
     chain_trace(P, g, 1);
-    // L(g,g) to memory, upper triangle zero (16-byte stores)
+    // PX(g) and PD(g+1), if both were published during the factorization: the
+    // loads land during step 2
+    const CTile xt = tile_g(P, g + 1, g);
+    TileRegs16 rx;
+    f64x4 pd[3];
+    auto load_px = [&]() {
+      tile_load16(xt, rx);
+      if (P.f32)
+        chain_pd_load<f32x4>(tile_g(P, g + 1, g + 1), wave, pd);
+      else
+        chain_pd_load<f64x4>(tile_g(P, g + 1, g + 1), wave, pd);
+    };
+    auto stage_px = [&]() {  // pitch 65: 8-byte stores
+#pragma unroll
+      for (int q = 0; q < 8; ++q) {
+        Ps[(rs + 8 * q) * TT_LD + c2] = rx.v[q].x;
+        Ps[(rs + 8 * q) * TT_LD + c2 + 1] = rx.v[q].y;
+      }
+    };
+    if (early) load_px();
+    // 2. Linv block row 3; L(g,g) to memory, upper triangle zero (16-byte
+    //    stores); Linv(g) to memory
+    if (wave >= 1) wave_trtri_offdiag(S2, X2, &X2[48][48], TT_LD, 3, wave - 1);
+    __syncthreads();
+    double* li_out = P.linv + (int64_t)g * CT * CT;
     {
+      cdbl2 v[8];
+#pragma unroll
+      for (int q = 0; q < 8; ++q) {
+        v[q].x = X2[rs + 8 * q][c2];
+        v[q].y = X2[rs + 8 * q][c2 + 1];
+      }
+#pragma unroll
+      for (int q = 0; q < 8; ++q) *reinterpret_cast<cdbl2*>(li_out + (rs + 8 * q) * CT + c2) = v[q];
+    }
+    auto store_l = [&]() {
       cdbl2 v[8];
 #pragma unroll
       for (int q = 0; q < 8; ++q) {
@@ -947,180 +1020,43 @@ __device__ __forceinline__ void chain_run_fused(const PobtafChain& P, double* Sa
 #pragma unroll
       for (int q = 0; q < 8; ++q)
         *reinterpret_cast<cdbl2*>(dt.p + (int64_t)(rs + 8 * q) * dt.ld + c2) = v[q];
-    }
-    double* li_out = P.linv + (int64_t)g * CT * CT;
-    if (!sub) {
-      // last diagonal tile of the matrix: Linv block row 3 and its release
-      if (wave < 3) {
-        double* xi = (wave == 0) ? &X2[48][48] : Ws + 16 * wave * WS_LD;
-        const int ldi = (wave == 0) ? TT_LD : WS_LD;
-        wave_diag_inv16_to(S2, 48, xi, ldi);
-        __builtin_amdgcn_wave_barrier();
-        wave_trtri_offdiag(S2, X2, xi, ldi, 3, 2 - wave);
-      }
-      __syncthreads();
-      cdbl2 v[8];
-#pragma unroll
-      for (int q = 0; q < 8; ++q) {
-        v[q].x = X2[rs + 8 * q][c2];
-        v[q].y = X2[rs + 8 * q][c2 + 1];
-      }
-#pragma unroll
-      for (int q = 0; q < 8; ++q) *reinterpret_cast<cdbl2*>(li_out + (rs + 8 * q) * CT + c2) = v[q];
+    };
+    if (!sub) {  // last diagonal tile of the matrix
+      store_l();
       chain_publish(P.cflags + 2 * g);
       continue;
     }
-    // PX(g) and PD(g+1): loaded now if both were published during the
-    // factorization, else each wave waits for them itself
-    const CTile xt = tile_g(P, g + 1, g);
-    TileRegs16 rx;
-    if (!early) wave_wait(P, f_px, f_pd);
-    tile_load16(xt, rx);
-    cacc_load(tile_g(P, g + 1, g + 1), pd_next);
-    // Ps[m][k] = PX(g)(m, k) (pitch 65: 8-byte stores)
-#pragma unroll
-    for (int q = 0; q < 8; ++q) {
-      Ps[(rs + 8 * q) * TT_LD + c2] = rx.v[q].x;
-      Ps[(rs + 8 * q) * TT_LD + c2 + 1] = rx.v[q].y;
-    }
+    if (early) stage_px();
+    wave_stores_done();
     __syncthreads();
+    if (tid == PUB) {
+      __builtin_amdgcn_fence(__ATOMIC_RELEASE, "agent");
+      wave_stores_done();
+      __hip_atomic_store(P.cflags + 2 * g, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    }
+    if (!early) {
+      wave_wait(P, f_px, f_pd);
+      load_px();
+      stage_px();
+      __syncthreads();
+    }
     chain_trace(P, g, 2);
-    // 2. wave 0: X_33 = L(g,g)[48:64, 48:64]^{-1};
-    //    wave J+1: column block J of L(g+1,g) = sum over k < 16J + 16 of
-    //    PX(:, k) Linv(16J + n, k)
-    f64x4 cb[4];
-    f32x4 cb32[4];
-    if (wave == 0) {
-      wave_diag_inv16(S2, X2, 48);
-    } else if (!P.f32) {
-      if (wave == 1) chain_colblock<0>(Ps, X2, cb);
-      else if (wave == 2) chain_colblock<1>(Ps, X2, cb);
-      else chain_colblock<2>(Ps, X2, cb);
-    } else {
-      if (wave == 1) chain_colblock<0>(Ps, X2, cb32);
-      else if (wave == 2) chain_colblock<1>(Ps, X2, cb32);
-      else chain_colblock<2>(Ps, X2, cb32);
-    }
-    __syncthreads();  // every read of PX(g)'s column blocks 0-2 is done; X_33 is visible
-    if (wave >= 1) {
-      const int J = wave - 1;
-#pragma unroll
-      for (int rb = 0; rb < 4; ++rb)
-#pragma unroll
-        for (int r = 0; r < 4; ++r) {
-          if (!P.f32)
-            Ps[(16 * rb + acc_row_f64(lane, r)) * TT_LD + 16 * J + acc_col(lane)] = cb[rb][r];
-          else
-            Ps[(16 * rb + acc_row_f32(lane, r)) * TT_LD + 16 * J + acc_col(lane)] = (double)cb32[rb][r];
-        }
-    }
-    __syncthreads();  // column blocks 0-2 of L(g+1,g) in Ps
+    // 3. L(g+1,g), wave w: rows 16w .. 16w + 15
+    if (P.f32)
+      chain_trsm_rows<f32x4>(Ps, X2, 16 * wave);
+    else
+      chain_trsm_rows<f64x4>(Ps, X2, 16 * wave);
+    __syncthreads();  // L(g+1,g) complete in Ps
     chain_trace(P, g, 3);
-    // 3. column block 3, wave w: rows 16w .. 16w + 15.  Ws receives the
-    //    product L(g+1,g)[:, 0:48] L(g,g)[48:64, 0:48]^T; the operand of the
-    //    X_33 product is PX(g)[:, 48:64] minus it, formed in FP64.
-    {
-      const int r0 = 16 * wave;
-      if (!P.f32) {
-        f64x4 v = {0.0, 0.0, 0.0, 0.0};
-#pragma unroll
-        for (int kk = 0; kk < 48; kk += 4)
-          v = mfma_f64(Ps[(r0 + li) * TT_LD + kk + lk], S[(48 + li) * TT_LD + kk + lk], v);
-#pragma unroll
-        for (int r = 0; r < 4; ++r) Ws[(r0 + acc_row_f64(lane, r)) * WS_LD + acc_col(lane)] = v[r];
-      } else {
-        f32x4 v = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-        for (int kk = 0; kk < 48; kk += 4)
-          v = mfma_acc(Ps[(r0 + li) * TT_LD + kk + lk], S[(48 + li) * TT_LD + kk + lk], v);
-#pragma unroll
-        for (int r = 0; r < 4; ++r)
-          Ws[(r0 + acc_row_f32(lane, r)) * WS_LD + acc_col(lane)] = (double)v[r];
-      }
-      __builtin_amdgcn_wave_barrier();
-      if (!P.f32) {
-        f64x4 y = {0.0, 0.0, 0.0, 0.0};
-#pragma unroll
-        for (int kk = 0; kk < 16; kk += 4) {
-          const double av = Ps[(r0 + li) * TT_LD + 48 + kk + lk] - Ws[(r0 + li) * WS_LD + kk + lk];
-          y = mfma_f64(av, X2[48 + li][48 + kk + lk], y);
-        }
-#pragma unroll
-        for (int r = 0; r < 4; ++r) Ps[(r0 + acc_row_f64(lane, r)) * TT_LD + 48 + acc_col(lane)] = y[r];
-      } else {
-        f32x4 y = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-        for (int kk = 0; kk < 16; kk += 4) {
-          const double av = Ps[(r0 + li) * TT_LD + 48 + kk + lk] - Ws[(r0 + li) * WS_LD + kk + lk];
-          y = mfma_acc(av, X2[48 + li][48 + kk + lk], y);
-        }
-#pragma unroll
-        for (int r = 0; r < 4; ++r)
-          Ps[(r0 + acc_row_f32(lane, r)) * TT_LD + 48 + acc_col(lane)] = (double)y[r];
-      }
-    }
-    // the rest of Linv's block row 3: wave J+1 forms X_3J
-    if (wave >= 1) wave_trtri_offdiag(S2, X2, &X2[48][48], TT_LD, 3, wave - 1);
-    __syncthreads();  // L(g+1,g) complete in Ps; Linv(g) complete
-    chain_trace(P, g, 4);
-    if (wave == 1) {
-      // Linv(g) to memory by wave 1 alone (released by it in step 4), two
-      // whole rows per store instruction
-      const int hr = lane >> 5, cc = (lane & 31) * 2;
-#pragma unroll 8
-      for (int k = 0; k < 32; ++k) {
-        const int row = 2 * k + hr;
-        cdbl2 v;
-        v.x = X2[row][cc];
-        v.y = X2[row][cc + 1];
-        *reinterpret_cast<cdbl2*>(li_out + row * CT + cc) = v;
-      }
-    }
     lds_tile_store(Ps, TT_LD, xt);
     pending = g;
-    // 4. D(g+1,g+1) = PD(g+1) - L(g+1,g) L(g+1,g)^T on the lower quadrants
-    //    (waves 0, 2, 3) into Sn; wave 1, which has no lower quadrant, waits
-    //    for its Linv(g) stores and releases them
-    f32x4 s32[2][2];
-    cacc32_zero(s32);
-    if (wn <= wm) {
-      if (!P.f32) {
-#pragma unroll
-        for (int kk = 0; kk < CT; kk += 4) {
-          const double a0 = -Ps[(wm + li) * TT_LD + kk + lk];
-          const double a1 = -Ps[(wm + 16 + li) * TT_LD + kk + lk];
-          const double b0 = Ps[(wn + li) * TT_LD + kk + lk];
-          const double b1 = Ps[(wn + 16 + li) * TT_LD + kk + lk];
-          pd_next[0][0] = mfma_f64(a0, b0, pd_next[0][0]);
-          pd_next[0][1] = mfma_f64(a0, b1, pd_next[0][1]);
-          pd_next[1][0] = mfma_f64(a1, b0, pd_next[1][0]);
-          pd_next[1][1] = mfma_f64(a1, b1, pd_next[1][1]);
-        }
-      } else {
-#pragma unroll
-        for (int kk = 0; kk < CT; kk += 4) {
-          const double a0 = -Ps[(wm + li) * TT_LD + kk + lk];
-          const double a1 = -Ps[(wm + 16 + li) * TT_LD + kk + lk];
-          const double b0 = Ps[(wn + li) * TT_LD + kk + lk];
-          const double b1 = Ps[(wn + 16 + li) * TT_LD + kk + lk];
-          s32[0][0] = mfma_acc(a0, b0, s32[0][0]);
-          s32[0][1] = mfma_acc(a0, b1, s32[0][1]);
-          s32[1][0] = mfma_acc(a1, b0, s32[1][0]);
-          s32[1][1] = mfma_acc(a1, b1, s32[1][1]);
-        }
-      }
-    } else {
-      wave_stores_done();
-      if (lane == 0) {
-        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "agent");
-        wave_stores_done();
-        __hip_atomic_store(P.cflags + 2 * g, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-      }
-    }
-    // FP32 products join the FP64 PD(g+1) through Sn (free until below)
-    if (P.f32) acc32_add(s32, pd_next, Sn, TT_LD);
-    cacc_to_lds(pd_next, Sn, TT_LD);
-    wave_stores_done();  // Linv(g), L(g,g), L(g+1,g): released at the start of step g+1
+    // 4. D(g+1,g+1) into Sn
+    if (P.f32)
+      chain_syrk<f32x4>(Ps, pd, wave, Sn);
+    else
+      chain_syrk<f64x4>(Ps, pd, wave, Sn);
+    store_l();
+    wave_stores_done();  // L(g,g), L(g+1,g): released at the start of step g+1
     __syncthreads();
     chain_trace(P, g, 5);
     double* t = S;
@@ -1160,13 +1096,13 @@ __device__ __forceinline__ void chain_helper_task(const PobtafChain& P, int task
     double (*S2)[TT_LD] = reinterpret_cast<double (*)[TT_LD]>(lds);
     cacc_to_lds(acc, lds, TT_LD);
     __syncthreads();
-    lds_potrf(S2, P.a, P.info, (int64_t)P.n * P.b);
+    double (*X2)[TT_LD] = reinterpret_cast<double (*)[TT_LD]>(lds + CT * TT_LD);
+    lds_potrf(S2, X2, P.a, P.info, (int64_t)P.n * P.b);
     for (int idx = tid; idx < P.a * P.a; idx += CH_THREADS) {
       const int rr = idx / P.a, cc = idx % P.a;
       P.T[idx] = (cc <= rr) ? S2[rr][cc] : 0.0;
     }
     if (P.tip_inv) {
-      double (*X2)[TT_LD] = reinterpret_cast<double (*)[TT_LD]>(lds + CT * TT_LD);
       double (*W2)[WS_LD] = reinterpret_cast<double (*)[WS_LD]>(lds + 2 * CT * TT_LD);
       __syncthreads();
       lds_trtri(S2, X2, W2, P.a);
@@ -1223,9 +1159,9 @@ __device__ __forceinline__ void chain_helper_task(const PobtafChain& P, int task
 }
 
 // LDS of the single-matrix kernel: the helper plan (XA, XB) or the chain's
-// (S, Xs, Ws, and Ps for the fused schedule), whichever is larger.
+// (S, Xs, Ws; fused: two D buffers, Xs, Ps), whichever is larger.
 constexpr int CH_LDS_HELPER = 2 * CT * KP + CT * WS_LD;
-constexpr int CH_LDS_FUSED = 4 * CT * TT_LD + CT * WS_LD;
+constexpr int CH_LDS_FUSED = 4 * CT * TT_LD;
 constexpr int CH_LDS = CH_LDS_HELPER > CH_LDS_FUSED ? CH_LDS_HELPER : CH_LDS_FUSED;
 
 __global__ void __launch_bounds__(CH_THREADS) pobtaf_chain_kernel(PobtafChain P) {
@@ -1241,8 +1177,7 @@ __global__ void __launch_bounds__(CH_THREADS) pobtaf_chain_kernel(PobtafChain P)
     if (tid == 0)
       __hip_atomic_store(P.chain_cu, 1 + hw_cu_key(), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     if (P.fused)
-      chain_run_fused<0>(P, lds, lds + CT * TT_LD, lds + 2 * CT * TT_LD, lds + 3 * CT * TT_LD,
-                         lds + 3 * CT * TT_LD + CT * WS_LD);
+      chain_run_fused<0>(P, lds, lds + CT * TT_LD, lds + 2 * CT * TT_LD, lds + 3 * CT * TT_LD);
     else
       chain_run<0>(P, lds, lds + CT * TT_LD, lds + 2 * CT * TT_LD);
     return;

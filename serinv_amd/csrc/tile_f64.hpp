@@ -107,71 +107,169 @@ __device__ __forceinline__ void wave_panel_potrf(double (*S)[TT_LD], int p, int 
     if (act && k < w && p + k <= i) S[i][p + k] = r[k];
 }
 
-// Full-width (16-column) form of the panel Cholesky, p + 16 <= m.  The wave
-// is bound by instruction issue, and most of the issue went into readlane
-// broadcasts of the row entries L(k,j) (two per double).  Here the panel is
-// cut into four 4-column sub-panels:
-//   * inside a sub-panel, right-looking with readlane broadcasts (at most
-//     3 values per pivot);
-//   * a finished sub-panel is written to S; the rows k of later sub-panels
-//     read their four entries L(k, c0..c0+3) back as LDS broadcasts (one
-//     address for all lanes), except the next pivot column c0+4, which
-//     takes readlanes because it is on the dependency path.
-// A non-positive or NaN pivot turns into NaN through the reciprocal square
-// root, so the loop has no branch; the first failing column is recorded
-// once after it.  Lanes above the diagonal of a column hold values that
-// are never read or written back.
-__device__ __forceinline__ void wave_panel_potrf16(double (*S)[TT_LD], int p, int m, int* info,
-                                                   int64_t row0) {
-  const int lane = threadIdx.x & 63;
-  const int i = p + lane;
-  const bool act = i < m;
-  const int ic = act ? i : p;  // clamped row for the loads
-  double r[PW];
+// Value of lane K of each 16-lane row, in every lane of the row.  The wait
+// states in front of a DPP read are written out (here and in row_fmac): the
+// compiler does not track that hazard into an asm statement.
+template <int K>
+__device__ __forceinline__ double row_bcast(double v) {
+  double r;
+  asm volatile("s_nop 1\n\tv_mov_b64_dpp %0, %1 row_newbcast:%2 row_mask:0xf bank_mask:0xf"
+               : "=v"(r)
+               : "v"(v), "n"(K));
+  return r;
+}
+// Lane K of a and of b.
+template <int K>
+__device__ __forceinline__ void row_bcast2(double a, double b, double& ra, double& rb) {
+  asm volatile(
+      "s_nop 1\n\tv_mov_b64_dpp %0, %2 row_newbcast:%4 row_mask:0xf bank_mask:0xf\n\t"
+      "v_mov_b64_dpp %1, %3 row_newbcast:%4 row_mask:0xf bank_mask:0xf"
+      : "=&v"(ra), "=v"(rb)
+      : "v"(a), "v"(b), "n"(K));
+}
+
+// x[K0 + i] -= s[lane K0 + i of the row] * y for i < N: one v_fmac_f64_dpp
+// each, the row broadcast being an operand modifier.  Eight share one wait,
+// which costs as much as two of them.
+#define ROCBTA_FMAC(x, k) \
+  "v_fmac_f64_dpp " x ", -%[s], %[y] row_newbcast:%[k]+" k " row_mask:0xf bank_mask:0xf\n\t"
+#define ROCBTA_IN : [s] "v"(s), [y] "v"(y), [k] "n"(K0)
+template <int K0, int N>
+__device__ __forceinline__ void row_fmac(double (&x)[PW], double s, double y) {
+  if constexpr (N == 1) {
+    asm volatile("s_nop 1\n\t" ROCBTA_FMAC("%0", "0") : "+v"(x[K0]) ROCBTA_IN);
+  } else if constexpr (N == 2) {
+    asm volatile("s_nop 1\n\t" ROCBTA_FMAC("%0", "0") ROCBTA_FMAC("%1", "1")
+                 : "+v"(x[K0]), "+v"(x[K0 + 1]) ROCBTA_IN);
+  } else if constexpr (N == 3) {
+    asm volatile("s_nop 1\n\t" ROCBTA_FMAC("%0", "0") ROCBTA_FMAC("%1", "1") ROCBTA_FMAC("%2", "2")
+                 : "+v"(x[K0]), "+v"(x[K0 + 1]), "+v"(x[K0 + 2]) ROCBTA_IN);
+  } else if constexpr (N >= 4 && N < 8) {
+    asm volatile("s_nop 1\n\t" ROCBTA_FMAC("%0", "0") ROCBTA_FMAC("%1", "1") ROCBTA_FMAC("%2", "2")
+                     ROCBTA_FMAC("%3", "3")
+                 : "+v"(x[K0]), "+v"(x[K0 + 1]), "+v"(x[K0 + 2]), "+v"(x[K0 + 3]) ROCBTA_IN);
+    row_fmac<K0 + 4, N - 4>(x, s, y);
+  } else if constexpr (N >= 8) {
+    asm volatile("s_nop 1\n\t" ROCBTA_FMAC("%0", "0") ROCBTA_FMAC("%1", "1") ROCBTA_FMAC("%2", "2")
+                     ROCBTA_FMAC("%3", "3") ROCBTA_FMAC("%4", "4") ROCBTA_FMAC("%5", "5")
+                         ROCBTA_FMAC("%6", "6") ROCBTA_FMAC("%7", "7")
+                 : "+v"(x[K0]), "+v"(x[K0 + 1]), "+v"(x[K0 + 2]), "+v"(x[K0 + 3]),
+                   "+v"(x[K0 + 4]), "+v"(x[K0 + 5]), "+v"(x[K0 + 6]), "+v"(x[K0 + 7]) ROCBTA_IN);
+    row_fmac<K0 + 8, N - 8>(x, s, y);
+  }
+}
+#undef ROCBTA_IN
+#undef ROCBTA_FMAC
+
+// Column J of the panel: x is its pivot (in every lane).  The steps of the
+// reciprocal square root (pivot_sqrt) are a dependent chain; the updates by
+// column J - 1, still open when column J starts, are dealt between them in
+// this order (the scheduling barriers keep it).  The next pivot is formed from
+// two broadcasts, A(J+1,J) and A(J+1,J+1), read ahead of the root, so neither
+// the scaled column nor a broadcast of it is on the path from pivot to pivot.
+// pv: lane J keeps its pivot.
+template <int J>
+__device__ __forceinline__ void panel_columns(double (&d)[PW], double (&r)[PW], double x,
+                                              double& pv, bool ident, int li) {
+  if constexpr (J < PW) {
+    constexpr int N = J == 0 ? 0 : PW - J;  // open updates of d[J ..] and of r[J ..]
+    constexpr int N1 = N < 8 ? N / 2 : N - 8;
+    constexpr int JP = J == 0 ? 0 : J - 1, JN = J + 1 < PW ? J + 1 : J;
+    const double sp = d[JP], srp = r[JP];
+    double u = 0.0, nx = 0.0;
+    __builtin_amdgcn_sched_barrier(0);
+    const double y0 = __builtin_amdgcn_rsq(x);
+    __builtin_amdgcn_sched_barrier(0);
+    row_fmac<J, N>(d, sp, sp);
+    __builtin_amdgcn_sched_barrier(0);
+    const double t = x * y0;
+    __builtin_amdgcn_sched_barrier(0);
+    if constexpr (J + 1 < PW) row_bcast2<JN>(d[J], d[JN], u, nx);
+    __builtin_amdgcn_sched_barrier(0);
+    const double e = __builtin_fma(-t, y0, 1.0);
+    __builtin_amdgcn_sched_barrier(0);
+    row_fmac<J, N1>(r, sp, srp);
+    if constexpr (J == 0) {
+      // the rows of the identity (see wave_panel_potrf16)
 #pragma unroll
-  for (int k = 0; k < PW; ++k) r[k] = act ? S[ic][p + k] : 0.0;
-  int bad = PW;
-#pragma unroll
-  for (int c0 = 0; c0 < PW; c0 += 4) {
-#pragma unroll
-    for (int jj = 0; jj < 4; ++jj) {
-      const int j = c0 + jj;
-      const double piv = readlane_f64(r[j], j);
-      bad = (bad == PW && !(piv > 0.0)) ? j : bad;
-      double d, inv;
-      pivot_sqrt(piv, d, inv);
-      // broadcasts read the scaled column before the diagonal entry d is
-      // selected in (d is off the path to the next pivot)
-      const double sc = r[j] * inv;
-#pragma unroll
-      for (int k = j + 1; k < c0 + 4; ++k) r[k] -= sc * readlane_f64(sc, k);
-      r[j] = (lane == j) ? d : sc;
+      for (int k = 0; k < PW; ++k) r[k] = ident ? (k == li ? 1.0 : 0.0) : r[k];
     }
+    __builtin_amdgcn_sched_barrier(0);
+    const double q = y0 * e;
+    const double p = __builtin_fma(0.375, e, 0.5);
+    __builtin_amdgcn_sched_barrier(0);
+    row_fmac<J + N1, N - N1>(r, sp, srp);
+    __builtin_amdgcn_sched_barrier(0);
+    const double y = __builtin_fma(q, p, y0);
+    pv = li == J ? x : pv;
+    __builtin_amdgcn_sched_barrier(0);
+    const double w = u * y;
+    d[J] *= y;
+    __builtin_amdgcn_sched_barrier(0);
+    const double xn = __builtin_fma(-w, w, nx);
+    r[J] *= y;
+    __builtin_amdgcn_sched_barrier(0);
+    panel_columns<J + 1>(d, r, xn, pv, ident, li);
+  }
+}
+
+// Cholesky of the 16-column panel S[p:m, p:p+16] (p + 16 <= m <= 64) by one
+// wave, and, with INV, the inverse of its diagonal block (16 x 16, zeros above
+// the diagonal).  factor() leaves the rows below the diagonal block in S;
+// finish() writes the block, and its inverse to Xp (row pitch ldx), which may
+// wait until other waves have been let on to those rows.
+//
+// Every 16-lane row of the wave holds the diagonal block (lane li of the row:
+// matrix row p + li, in d), so the broadcast of a column entry is the
+// row_newbcast modifier of a multiply-add and costs no instruction.  Beside
+// it, r holds one further row per lane that is solved against the block as it
+// is factored: lanes 16 .. 63 the panel rows below it, lanes 0 .. 15 the
+// identity, whose solution is the transposed inverse of the block.
+//
+// Bound by FP64 issue on one wave: 272 multiply-adds of 4 cycles and 16
+// dependent pivot steps of about 80.  Entries of S above the diagonal of the
+// block are left undefined.  A non-positive or NaN pivot turns into NaN
+// through the reciprocal square root, so the loop has no branch; the first
+// failing column is recorded once after it.
+template <bool INV>
+struct WavePanel16 {
+  double d[PW], r[PW], pv;
+  __device__ __forceinline__ void factor(double (*S)[TT_LD], int p, int m) {
+    const int lane = threadIdx.x & 63, li = lane & 15;
+    const int row = p + lane;
+    const double* sd = &S[p + li][p];
+    const double* sr = &S[row < m ? row : p + li][p];
 #pragma unroll
-    for (int q = 0; q < 4; ++q)
-      if (act && p + c0 + q <= i) S[i][p + c0 + q] = r[c0 + q];
-    if (c0 + 4 < PW) {
-      __builtin_amdgcn_wave_barrier();  // the sub-panel's LDS stores precede the reads below
-      // Every broadcast read of the finished rows is issued before the next
-      // pivot column's update, which takes readlanes: the reads' latency
-      // then overlaps it instead of stalling the pivot path read by read.
-      double lrow[PW - 5][4];
+    for (int k = 0; k < PW; ++k) d[k] = sd[k];
 #pragma unroll
-      for (int k = c0 + 5; k < PW; ++k)
+    for (int k = 0; k < PW; ++k) r[k] = sr[k];
+    pv = 0.0;
+    panel_columns<0>(d, r, row_bcast<0>(d[0]), pv, INV && lane < 16, li);
+    if (lane >= 16 && row < m) {
+      double* dst = &S[row][p];
 #pragma unroll
-        for (int q = 0; q < 4; ++q) lrow[k - c0 - 5][q] = S[p + k][p + c0 + q];
-      __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-      for (int q = 0; q < 4; ++q) r[c0 + 4] -= r[c0 + q] * readlane_f64(r[c0 + q], c0 + 4);
-#pragma unroll
-      for (int k = c0 + 5; k < PW; ++k)
-#pragma unroll
-        for (int q = 0; q < 4; ++q) r[k] -= r[c0 + q] * lrow[k - c0 - 5][q];
-      __builtin_amdgcn_wave_barrier();
+      for (int k = 0; k < PW; ++k) dst[k] = r[k];
     }
   }
-  if (bad < PW && lane == 0) record_info(info, (int)(row0 + p + bad + 1));
-}
+  __device__ __forceinline__ void finish(double (*S)[TT_LD], int p, double* Xp, int ldx, int* info,
+                                         int64_t row0) {
+    const int lane = threadIdx.x & 63;
+    if (lane < 16) {
+      if (INV) {
+#pragma unroll
+        for (int k = 0; k < PW; ++k) Xp[k * ldx + lane] = r[k];
+      }
+      double* dst = &S[p + lane][p];
+#pragma unroll
+      for (int k = 0; k < PW; ++k) dst[k] = d[k];
+      double s, inv;
+      pivot_sqrt(pv, s, inv);
+      dst[lane] = s;
+    }
+    const uint64_t bad = __ballot(!(pv > 0.0)) & 0xffffull;
+    if (bad && lane == 0) record_info(info, (int)(row0 + p + __builtin_ctzll(bad) + 1));
+  }
+};
 
 // S[q:m, q:m] (lower part) -= P P^T with P = S[q:m, p:p+w], on MFMA, all
 // waves.  Output 16x16 blocks are dealt round-robin to the waves.
@@ -204,9 +302,11 @@ __device__ __forceinline__ void lds_syrk_update(double (*S)[TT_LD], int p, int w
     }
 }
 
-// Full 64-tile form: S[c0:64, c0:c1] (lower part) -= P P^T restricted to
-// the 16-wide column blocks [c0, c1), P = S[:, p:p+16].  Block t of the
-// enumeration goes to wave wave0 + t % nw; other waves return at once.
+// Full 64-tile form: S[c0:64, c0:c1] (lower 16 x 16 blocks) -= P P^T
+// restricted to the 16-wide column blocks [c0, c1), P = S[:, p:p+16].  Block t
+// of the enumeration goes to wave wave0 + t % nw; other waves return at once.
+// Diagonal blocks are written in full (nothing reads a tile above its
+// diagonal).
 __device__ __forceinline__ void lds_syrk_cols(double (*S)[TT_LD], int p, int c0, int c1,
                                               int wave0, int nw) {
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
@@ -215,15 +315,22 @@ __device__ __forceinline__ void lds_syrk_cols(double (*S)[TT_LD], int p, int c0,
   for (int cb = c0 / 16; cb < c1 / 16; ++cb)
     for (int rb = cb; rb < TT / 16; ++rb, ++t) {
       if (wave != wave0 + t % nw) continue;
-      f64x4 acc = {0.0, 0.0, 0.0, 0.0};
-      const int ra = rb * 16 + li, rc = cb * 16 + li;
+      const double* ra = &S[rb * 16 + li][p + lk];
+      const double* rc = &S[cb * 16 + li][p + lk];
+      double av[4], bv[4], cv[4];
 #pragma unroll
-      for (int kk = 0; kk < PW; kk += 4) acc = mfma_f64(S[ra][p + kk + lk], S[rc][p + kk + lk], acc);
-#pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        const int row = rb * 16 + acc_row_f64(lane, r), col = cb * 16 + acc_col(lane);
-        if (col <= row) S[row][col] -= acc[r];
+      for (int k = 0; k < 4; ++k) {
+        av[k] = ra[4 * k];
+        bv[k] = rc[4 * k];
       }
+      double* c = &S[rb * 16 + lk][cb * 16 + li];  // accumulator register r: row + 4 r
+#pragma unroll
+      for (int r = 0; r < 4; ++r) cv[r] = c[4 * r * TT_LD];
+      f64x4 acc = {0.0, 0.0, 0.0, 0.0};
+#pragma unroll
+      for (int k = 0; k < 4; ++k) acc = mfma_f64(av[k], bv[k], acc);
+#pragma unroll
+      for (int r = 0; r < 4; ++r) c[4 * r * TT_LD] = cv[r] - acc[r];
     }
 }
 
@@ -233,26 +340,33 @@ struct NoIdle {
 
 // Blocked Cholesky of S (m x m, lower part valid) in place.  MFIX = 64
 // compiles the full-tile case with all sizes constant and a look-ahead: after
-// panel p only the next panel's columns are updated before the next panel
-// is factored (wave 0), while waves 1-3 apply panel p to the columns beyond
-// it.  Full tiles: after that update (if any), waves 1-3 run idle(p) while
-// wave 0 factors panel p + 16; panels 0 .. p are final by then.  The call
-// ends with a barrier after the last of them.  MFIX = 0 handles any m <= 64.
+// panel p only the next panel's columns are updated (waves 1-3) before the
+// next panel is factored (wave 0), while waves 1-3 apply panel p to the
+// columns beyond it.  Full tiles also leave the inverses of the four diagonal
+// blocks in X's (each written with its panel), and after the update beside a
+// panel, waves 1-3 run idle(p) while wave 0 factors panel p + 16; panels 0 ..
+// p and their blocks' inverses are final by then.  The call ends with a barrier
+// after the last of them.  MFIX = 0 handles any m <= 64 and leaves X alone.
 template <int MFIX, typename IDLE = NoIdle>
-__device__ __forceinline__ void lds_potrf_t(double (*S)[TT_LD], int m_rt, int* info,
-                                            int64_t row0, IDLE idle = IDLE()) {
+__device__ __forceinline__ void lds_potrf_t(double (*S)[TT_LD], double (*X)[TT_LD], int m_rt,
+                                            int* info, int64_t row0, IDLE idle = IDLE()) {
   const int m = MFIX ? MFIX : m_rt;
   const int wave = threadIdx.x >> 6;
   if (MFIX == TT) {
-    if (wave == 0) wave_panel_potrf16(S, 0, TT, info, row0);
+    WavePanel16<true> w;
+    if (wave == 0) w.factor(S, 0, TT);
     __syncthreads();
 #pragma unroll
     for (int p = 0; p + PW < TT; p += PW) {
-      lds_syrk_cols(S, p, p + PW, p + 2 * PW, 0, 4);  // next panel's columns
-      __syncthreads();
       if (wave == 0)
-        wave_panel_potrf16(S, p + PW, TT, info, row0);
-      else {
+        w.finish(S, p, &X[p][p], TT_LD, info, row0);
+      else
+        lds_syrk_cols(S, p, p + PW, p + 2 * PW, 1, 3);  // next panel's columns
+      __syncthreads();
+      if (wave == 0) {
+        w.factor(S, p + PW, TT);
+        if (p + 2 * PW == TT) w.finish(S, p + PW, &X[p + PW][p + PW], TT_LD, info, row0);
+      } else {
         if (p + 2 * PW < TT) lds_syrk_cols(S, p, p + 2 * PW, TT, 1, 3);  // the rest, beside the panel
         idle(p);
       }
@@ -263,80 +377,73 @@ __device__ __forceinline__ void lds_potrf_t(double (*S)[TT_LD], int m_rt, int* i
 #pragma unroll
   for (int p = 0; p < m; p += PW) {
     const int w = min(PW, m - p);
-    if (MFIX || w == PW) {
-      if (wave == 0) wave_panel_potrf16(S, p, m, info, row0);
+    if (w == PW) {
+      if (wave == 0) {
+        WavePanel16<false> wp;
+        wp.factor(S, p, m);
+        wp.finish(S, p, nullptr, 0, info, row0);
+      }
     } else {
       if (wave == 0) wave_panel_potrf<0>(S, p, m, w, info, row0);
     }
     __syncthreads();
     if (p + w < m) {
-      if (MFIX)
-        lds_syrk_update<PW>(S, p, PW, p + w, m);
-      else
-        lds_syrk_update<0>(S, p, w, p + w, m);
+      lds_syrk_update<0>(S, p, w, p + w, m);
       __syncthreads();
     }
   }
 }
 
-__device__ __forceinline__ void lds_potrf(double (*S)[TT_LD], int m, int* info, int64_t row0) {
+__device__ __forceinline__ void lds_potrf(double (*S)[TT_LD], double (*X)[TT_LD], int m, int* info,
+                                          int64_t row0) {
   if (m == TT)
-    lds_potrf_t<TT>(S, TT, info, row0);
+    lds_potrf_t<TT>(S, X, TT, info, row0);
   else
-    lds_potrf_t<0>(S, m, info, row0);
+    lds_potrf_t<0>(S, X, m, info, row0);
 }
 
 // X = L^{-1} (m x m lower, in S) into Xs (lower; strict upper zero).
-// Step 1: each wave inverts 16x16 diagonal blocks by Gauss-Jordan sweeps,
-// lane = (row i, column group g of four columns).  Step 2: off-diagonal
-// blocks by increasing distance d from the diagonal on MFMA:
+// Step 1: each wave inverts 16x16 diagonal blocks (full tiles: as the rows
+// of a triangular solve; ragged ones by Gauss-Jordan sweeps, lane = (row i,
+// column group g of four columns)).  Step 2: off-diagonal blocks by
+// increasing distance d from the diagonal on MFMA:
 //   X_IJ = -X_II * sum_{K=J}^{I-1} L_IK X_KJ.
-// Ws: 64 x 17 scratch; at distance d the block (I, I-d) of W sits in rows
-// 16I .. 16I+15.
+// Ws: 64 x 17 scratch of the ragged form; at distance d the block (I, I-d) of
+// W sits in rows 16I .. 16I+15.
 constexpr int WS_LD = 17;
 
+// Columns J .. 15 of r <- r L^{-T} for the 16 x 16 lower triangle whose rows
+// lie in d (replicated in every 16-lane row) and whose inverse diagonal lies
+// in dinv, lane = row.
+template <int J>
+__device__ __forceinline__ void trinv_columns(const double (&d)[PW], double (&r)[PW], double dinv) {
+  if constexpr (J < PW) {
+    r[J] *= row_bcast<J>(dinv);
+    row_fmac<(J + 1 < PW ? J + 1 : J), PW - 1 - J>(r, d[J], r[J]);
+    trinv_columns<J + 1>(d, r, dinv);
+  }
+}
+
 // Inverse of the full 16x16 lower-triangular block of S at (o, o) by the
-// calling wave, written to Xs as a full block (zeros above the diagonal).
-// Lane c (and its copies c + 16, c + 32, c + 48) forms column c by forward
-// substitution, x_i = (delta_ic - sum_{k<i} L_ik x_k) / L_ii; the entries
-// L_ik are LDS broadcasts and 1 / L_ii comes from lane i by readlane, so the
-// step needs no division on its dependency path and no cross-lane shuffle.
-// The block is written to dst (row pitch ld).
+// calling wave, written to dst (row pitch ld) as a full block (zeros above
+// the diagonal): the rows of the identity solved against the block give the
+// rows of its transposed inverse, with the broadcasts of a column as operand
+// modifiers (row_fmac), 120 multiply-adds in all.  Lanes 16 .. 63 repeat
+// lanes 0 .. 15.  Measured with the block in LDS: 2939 cycles before (column
+// substitution on LDS broadcasts).
 __device__ __forceinline__ void wave_diag_inv16_to(const double (*S)[TT_LD], int o, double* dst,
                                                    int ld) {
-  const int lane = threadIdx.x & 63;
-  const int c = lane & 15;
-  const double dinv = 1.0 / S[o + c][o + c];
-  const double* S0 = &S[0][0];
-  double x[16];
-  // The LDS broadcast reads of row i+1, L(i+1, 0..i), are issued while row i
-  // is substituted, so each row's reads have landed when it starts.  Left to
-  // itself the compiler either waits after every read or hoists every row's
-  // reads to the top (all 120 entries live at once).  The read address of
-  // row i+1 takes a zero produced from x[i-1] (an asm move with that input),
-  // which keeps the reads below x[i-1]; the scheduling barrier keeps them
-  // above row i's work.
-  double cur[16], nxt[16];
+  const int lane = threadIdx.x & 63, li = lane & 15;
+  double d[PW], r[PW];
+  const double dinv = 1.0 / S[o + li][o + li];
 #pragma unroll
-  for (int i = 0; i < 16; ++i) {
-    if (i + 1 < 16) {
-      int zero = 0;
-      if (i >= 1) asm volatile("v_mov_b32 %0, 0" : "=v"(zero) : "v"(x[i - 1]));
-      const double* row = S0 + (o + i + 1) * TT_LD + o + zero;
+  for (int k = 0; k < PW; ++k) d[k] = S[o + li][o + k];
 #pragma unroll
-      for (int k = 0; k <= i; ++k) nxt[k] = row[k];
-    }
-    __builtin_amdgcn_sched_barrier(0);
-    double acc = (i == c) ? 1.0 : 0.0;
-#pragma unroll
-    for (int k = 0; k < i; ++k) acc -= cur[k] * x[k];
-    x[i] = acc * readlane_f64(dinv, i);
-#pragma unroll
-    for (int k = 0; k <= i; ++k) cur[k] = nxt[k];
-  }
+  for (int k = 0; k < PW; ++k) r[k] = k == li ? 1.0 : 0.0;
+  trinv_columns<0>(d, r, dinv);
   if (lane < 16) {
 #pragma unroll
-    for (int i = 0; i < 16; ++i) dst[i * ld + c] = x[i];
+    for (int k = 0; k < PW; ++k) dst[k * ld + li] = r[k];
   }
 }
 __device__ __forceinline__ void wave_diag_inv16(const double (*S)[TT_LD], double (*Xs)[TT_LD],
@@ -369,7 +476,8 @@ __device__ __forceinline__ void wave_trtri_offdiag(const double (*S)[TT_LD], dou
 
 // ZERO = false: the caller guarantees that the blocks of Xs strictly above
 // the 16x16 block diagonal already hold zeros (they are never written here).
-template <int MFIX, bool ZERO = true>
+// DIAG = false (full tiles): the inverses of the diagonal blocks are there.
+template <int MFIX, bool ZERO = true, bool DIAG = true>
 __device__ __forceinline__ void lds_trtri_t(const double (*S)[TT_LD], double (*Xs)[TT_LD],
                                             double (*Ws)[WS_LD], int m_rt) {
   const int m = MFIX ? MFIX : m_rt;
@@ -379,10 +487,20 @@ __device__ __forceinline__ void lds_trtri_t(const double (*S)[TT_LD], double (*X
     for (int idx = tid; idx < TT * TT; idx += TT_THREADS) Xs[idx / TT][idx % TT] = 0.0;
     __syncthreads();
   }
-  const int nb = (m + 15) / 16;
   if (MFIX == TT) {
-    wave_diag_inv16(S, Xs, __builtin_amdgcn_readfirstlane(16 * wave));
-  } else
+    if (DIAG) {
+      wave_diag_inv16(S, Xs, __builtin_amdgcn_readfirstlane(16 * wave));
+      __syncthreads();
+    }
+#pragma unroll
+    for (int dist = 1; dist < TT / 16; ++dist) {
+      const int I = wave + dist;
+      if (I < TT / 16) wave_trtri_offdiag(S, Xs, &Xs[16 * I][16 * I], TT_LD, I, wave);
+      __syncthreads();
+    }
+    return;
+  }
+  const int nb = (m + 15) / 16;
   for (int blk = wave; blk < nb; blk += 4) {
     const int o = blk * 16, w = min(16, m - o);
     const int i = lane & 15, g = lane >> 4;
@@ -472,9 +590,12 @@ __device__ __forceinline__ void tile_factor_body(const TileBatch& tb, int bz, do
     if (r < m && c <= r) v = A[(int64_t)r * tb.lda + c];
     S[r][c] = v;
   }
+  if (MODE == 0 && m == TT) {  // the factorization fills in the diagonal blocks' inverses
+    for (int idx = tid; idx < TT * TT; idx += TT_THREADS) Xs[idx / TT][idx % TT] = 0.0;
+  }
   __syncthreads();
   if (MODE == 0) {
-    lds_potrf(S, m, tb.info, tb.info_row0 + b1 * tb.info_s1 + b2 * tb.info_s2);
+    lds_potrf(S, Xs, m, tb.info, tb.info_row0 + b1 * tb.info_s1 + b2 * tb.info_s2);
     // write L back, upper triangle zero-filled
     for (int idx = tid; idx < m * m; idx += TT_THREADS) {
       int r = idx / m, c = idx % m;
@@ -486,7 +607,10 @@ __device__ __forceinline__ void tile_factor_body(const TileBatch& tb, int bz, do
     }
   }
   if (tb.X != nullptr) {
-    lds_trtri(S, Xs, Ws, m);
+    if (MODE == 0 && m == TT)
+      lds_trtri_t<TT, false, false>(S, Xs, Ws, TT);
+    else
+      lds_trtri(S, Xs, Ws, m);
     double* X = tb.X + b1 * tb.sX1 + b2 * tb.sX2;
     for (int idx = tid; idx < m * m; idx += TT_THREADS) {
       int r = idx / m, c = idx % m;
