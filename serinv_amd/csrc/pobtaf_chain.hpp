@@ -810,6 +810,30 @@ __device__ __forceinline__ void chain_run(const PobtafChain& P, double* S, doubl
 }
 
 
+// Columns p .. p + 15 of the factored tile S to memory by the calling wave,
+// zeros above the diagonal.
+__device__ __forceinline__ void chain_store_panel(const double (*S)[TT_LD], int p, const CTile& t) {
+  const int lane = threadIdx.x & 63, c = p + (lane & 7) * 2;
+  cdbl2 v[8];
+#pragma unroll
+  for (int q = 0; q < 8; ++q) {
+    const int r = (lane >> 3) + 8 * q;
+    v[q].x = c <= r ? S[r][c] : 0.0;
+    v[q].y = c + 1 <= r ? S[r][c + 1] : 0.0;
+  }
+  double* dst = t.p + (int64_t)(lane >> 3) * t.ld + c;
+  if ((t.ld & 1) == 0 && (reinterpret_cast<uintptr_t>(t.p) & 15) == 0) {
+#pragma unroll
+    for (int q = 0; q < 8; ++q) *reinterpret_cast<cdbl2*>(dst + 8 * q * t.ld) = v[q];
+  } else {
+#pragma unroll
+    for (int q = 0; q < 8; ++q) {
+      dst[8 * q * t.ld] = v[q].x;
+      dst[8 * q * t.ld + 1] = v[q].y;
+    }
+  }
+}
+
 // Rows r0 .. r0 + 15 of Ps (64 x 64, K-contiguous) <- Ps Linv^T, by the calling
 // wave, in place: column block J takes K < 16 J + 16 (Linv is lower
 // triangular), 40 MFMA steps on four accumulators, each operand of Ps read
@@ -954,22 +978,26 @@ __device__ __forceinline__ void chain_run_fused(const PobtafChain& P, double* Sa
     }
     pending = -1;
     chain_trace(P, g, 0);
-    // 1. factorization with Linv block rows 1 and 2 beside it; PX(g) and
-    //    PD(g+1) flags checked by wave 1 during the last panel
+    // 1. factorization with Linv block rows 1 and 2 and the stores of
+    //    finished panels beside it; PX(g) and PD(g+1) flags checked by wave 1
+    //    during the last panel
     const int64_t row0 = (int64_t)(g / P.nt) * P.b + (int64_t)(g % P.nt) * CT;
     lds_potrf_t<CT>(S2, X2, CT, P.info, row0, [&](int p) {
-      if (p == 16 && wave == 2) wave_trtri_offdiag(S2, X2, &X2[16][16], TT_LD, 1, 0);
-      if (p == 32) {
-        if (wave == 1) {
-          int ok = sub ? (__hip_atomic_load(f_px, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) &
-                          __hip_atomic_load(f_pd, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT))
-                       : 0;
-          ok = __builtin_amdgcn_readfirstlane(ok);
-          if (ok) __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
-          if (lane == 0) s_early = ok;
-        } else {
-          wave_trtri_offdiag(S2, X2, &X2[32][32], TT_LD, 2, wave == 2 ? 1 : 0);
-        }
+      if (p < 32) {
+        if (wave == 3) chain_store_panel(S2, p, dt);
+        if (p == 16 && wave == 2) wave_trtri_offdiag(S2, X2, &X2[16][16], TT_LD, 1, 0);
+      } else if (wave == 1) {
+        chain_store_panel(S2, 32, dt);
+        // a few looks: a flag set while the panel runs saves the wait after it
+        int ok = 0;
+        for (int look = 0; sub && !ok && look < 3; ++look)
+          ok = __builtin_amdgcn_readfirstlane(
+              __hip_atomic_load(f_px, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) &
+              __hip_atomic_load(f_pd, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT));
+        if (ok) __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
+        if (lane == 0) s_early = ok;
+      } else {
+        wave_trtri_offdiag(S2, X2, &X2[32][32], TT_LD, 2, wave == 2 ? 1 : 0);
       }
     });
     const int early = s_early;
@@ -994,9 +1022,11 @@ __device__ __forceinline__ void chain_run_fused(const PobtafChain& P, double* Sa
       }
     };
     if (early) load_px();
-    // 2. Linv block row 3; L(g,g) to memory, upper triangle zero (16-byte
-    //    stores); Linv(g) to memory
-    if (wave >= 1) wave_trtri_offdiag(S2, X2, &X2[48][48], TT_LD, 3, wave - 1);
+    // 2. Linv block row 3; the last panel of L(g,g) and Linv(g) to memory
+    if (wave >= 1)
+      wave_trtri_offdiag(S2, X2, &X2[48][48], TT_LD, 3, wave - 1);
+    else
+      chain_store_panel(S2, 48, dt);
     __syncthreads();
     double* li_out = P.linv + (int64_t)g * CT * CT;
     {
@@ -1009,20 +1039,7 @@ __device__ __forceinline__ void chain_run_fused(const PobtafChain& P, double* Sa
 #pragma unroll
       for (int q = 0; q < 8; ++q) *reinterpret_cast<cdbl2*>(li_out + (rs + 8 * q) * CT + c2) = v[q];
     }
-    auto store_l = [&]() {
-      cdbl2 v[8];
-#pragma unroll
-      for (int q = 0; q < 8; ++q) {
-        const int rr = rs + 8 * q;
-        v[q].x = (c2 <= rr) ? S2[rr][c2] : 0.0;
-        v[q].y = (c2 + 1 <= rr) ? S2[rr][c2 + 1] : 0.0;
-      }
-#pragma unroll
-      for (int q = 0; q < 8; ++q)
-        *reinterpret_cast<cdbl2*>(dt.p + (int64_t)(rs + 8 * q) * dt.ld + c2) = v[q];
-    };
     if (!sub) {  // last diagonal tile of the matrix
-      store_l();
       chain_publish(P.cflags + 2 * g);
       continue;
     }
@@ -1055,8 +1072,7 @@ __device__ __forceinline__ void chain_run_fused(const PobtafChain& P, double* Sa
       chain_syrk<f32x4>(Ps, pd, wave, Sn);
     else
       chain_syrk<f64x4>(Ps, pd, wave, Sn);
-    store_l();
-    wave_stores_done();  // L(g,g), L(g+1,g): released at the start of step g+1
+    wave_stores_done();  // L(g+1,g): released at the start of step g+1
     __syncthreads();
     chain_trace(P, g, 5);
     double* t = S;
