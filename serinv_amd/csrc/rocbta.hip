@@ -1172,10 +1172,10 @@ StLayout st_layout(int64_t b, int64_t a, bool selinv) {
   return l;
 }
 
-// Workspace of the non-SPD sweeps: the blocked inverse's pivot-tile
-// inverse P and its row / column panels, and the products of one step.
+// Workspace of the non-SPD sweeps: the blocked inverse's second copy of the
+// block, and the products of one step.
 struct DdLayout {
-  size_t p, r, c, w, v, b1, b2, c1, c2, e, g, dc, y;
+  size_t inv, w, v, b1, b2, c1, c2, e, g, dc, y;
   // quadratic (A X A^T = B) forms
   size_t bdc, df1, df2, dk1, dk2, sm, mt, q1, q2, q3, z, p1, p2, m1, m2, v1, zt, p3, d2, bbt, y2,
       total;
@@ -1190,9 +1190,7 @@ DdLayout dd_layout(int64_t b, int64_t a) {
   };
   const int64_t mm = std::max(b, a), a1 = std::max<int64_t>(a, 1);
   const size_t bb = (size_t)b * b * sizeof(double), ab = (size_t)a1 * b * sizeof(double);
-  l.p = take(TT * TT * sizeof(double));
-  l.r = take((size_t)TT * mm * sizeof(double));
-  l.c = take((size_t)mm * TT * sizeof(double));
+  l.inv = take((size_t)mm * mm * sizeof(double));
   l.w = take(bb);
   l.v = take(ab);
   l.b1 = take(bb);
@@ -1231,8 +1229,11 @@ DdLayout dd_layout(int64_t b, int64_t a) {
 
 // A <- A^{-1} for a general m x m matrix (row stride ld), in place, by
 // blocked Gauss-Jordan elimination over 64-wide pivot blocks without
-// pivoting (the ddbt* blocks are diagonally dominant).  Step k, with
-// P = A_kk^{-1}:
+// pivoting (the ddbt* blocks are diagonally dominant).  While the matrix has
+// at most one tile per CU a step is one launch in which every workgroup
+// inverts the pivot tile itself (block_getri_kernel), alternating between A
+// and the workspace copy.  Larger matrices would repeat that inverse several
+// times per CU; they take four launches per step, with P = A_kk^{-1}:
 //   (1) A_kk <- P (tile kernel, in place);
 //   (2) A_kj <- P A_kj (j != k);
 //   (3) A_ij -= A_ik A_kj (i, j != k; A_kj is the new row block);
@@ -1241,8 +1242,22 @@ DdLayout dd_layout(int64_t b, int64_t a) {
 // aliased operand, only that tile (K = the pivot block's width), and reads
 // it in full before its epilogue writes.
 int block_inverse(double* A, int64_t ld, int m, char* ws, const DdLayout& lay, hipStream_t s) {
-  (void)ws;
-  (void)lay;
+  const int nt = cdiv(m, TT);
+  if (nt > 1 && nt * nt <= device_cus()) {
+    double* W = (double*)(ws + lay.inv);
+    for (int k = 0; k < nt; ++k) {
+      if (k % 2 == 0)
+        block_getri_kernel<<<nt * nt, CH_THREADS, 0, s>>>(A, ld, W, m, m, nt, k);
+      else
+        block_getri_kernel<<<nt * nt, CH_THREADS, 0, s>>>(W, m, A, ld, m, nt, k);
+      RB_CHECK(hipGetLastError());
+    }
+    if (nt % 2) {
+      wide_copy_rows_kernel<<<cdiv((int64_t)m * m, 256), 256, 0, s>>>(A, ld, W, m, m, m);
+      RB_CHECK(hipGetLastError());
+    }
+    return ROCBTA_OK;
+  }
   for (int k0 = 0; k0 < m; k0 += TT) {
     const int tk = std::min(TT, m - k0), k1 = k0 + tk;
     double* Pk = A + (int64_t)k0 * ld + k0;
