@@ -173,9 +173,9 @@ int rocbta_dquad(int64_t rows, int64_t r, const double* y, const double* x, int6
 /* Launch shapes (no counterpart in the reference; set by the autotuner):
  * ROCBTA_BATCHED_RC1 / _RC4 / _RC8 force the solve sweeps' column-chunk
  * width (right-hand-side columns per chain workgroup; default: 1 for r = 1,
- * 4 for r <= 4, else 8), ROCBTA_BATCHED_GEMM512 runs the selected-inversion
- * GEMM phases on 512-thread workgroups whose two halves split each 64x64
- * tile's K range (default: 256 threads, two workgroups per CU). */
+ * 4 for r <= 4, else 8), ROCBTA_BATCHED_GEMM512 runs every selected-inversion
+ * GEMM phase on 32x32 tiles (512 threads, the K range split over the eight
+ * waves; default: phases of many tiles take 64x64 ones). */
 #define ROCBTA_BATCHED_RC1 16
 #define ROCBTA_BATCHED_RC4 32
 #define ROCBTA_BATCHED_RC8 64

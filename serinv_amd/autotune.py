@@ -6,9 +6,8 @@ batch: small b gives many short chains that want few helpers each, large b
 long chains whose helper queues can keep more workgroups busy.  The plan
 also has two tile shapes: the solve sweeps' column-chunk width (narrow
 chunks give more, shorter chains; wide ones read each factor tile once for
-more columns) and the workgroup size of the selected-inversion GEMM phases
-(256 threads, two workgroups per CU, or 512 threads whose halves split a
-tile's K range, which suits phases with few tiles).
+more columns) and the tile shape of the selected-inversion GEMM phases (512:
+32 x 32 tiles throughout, 256: 64 x 64 ones in phases of many tiles).
 
 tune_batched times the workgroup counts first (with the default shapes),
 then the tile shapes with the best counts, on scratch copies of the batch

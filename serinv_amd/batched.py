@@ -19,8 +19,9 @@ potrf/trtri, tip, log-determinant and solves).
 Launch shapes (picked per batch class by serinv_amd.autotune): sweep_width
 forces the solve sweeps' column-chunk width (1, 4 or 8 right-hand-side
 columns per chain workgroup; None: 1 for one column, 4 up to four, else 8),
-gemm_threads (256 or 512) the workgroup size of the selected-inversion GEMM
-phases (512: two halves split each 64 x 64 tile's K range).
+gemm_threads (256 or 512) the tile shape of the selected-inversion GEMM
+phases (512: 32 x 32 tiles in every phase, 512 threads splitting K; 256 or
+None: phases of many tiles take 64 x 64 ones).
 """
 
 import ctypes

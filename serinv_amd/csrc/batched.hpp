@@ -29,7 +29,7 @@ __global__ void fill_list_kernel(const FillOp* ops) {
 struct PhaseLaunch {
   int nfill = 0, ntile = 0, ngemm = 0;
   int64_t maxfill = 0;
-  int tile_grid = 0, gemm_tiles = 0;
+  int tile_grid = 0, gemm_tiles = 0, gemm_width = 1;
   size_t fill_off = 0, tile_off = 0, gemm_off = 0;  // offsets into the descriptor buffer
 };
 
@@ -65,7 +65,7 @@ struct BatchedPlan {
   int64_t nempty = 0;
   int sweep_rc = 1;
   int sweep_grid = 0;
-  int gemm512 = 0;  // selected-inversion GEMM phases on 512-thread workgroups
+  int gemm512 = 0;  // selected-inversion GEMM phases on 32-wide tiles throughout
   // selected inversion
   std::vector<PhaseLaunch> phases;
   // graph
@@ -190,11 +190,11 @@ int batched_enqueue(const BatchedPlan& p, hipStream_t s) {
         RB_CHECK(hipGetLastError());
       }
       if (ph.ngemm && ph.gemm_tiles > 0) {
-        if (p.gemm512)
-          gemm_list_kernel_h2<<<ph.gemm_tiles, 2 * GT_THREADS, 0, s>>>(
+        if (ph.gemm_width == 2)
+          gemm_list_kernel<2><<<ph.gemm_tiles, GT_THREADS, 0, s>>>(
               (const GemmProblem*)(p.desc + ph.gemm_off), ph.ngemm);
         else
-          gemm_list_kernel<<<ph.gemm_tiles, GT_THREADS, 0, s>>>(
+          gemm_list_kernel<1><<<ph.gemm_tiles, GT_THREADS, 0, s>>>(
               (const GemmProblem*)(p.desc + ph.gemm_off), ph.ngemm);
         RB_CHECK(hipGetLastError());
       }
@@ -443,9 +443,10 @@ int rocbta_batched_create(int nmat, const int64_t* n, const int64_t* b, const in
     pl.tile_grid = grid;
     if (pl.ntile) pl.tile_off = dtake(ph.tiles.size() * sizeof(TileBatch));
     int64_t tiles = 0;
+    pl.gemm_width = p->gemm512 ? 1 : gemm_width(ph.gemms);
     for (GemmProblem& g : ph.gemms) {
       g.tile_begin = (int)tiles;
-      tiles += (int64_t)g.tiles_m * g.tiles_n * g.batch1 * g.batch2;
+      tiles += gemm_set_tiles(g, pl.gemm_width);
     }
     pl.ngemm = (int)ph.gemms.size();
     pl.gemm_tiles = (int)tiles;

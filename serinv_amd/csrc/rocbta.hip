@@ -66,7 +66,6 @@ struct GemmList {
     p.beta = beta;
     p.nterms = 0;
     p.uplo = uplo;
-    p.ksplit = 1;
     probs.push_back(p);
     return probs.back();
   }
@@ -139,26 +138,32 @@ struct MixedScope {
 
 int device_cus();  // CUs of the current device (below)
 
-// Output tile size for a launch list.  64 by default: measured on the
-// selected inversion at n=256, b=1024 the 128-tile kernel (one workgroup
-// per CU, split-K 4) took 107.6 ms against 62.1 ms for the 64-tile kernel
-// (two workgroups per CU).  ROCBTA_GEMM_TILE=128 selects it for lists whose
-// largest problem is large in both output dimensions and in K.
-bool gemm_tile128_enabled() {
-  const char* e = getenv("ROCBTA_GEMM_TILE");
-  return e && strcmp(e, "128") == 0;
-}
-int gemm_ts_for(int M, int N, int K) {
-  return (gemm_tile128_enabled() && M >= 256 && N >= 256 && K >= 256) ? 128 : 64;
-}
-int gemm_ts(const GemmList& list) {
-  int ts = 64;
-  for (const GemmProblem& p : list.probs) {
-    int kmax = 0;
-    for (int t = 0; t < p.nterms; ++t) kmax = std::max(kmax, p.t[t].K);
-    if (gemm_ts_for(p.M, p.N, kmax) == 128) ts = 128;
+// Width (in 32s) of the output tiles of a launch: 1, with the K range split
+// over the eight waves of a workgroup, or 2, with it split in two.  Wide tiles
+// read each operand half as often from L2: sixteen 1024^3 products take 630
+// instead of 733 us.  A launch of fewer wide tiles than two rounds of
+// the CUs leaves more of them idle than that is worth: 10.7 against 25 us at
+// 512^3, 50 us both at 1024^3 (one wide tile per CU).  In-place problems need
+// the wide ones (aliasing contract of gemm_f64.hpp).
+template <class V>
+int gemm_width(const V& probs) {
+  int64_t wide = 0;
+  for (const GemmProblem& p : probs) {
+    for (int t = 0; t < p.nterms; ++t)
+      if (p.t[t].A == p.C || p.t[t].B == p.C) return 2;
+    const int64_t tm = cdiv(p.M, 2 * GW), tn = cdiv(p.N, 2 * GW);
+    wide += (p.uplo == TRI_NONE ? tm * tn : tm * (tn + 1) / 2) * p.batch1 * p.batch2;
   }
-  return ts;
+  return wide >= 2 * (int64_t)device_cus() ? 2 : 1;
+}
+// Tile counts of a problem for tiles of that width; returns its workgroups.
+int64_t gemm_set_tiles(GemmProblem& p, int width) {
+  p.tiles_m = cdiv(p.M, GW * width);
+  p.tiles_n = cdiv(p.N, GW * width);
+  p.lower_packed = (p.uplo == TRI_LOWER && p.tiles_m == p.tiles_n) ? 1 : 0;
+  const int64_t per_batch =
+      p.lower_packed ? (int64_t)p.tiles_m * (p.tiles_m + 1) / 2 : (int64_t)p.tiles_m * p.tiles_n;
+  return per_batch * p.batch1 * p.batch2;
 }
 
 int run_gemms(GemmList& list, hipStream_t s) {
@@ -169,34 +174,20 @@ int run_gemms(GemmList& list, hipStream_t s) {
     for (GemmProblem p : list.probs) {
       if (p.M <= 0 || p.N <= 0 || p.batch1 <= 0 || p.batch2 <= 0) continue;
       if (p.nterms == 0 && p.beta == 1.0) continue;
-      p.tiles_m = cdiv(p.M, GT_M);
-      p.tiles_n = cdiv(p.N, GT_N);
-      p.ksplit = 1;
-      p.partial = nullptr;
-      p.counters = nullptr;
       p.f32 = g_mixed ? 1 : 0;
       ph.gemms.push_back(p);
     }
     return ROCBTA_OK;
   }
-  const int ts = gemm_ts(list);
-  // 512-thread 64-tile kernel for launches of at most one tile per CU (two
-  // waves per SIMD instead of one); ROCBTA_GEMM_H2=0 / 1 forces it off / on.
-  static const int h2_mode = [] {
-    const char* e = getenv("ROCBTA_GEMM_H2");
-    return e ? (strcmp(e, "1") == 0 ? 1 : 0) : -1;
-  }();
-  const int cus = device_cus();
+  const int width = gemm_width(list.probs);
   GemmGroup g{};
   auto flush = [&]() -> int {
     if (g.nprob == 0) return ROCBTA_OK;
     if (g.total_tiles > 0) {
-      if (ts == 128)
-        gemm_group_kernel_t128<<<g.total_tiles, GT_THREADS, 0, s>>>(g);
-      else if (h2_mode == 1 || (h2_mode < 0 && g.total_tiles <= cus))
-        gemm_group_kernel_h2<<<g.total_tiles, 2 * GT_THREADS, 0, s>>>(g);
+      if (width == 2)
+        gemm_group_kernel<2><<<g.total_tiles, GT_THREADS, 0, s>>>(g);
       else
-        gemm_group_kernel<<<g.total_tiles, GT_THREADS, 0, s>>>(g);
+        gemm_group_kernel<1><<<g.total_tiles, GT_THREADS, 0, s>>>(g);
       RB_CHECK(hipGetLastError());
     }
     g = GemmGroup{};
@@ -205,14 +196,8 @@ int run_gemms(GemmList& list, hipStream_t s) {
   for (GemmProblem p : list.probs) {
     if (p.M <= 0 || p.N <= 0 || p.batch1 <= 0 || p.batch2 <= 0) continue;
     if (p.nterms == 0 && p.beta == 1.0) continue;
-    p.tiles_m = cdiv(p.M, ts);
-    p.tiles_n = cdiv(p.N, ts);
     p.f32 = g_mixed ? 1 : 0;
-    if (p.ksplit < 1 || !p.partial || !p.counters) p.ksplit = 1;
-    p.lower_packed = (p.uplo == TRI_LOWER && p.tiles_m == p.tiles_n) ? 1 : 0;
-    const int64_t per_batch =
-        p.lower_packed ? (int64_t)p.tiles_m * (p.tiles_m + 1) / 2 : (int64_t)p.tiles_m * p.tiles_n;
-    const int64_t tiles = per_batch * p.batch1 * p.batch2 * p.ksplit;
+    const int64_t tiles = gemm_set_tiles(p, width);
     if (g.nprob == ROCBTA_MAX_PROBLEMS || (int64_t)g.total_tiles + tiles > (1ll << 30)) {
       int rc = flush();
       if (rc) return rc;
@@ -339,8 +324,8 @@ int factor_block_column(double* Dm, int64_t ld, int m, const std::vector<Panel>&
 // Inverse of `batch` lower-triangular m x m matrices (source stride sL,
 // row stride lds) into X (row stride ldx, stride sX), upper part zeroed.
 // W: scratch of batch * ceil(m/64) * 64 * 64 doubles.
-// zero_upper = false (halving path, 64-tile products only): the strictly
-// upper 64-tiles of X are left unwritten.  The halving recursion reads X's
+// zero_upper = false (halving path): the strictly upper 64-tiles of X are
+// left unwritten.  The halving recursion reads X's
 // blocks only as lower triangular operands, whose products clip their K
 // range at the output tile and so skip those tiles, and the diagonal tiles
 // come zero above their diagonal from the tile kernel; callers that read X
@@ -354,9 +339,7 @@ int block_trtri(const double* Ls, int64_t lds, int64_t sL, double* X, int64_t ld
   const int tail = m - nfull * TT;
   if (ldx != m || sX != (int64_t)m * m) return ROCBTA_ERR_ARG;  // X is a dense stack
   const bool halves = halving && tail == 0 && (nt & (nt - 1)) == 0;
-  // 128-tiles clip the K range of a triangular operand at 128, which reaches
-  // into the strictly upper 64-tiles: those must then be zero
-  const bool skip = !zero_upper && halves && !gemm_tile128_enabled();
+  const bool skip = !zero_upper && halves;
   int rc = skip ? ROCBTA_OK : fill(X, (int64_t)batch * m * m, 0.0, s);
   if (rc) return rc;
   rc = tile_factor(1, const_cast<double*>(Ls), lds, (int64_t)TT * (lds + 1), sL, X, ldx,
@@ -492,7 +475,7 @@ class SideLease {
 
 
 struct SiLayout {
-  size_t linv, g, gt, w, tinv, wt, part, cnt, total;
+  size_t linv, g, gt, w, tinv, wt, total;
 };
 
 SiLayout si_layout(int64_t n, int64_t b, int64_t a) {
@@ -512,11 +495,6 @@ SiLayout si_layout(int64_t n, int64_t b, int64_t a) {
   l.w = take((size_t)nch * std::max<int64_t>(ntb * TT * TT, ntb * TT * ntb * TT / 4));
   l.tinv = take((size_t)a * a);
   l.wt = take((size_t)nta * TT * TT);
-  // split-K partial tiles: up to 2 splits of 64-tiles or 8 splits of 128-tiles
-  const int64_t t128 = (b + 127) / 128, a128 = (a + 127) / 128;
-  l.part = take((size_t)std::max<int64_t>((ntb * ntb + ntb * nta + ntb) * 2 * TT * TT,
-                                          (t128 * t128 + t128 * a128 + t128) * 8 * 128 * 128));
-  l.cnt = take((size_t)(ntb * ntb + ntb + 64) / 2 + 1);  // split-K tile counters (ints)
   l.total = off;
   return l;
 }
@@ -1465,26 +1443,6 @@ int rocbta_dpobtasi(int64_t n, int64_t b, int64_t a, double* D, double* L, doubl
   double* W = (double*)(ws + lay.w);
   double* Tinv = (double*)(ws + lay.tinv);
   double* Wt = (double*)(ws + lay.wt);
-  double* part = (double*)(ws + lay.part);
-  int* cnt = (int*)(ws + lay.cnt);
-  const int ntb = cdiv(b, TT);
-  // Split the K loop of the recurrence's b x b products when one product
-  // alone has too few output tiles to occupy every CU (128-tiles: one
-  // workgroup per CU; 64-tiles: two).
-  const int ts = gemm_ts_for((int)b, (int)b, (int)b);
-  const int nts = cdiv(b, ts);
-  const int cus = device_cus();
-  // 64-tiles: no split (one 1024^2 product is 256 tiles, one per CU, and a
-  // split through global partials measured slower than none).
-  int ksplit = 1;
-  if (ts == 128) ksplit = std::max(1, std::min(8, cus / (nts * nts)));
-  if (ksplit > 1) {
-    fill_i32_kernel<<<1, 256, 0, s>>>(cnt, ntb * ntb + ntb, 0);
-    RB_CHECK(hipGetLastError());
-  }
-  // the arrow problem of a step has its own split-K bookkeeping
-  double* part_r = part + (int64_t)nts * nts * ksplit * ts * ts;
-  int* cnt_r = cnt + nts * nts;
   const int bi = (int)b, ai = (int)a;
   const int64_t bb = b * b, ab = a * b;
   // Blocks whose factor is still stored: all of them, or all but the last
@@ -1572,9 +1530,6 @@ int rocbta_dpobtasi(int64_t n, int64_t b, int64_t a, double* D, double* L, doubl
   // X_{i+1,i}, which then is exactly one 64-tile per CU at b = 1024.
   auto arrow_row = [&](GemmList& gl, int64_t i) {
     GemmProblem& pr = gl.add(R + i * ab, b, ai, bi, 0.0);
-    pr.ksplit = ksplit;
-    pr.partial = part_r;
-    pr.counters = cnt_r;
     push_term(pr, term(R + (i + 1) * ab, b, false, G + i * bb, b, false, bi, -1.0));
     push_term(pr, term(T, a, false, Gt + i * ab, b, false, ai, -1.0));
   };
@@ -1591,9 +1546,6 @@ int rocbta_dpobtasi(int64_t n, int64_t b, int64_t a, double* D, double* L, doubl
     if (rc) return rc;
     GemmList off;
     GemmProblem& pl = off.add(L + i * bb, b, bi, bi, 0.0);
-    pl.ksplit = ksplit;
-    pl.partial = part;
-    pl.counters = cnt;
     push_term(pl, term(D + (i + 1) * bb, b, false, G + i * bb, b, false, bi, -1.0));
     if (a > 0) push_term(pl, term(R + (i + 1) * ab, b, true, Gt + i * ab, b, false, ai, -1.0));
     rc = run_gemms(off, s);
@@ -1603,9 +1555,6 @@ int rocbta_dpobtasi(int64_t n, int64_t b, int64_t a, double* D, double* L, doubl
     GemmList dia;
     GemmProblem& pd = dia.add(D + i * bb, b, bi, bi, 1.0, TRI_LOWER);
     pd.mirror = 1;
-    pd.ksplit = ksplit;
-    pd.partial = part;
-    pd.counters = cnt;
     push_term(pd, term(L + i * bb, b, true, G + i * bb, b, false, bi, -1.0));
     if (a > 0) push_term(pd, term(R + i * ab, b, true, Gt + i * ab, b, false, ai, -1.0));
     if (a > 0 && i >= 1) {
