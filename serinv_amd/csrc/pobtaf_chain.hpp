@@ -1221,7 +1221,7 @@ __global__ void __launch_bounds__(CH_THREADS) pobtaf_chain_kernel(PobtafChain P)
 __global__ void __launch_bounds__(CH_THREADS) pobtaf_chain_multi_kernel(const PobtafChain* Ps,
                                                                         int nmat, int* gclaim,
                                                                         int* cu_busy) {
-  __shared__ __attribute__((aligned(16))) double lds[2 * CT * KP + CT * WS_LD];
+  __shared__ __attribute__((aligned(16))) double lds[CH_LDS];
   __shared__ int s_task;
   const int tid = threadIdx.x;
   if (tid == 0) s_task = atomicAdd(gclaim, 1);
@@ -1232,7 +1232,10 @@ __global__ void __launch_bounds__(CH_THREADS) pobtaf_chain_multi_kernel(const Po
   if (first < nmat) {
     if (tid == 0) __hip_atomic_store(cu_busy + my_key, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     const PobtafChain& P = Ps[first];
-    chain_run<1>(P, lds, lds + CT * TT_LD, lds + 2 * CT * TT_LD);
+    if (P.fused)
+      chain_run_fused<1>(P, lds, lds + CT * TT_LD, lds + 2 * CT * TT_LD, lds + 3 * CT * TT_LD);
+    else
+      chain_run<1>(P, lds, lds + CT * TT_LD, lds + 2 * CT * TT_LD);
     return;
   }
   int m = (int)(blockIdx.x % (unsigned)nmat);

@@ -714,36 +714,47 @@ __global__ void fill_u64_kernel(unsigned long long* p, int64_t count, unsigned l
 }
 
 // Solve algorithm: the block-level sweep (precomputed diagonal-block
-// inverses, two dependent device-wide products per block row) for large
-// blocks and at most 8 right-hand sides, its wide form (64 columns per
-// launch, MFMA tiles) for more, the 64-row-tile sweep otherwise, the
-// launch-per-tile form for partial solves on small blocks.
+// inverses, two dependent device-wide products per block row) for at most 4
+// right-hand sides, its wide form (64 columns per launch, MFMA tiles) for
+// more, the 64-row-tile sweep for blocks of one tile and what the others do
+// not fit, the launch-per-tile form for partial solves there.  Per block row
+// the block sweep takes 5.5 us at r = 1 and 8.5 us at r = 4 whatever b is, the
+// wide one 10 us, the tile sweep 4 to 7 us per 64-row tile.  Measured, N + C
+// at n = 64, b = 130, a = 16: r = 1 853 us against 1722 us for the tile sweep,
+// r = 4 1239 against 1959; b = 256, r = 8: wide 1469, block 1905, tile 3539.
 // ROCBTA_POBTAS_ALGO = block | wide | sweep | loop forces one (tests cover
 // all four; block and wide fall back when the shape does not fit them).
 enum SolveAlgo { SOLVE_LOOP = 0, SOLVE_SWEEP = 1, SOLVE_BLOCK = 2, SOLVE_WIDE = 3 };
-constexpr int BS_MIN_B = 256;   // default: block sweep from this block size on
+// The block and wide sweeps need their inverses' launches first (about 40 us
+// a call): they are taken from this many tile steps saved on.  n = 8, b = 96
+// (8 saved): 236 us against 228 for the tile sweep at r = 4; b = 130 (16): 258
+// against 297.
+constexpr int BS_MIN_SAVED = 12;
+constexpr int BS_MIN_B = 256;   // and for these blocks always
 constexpr int BS_MAX_G = 1024;  // workgroups of the block sweep (tip partial sums sized for it)
 
 int bs_cw(int64_t r) { return r <= 1 ? 1 : (r <= 4 ? 4 : 8); }
 bool bs_fits(int64_t a, int64_t r) { return a * bs_cw(r) <= BS_TIPMAX; }
-// Wider right-hand sides take the 64-row-tile sweep by default: the block
-// sweep re-reads the factor once per group of 8 columns (measured at n=256,
-// b=1024, a=32, N+C: r=8 19.8 ms, r=64 89 ms against 59 and 58 ms for the
-// sweep).
+// The block sweep re-reads the factor once per group of columns, and groups of
+// 8 cost it 13.6 us per block row, so it serves 5 to 8 columns only where the
+// wide one does not fit (b = 130, r = 8: 1839 us against 2673 for the tiles).
 constexpr int BS_MAX_R = 8;
 
 // The wide sweep: full solves with b a multiple of its 16-row tiles.
 bool wd_fits(int64_t b, int partial) { return !partial && b >= WD_CW && b % WD_T == 0; }
 
-int pobtas_algo(int64_t b, int64_t a, int64_t r, int partial) {
+int pobtas_algo(int64_t n, int64_t b, int64_t a, int64_t r, int partial) {
   const char* e = getenv("ROCBTA_POBTAS_ALGO");
   if (e && strcmp(e, "loop") == 0) return SOLVE_LOOP;
   if (e && strcmp(e, "wide") == 0)
     return wd_fits(b, partial) ? SOLVE_WIDE : (partial ? SOLVE_LOOP : SOLVE_SWEEP);
   if (e && strcmp(e, "sweep") == 0) return partial ? SOLVE_LOOP : SOLVE_SWEEP;
   if (e && strcmp(e, "block") == 0) return bs_fits(a, r) ? SOLVE_BLOCK : (partial ? SOLVE_LOOP : SOLVE_SWEEP);
-  if (b >= BS_MIN_B && r <= BS_MAX_R && bs_fits(a, r)) return SOLVE_BLOCK;
-  if (b >= BS_MIN_B && r > BS_MAX_R && wd_fits(b, partial)) return SOLVE_WIDE;
+  if (b >= BS_MIN_B || n * (cdiv(b, SW_T) - 1) >= BS_MIN_SAVED) {
+    const bool wide = wd_fits(b, partial);
+    if (r <= (wide ? 4 : BS_MAX_R) && bs_fits(a, r)) return SOLVE_BLOCK;
+    if (wide) return SOLVE_WIDE;
+  }
   return partial ? SOLVE_LOOP : SOLVE_SWEEP;
 }
 
@@ -1306,9 +1317,9 @@ size_t rocbta_workspace_bytes(int op, int64_t n, int64_t b, int64_t a, int64_t r
       // enough for the algorithm the shape selects (partial or not)
       const int64_t rr = std::max<int64_t>(r, 1);
       size_t need = sw_layout(n, b, a, rr).total;
-      if (pobtas_algo(b, a, rr, 0) == SOLVE_BLOCK || pobtas_algo(b, a, rr, 1) == SOLVE_BLOCK)
+      if (pobtas_algo(n, b, a, rr, 0) == SOLVE_BLOCK || pobtas_algo(n, b, a, rr, 1) == SOLVE_BLOCK)
         need = std::max(need, bs_layout(n, b, a, rr).total);
-      if (pobtas_algo(b, a, rr, 0) == SOLVE_WIDE) need = std::max(need, wd_layout(n, b, a).total);
+      if (pobtas_algo(n, b, a, rr, 0) == SOLVE_WIDE) need = std::max(need, wd_layout(n, b, a).total);
       return need;
     }
     case ROCBTA_OP_LOGDET:
@@ -1647,7 +1658,7 @@ int rocbta_dpobtas(int64_t n, int64_t b, int64_t a, const double* D, const doubl
   if (trans != 'N' && trans != 'T' && trans != 'C') return ROCBTA_ERR_ARG;
   if (r == 0) return ROCBTA_OK;
   hipStream_t s = (hipStream_t)stream;
-  const int algo = pobtas_algo(b, a, r, partial);
+  const int algo = pobtas_algo(n, b, a, r, partial);
   if (algo == SOLVE_BLOCK) {
     if (!workspace || workspace_bytes < bs_layout(n, b, a, r).total) return ROCBTA_ERR_WORKSPACE;
     return pobtas_block(n, b, a, D, L, R, T, B, r, ldb, trans == 'N' ? 0 : 1, partial,
