@@ -153,7 +153,7 @@ int batched_enqueue(const BatchedPlan& p, hipStream_t s) {
   for (int w = 0; w < nfw; ++w) {
     const int m0 = p.fwave[w], nm = p.fwave[w + 1] - m0;
     pobtaf_chain_multi_kernel<<<std::max(nm + 1, p.chain_grid), CH_THREADS, 0, s>>>(
-        p.d_chains + m0, nm, p.d_gclaim + w, p.d_cu_busy + (int64_t)w * 4096);
+        p.d_chains + m0, nm, std::min(std::max(nm + 1, p.chain_grid), device_cus()), p.d_gclaim + w, p.d_cu_busy + (int64_t)w * 4096);
     RB_CHECK(hipGetLastError());
   }
   logdet_multi_kernel<<<p.nmat, 256, 0, s>>>(p.d_logdet);

@@ -41,6 +41,25 @@ __device__ __forceinline__ f32x4 mfma_acc(double a, double b, f32x4 c) {
 __device__ __forceinline__ int acc_row(const f64x4&, int lane, int r) { return acc_row_f64(lane, r); }
 __device__ __forceinline__ int acc_row(const f32x4&, int lane, int r) { return acc_row_f32(lane, r); }
 
+// Batched launches: matrix that helper workgroup idx of nhelp serves first.
+// Every matrix gets one helper; the others are dealt in proportion to the
+// matrices' work weight(m), so that a long matrix has as many as its chain can
+// use from the start.  Helpers past nhelp (those that start when others have
+// left) are dealt in turn.
+template <typename W>
+__device__ __forceinline__ int helper_home(int idx, int nhelp, int nmat, const W& weight) {
+  if (idx < nmat || idx >= nhelp) return idx % nmat;
+  double total = 0.0;
+  for (int m = 0; m < nmat; ++m) total += weight(m);
+  const double at = total * (idx - nmat + 0.5) / (nhelp - nmat);
+  double sum = 0.0;
+  for (int m = 0; m < nmat; ++m) {
+    sum += weight(m);
+    if (sum > at) return m;
+  }
+  return nmat - 1;
+}
+
 // Record an LAPACK-style failure index (1-based; smallest index wins; 0 = ok).
 __device__ __forceinline__ void record_info(int* info, int value) {
   if (!info) return;

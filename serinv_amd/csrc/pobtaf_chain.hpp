@@ -1213,14 +1213,18 @@ __global__ void __launch_bounds__(CH_THREADS) pobtaf_chain_kernel(PobtafChain P)
 }
 
 // Many independent matrices in one persistent launch (batched plans).  The
-// first nmat claims of *gclaim become the chains of matrices 0..nmat-1;
-// every other workgroup serves the matrices' helper queues round-robin,
-// taking each task from that matrix's own in-order counter, and leaves when
-// a full round finds every queue drained.  cu_busy (4096 ints, zero on
-// entry) marks the CUs that run a chain; helpers there leave at once.
+// first nmat claims of *gclaim become the chains of matrices 0..nmat-1; every
+// other workgroup serves one matrix's helper queue in order until it is
+// drained, then the next one's, and leaves when a full round finds every queue
+// drained.  It starts at its home (helper_home; nres: workgroups resident at
+// once).  With fewer helpers than matrices they go round after every task, so
+// that no chain waits for others to end.  Going round the matrices after every task instead left the longest
+// chain waiting for helpers: 24.7 ms for 64 systems of up to 1024 diagonal
+// tiles.  cu_busy (4096 ints, zero on entry) marks the CUs that run a chain;
+// helpers there leave at once.
 __global__ void __launch_bounds__(CH_THREADS) pobtaf_chain_multi_kernel(const PobtafChain* Ps,
-                                                                        int nmat, int* gclaim,
-                                                                        int* cu_busy) {
+                                                                        int nmat, int nres,
+                                                                        int* gclaim, int* cu_busy) {
   __shared__ __attribute__((aligned(16))) double lds[CH_LDS];
   __shared__ int s_task;
   const int tid = threadIdx.x;
@@ -1238,7 +1242,15 @@ __global__ void __launch_bounds__(CH_THREADS) pobtaf_chain_multi_kernel(const Po
       chain_run<1>(P, lds, lds + CT * TT_LD, lds + 2 * CT * TT_LD);
     return;
   }
-  int m = (int)(blockIdx.x % (unsigned)nmat);
+  if (tid == 0)
+    s_task = helper_home(first - nmat, nres - nmat, nmat, [&](int i) {
+      const double nt = Ps[i].nt;  // products of a step's tasks, and a part per task
+      return Ps[i].NT * (3.0 + nt * (5.0 + 3.0 * nt));
+    });
+  __syncthreads();
+  int m = s_task;
+  __syncthreads();
+  const bool stay = nres - nmat >= nmat;
   int drained = 0;  // consecutive matrices found without tasks
   while (drained < nmat) {
     const PobtafChain& P = Ps[m];
@@ -1252,11 +1264,12 @@ __global__ void __launch_bounds__(CH_THREADS) pobtaf_chain_multi_kernel(const Po
     if (task < 0) return;
     if (task >= P.ntasks) {
       ++drained;
+      m = (m + 1 == nmat) ? 0 : m + 1;
     } else {
       drained = 0;
       chain_helper_task<1>(P, task, lds);
+      if (!stay) m = (m + 1 == nmat) ? 0 : m + 1;
     }
-    m = (m + 1 == nmat) ? 0 : m + 1;
   }
 }
 

@@ -553,9 +553,10 @@ __global__ void __launch_bounds__(SW_THREADS) pobtas_sweep_kernel(SweepP P) {
 // Many independent systems in one persistent launch (batched plans): claims
 // below chain_begin[nmat] become the chains of (matrix, chunk) pairs
 // (chain_begin: prefix sums of the matrices' chunk counts); every other
-// workgroup serves the matrices' helper queues round-robin from each
-// matrix's own in-order counter and leaves when a full round finds every
-// queue drained.
+// workgroup serves one matrix's helper queue in order until it is drained,
+// then the next one's, starting at its home (helper_home), and leaves when a
+// full round finds every queue drained.  With fewer helpers than matrices they
+// go round after every task.
 template <int RC>
 __global__ void __launch_bounds__(SW_THREADS)
     pobtas_sweep_multi_kernel(const SweepP* Ps, const int* chain_begin, int nmat, int* gclaim) {
@@ -571,7 +572,15 @@ __global__ void __launch_bounds__(SW_THREADS)
     sw_chain<RC>(Ps[m], first - chain_begin[m], S);
     return;
   }
-  int m = (int)(blockIdx.x % (unsigned)nmat);
+  const int nchains = chain_begin[nmat];
+  if (threadIdx.x == 0)
+    s_task = helper_home(first - nchains, (int)gridDim.x - nchains, nmat, [&](int i) {
+      return Ps[i].NT * (1.0 + Ps[i].nt) * Ps[i].nchunks;
+    });
+  __syncthreads();
+  int m = s_task;
+  __syncthreads();
+  const bool stay = (int)gridDim.x - nchains >= nmat;
   int drained = 0;
   while (drained < nmat) {
     const SweepP& P = Ps[m];
@@ -581,13 +590,14 @@ __global__ void __launch_bounds__(SW_THREADS)
     __syncthreads();
     if (task >= P.ntasks) {
       ++drained;
+      m = (m + 1 == nmat) ? 0 : m + 1;
     } else {
       drained = 0;
       int chunk, g;
       const int kind = sw_decode(P, task, chunk, g);
       if (kind != SK_NOOP) sw_helper<RC>(P, kind, chunk, g, S);
+      if (!stay) m = (m + 1 == nmat) ? 0 : m + 1;
     }
-    m = (m + 1 == nmat) ? 0 : m + 1;
   }
 }
 
