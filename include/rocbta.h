@@ -370,6 +370,9 @@ int rocbta_dpobtasi_streaming(int64_t n, int64_t b, int64_t a, double* D, double
  * decode back to itself, a tile outside its array); 0 means the schedule is
  * deadlock-free and in bounds.  -1: shape not handled by that kernel. */
 int64_t rocbta_dag_selfcheck(int64_t n, int64_t b, int64_t a);
+/* The same for any arrow width; rocbta_dag_selfcheck covers arrows of one
+ * 64-row tile, the form whose tip is factored inside the launch. */
+int64_t rocbta_dag_selfcheck_arrows(int64_t n, int64_t b, int64_t a);
 
 #ifdef __cplusplus
 }

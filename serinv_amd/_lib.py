@@ -75,6 +75,7 @@ SIGNATURES = {
                                             [_c_p, _c_size, _c_p]),
     "rocbta_dlogdet": (_c_int, [_c_i64, _c_i64, _c_i64, _c_p, _c_p, _c_p, _c_p, _c_size, _c_p]),
     "rocbta_dag_selfcheck": (_c_i64, [_c_i64, _c_i64, _c_i64]),
+    "rocbta_dag_selfcheck_arrows": (_c_i64, [_c_i64, _c_i64, _c_i64]),
     "rocbta_mpobtaf": (_c_int, [_c_i64, _c_i64, _c_i64, _c_p, _c_p, _c_p, _c_p, _c_int, _c_p,
                                 _c_p, _c_size, _c_p]),
     "rocbta_mpobtasi": (_c_int, [_c_i64, _c_i64, _c_i64, _c_p, _c_p, _c_p, _c_p, _c_int, _c_p,

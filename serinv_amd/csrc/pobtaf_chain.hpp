@@ -16,9 +16,10 @@
 // PX(g) = X(g+1,g) minus the products of all columns k < g are prepared by
 // helpers.  Helper tasks:
 //   TRSM(r, j), r >= j + 2 : X(r,j) - sum_k L(r,k) L(j,k)^T, then * Linv(j)^T
-//   ARR(j)                 : the same for the arrow tile of column j
+//   ARR(j, q)              : the same for arrow tile q (64 arrow rows) of column j
 //   PX(g), PD(g)           : the partial sums above (stored in place)
 //   TIPP(i)                : P_i = R_i R_i^T;  TIP: chol(T - P_0 - ... - P_{n-1})
+//                            (arrows of one tile; wider ones leave the tip to the caller)
 // Helper tasks are taken from an atomic queue organised in stages; stage h
 // holds the tasks that need chain outputs of steps <= h - 1 only, and inside
 // a stage every task only waits on earlier slots.  The chain step g needs
@@ -42,7 +43,8 @@ struct PobtafChain {
   double* L;
   double* R;
   double* T;
-  int n, b, a, nt, ha;
+  int n, b, a, nt;
+  int na;       // arrow tiles of a column: ceil(a / 64)
   int NT;       // number of diagonal tiles (n * nt)
   int slots;    // helper slots per stage
   int nstages;  // NT + 2
@@ -61,16 +63,12 @@ struct PobtafChain {
   // FP64 operands to FP32 and accumulate in FP32 MFMA; the tiles stay FP64
   // in memory and the diagonal potrf / trtri and the tip run in FP64.
   int f32;
-  // Chain schedule for full 64-wide tiles (b % 64 == 0): the sub-diagonal
-  // solve is formed by column blocks around the tile factorization
-  // (chain_run_fused); 0 selects the step-after-step schedule (chain_run).
-  int fused;
   // Diagnostic timeline (nullptr normally): 100 MHz timestamps, CHAIN_TRACE_EV
   // per chain step g at trace[CHAIN_TRACE_EV * g + e], see chain_trace.
   long long* trace;
 };
 
-// Timeline events of the fused chain step g (diagnostic builds of a run):
+// Timeline events of chain step g (diagnostic builds of a run):
 //   0 step start, 1 factorization done, 2 Linv(g) released, PX(g)/PD(g+1)
 //   staged, 3 L(g+1,g) complete, 5 step end, 6 PX(g) published (by its helper), 7 L(g+2,g) published (by its helper).
 constexpr int CHAIN_TRACE_EV = 8;
@@ -123,10 +121,11 @@ __host__ __device__ __forceinline__ CTile tile_mirror(const PobtafChain& P, int 
   return {P.D + (int64_t)jb * b * b + (int64_t)jc * CT * b + (int64_t)rc * CT, b,
           cmin(CT, P.b - jc * CT), cmin(CT, P.b - rc * CT)};
 }
-__host__ __device__ __forceinline__ CTile tile_arrow(const PobtafChain& P, int j) {
+__host__ __device__ __forceinline__ CTile tile_arrow(const PobtafChain& P, int j, int q) {
   const int jb = j / P.nt, jc = j % P.nt;
   const int64_t b = P.b;
-  return {P.R + (int64_t)jb * P.a * b + (int64_t)jc * CT, b, P.a, cmin(CT, P.b - jc * CT)};
+  return {P.R + ((int64_t)jb * P.a + q * CT) * b + (int64_t)jc * CT, b, cmin(CT, P.a - q * CT),
+          cmin(CT, P.b - jc * CT)};
 }
 
 // ---------------------------------------------------------- task indexing
@@ -135,9 +134,10 @@ __host__ __device__ __forceinline__ CTile tile_arrow(const PobtafChain& P, int j
 //   1             PX(h)
 //   2             PD(h+1)
 //   3 .. 3+2nt-1  TRSM(j+3+q, j)
-//   3+2nt         ARR(j)
-//   4+2nt         TIPP(h/nt - 1) when h is a multiple of nt
-// stage NT+1, slot 0: TIP
+//   3+2nt+q       ARR(j, q), q < na
+//   slots - 1     TIPP(h/nt - 1) when h is a multiple of nt (na = 1)
+// stage NT+1, slot 0: TIP (na = 1)
+__host__ __device__ __forceinline__ int chain_slots(int nt, int na) { return 4 + 2 * nt + cmax(na, 1); }
 __host__ __device__ __forceinline__ int t_trsm(const PobtafChain& P, int r, int j) {
   const int h = j + 1;
   return h * P.slots + ((r == j + 2) ? 0 : 3 + (r - (j + 3)));
@@ -146,24 +146,24 @@ __host__ __device__ __forceinline__ int t_px(const PobtafChain& P, int g) { retu
 __host__ __device__ __forceinline__ int t_pd(const PobtafChain& P, int g) {
   return (g - 1) * P.slots + 2;
 }
-__host__ __device__ __forceinline__ int t_arr(const PobtafChain& P, int j) {
-  return (j + 1) * P.slots + 3 + 2 * P.nt;
+__host__ __device__ __forceinline__ int t_arr(const PobtafChain& P, int j, int q) {
+  return (j + 1) * P.slots + 3 + 2 * P.nt + q;
 }
 __host__ __device__ __forceinline__ int t_tippc(const PobtafChain& P, int i) {
-  return ((i + 1) * P.nt) * P.slots + 4 + 2 * P.nt;
+  return ((i + 1) * P.nt) * P.slots + P.slots - 1;
 }
 __host__ __device__ __forceinline__ int t_tipc(const PobtafChain& P) {
   return (P.NT + 1) * P.slots;
 }
 
 // Decode a helper task: kind, and (r, j) = output tile (TRSM), g in j (PX/PD),
-// column j (ARR), block i in j (TIPP).
+// arrow tile r of column j (ARR), block i in j (TIPP).
 __host__ __device__ __forceinline__ int chain_decode(const PobtafChain& P, int task, int& r,
                                                      int& j) {
   const int h = task / P.slots, slot = task % P.slots;
   r = 0;
   j = 0;
-  if (h == P.NT + 1) return (slot == 0 && P.ha) ? HK_TIP : HK_NOOP;
+  if (h == P.NT + 1) return (slot == 0 && P.na == 1) ? HK_TIP : HK_NOOP;
   const int jj = h - 1;
   if (slot == 0) {
     if (jj >= 0 && jj + 2 < band_end(P, jj)) {
@@ -196,29 +196,30 @@ __host__ __device__ __forceinline__ int chain_decode(const PobtafChain& P, int t
     }
     return HK_NOOP;
   }
-  if (slot == 3 + 2 * P.nt) {
-    if (P.ha && jj >= 0) {
+  if (slot < 3 + 2 * P.nt + P.na) {
+    if (jj >= 0) {
+      r = slot - (3 + 2 * P.nt);
       j = jj;
       return HK_ARR;
     }
     return HK_NOOP;
   }
-  if (slot == 4 + 2 * P.nt && P.ha && h >= P.nt && h % P.nt == 0) {
+  if (slot == P.slots - 1 && P.na == 1 && h >= P.nt && h % P.nt == 0) {
     j = h / P.nt - 1;
     return HK_TIPP;
   }
   return HK_NOOP;
 }
 
-// Readiness flag of the factor tile (r, k), r > k (arrow: r < 0).
+// Readiness flag of the factor tile (r, k), r > k (r < 0: arrow tile -1 - r).
 __host__ __device__ __forceinline__ int* factor_flag(const PobtafChain& P, int r, int k) {
-  if (r < 0) return P.hflags + t_arr(P, k);
+  if (r < 0) return P.hflags + t_arr(P, k, -1 - r);
   if (r == k + 1) return P.cflags + 2 * k + 1;
   return P.hflags + t_trsm(P, r, k);
 }
 
 // Contribution list of a helper task: columns k in [k0, k1) with operands
-// A = factor tile (ra, k) (ra < 0: arrow tile k) and B = factor tile (jb, k).
+// A = factor tile (ra, k) (ra < 0: arrow tile -1 - ra) and B = factor tile (jb, k).
 struct ContribRange {
   int ra, jb, k0, k1;
 };
@@ -228,7 +229,7 @@ __host__ __device__ __forceinline__ ContribRange chain_contribs(const PobtafChai
     case HK_TRSM:
       return {r, j, kmin_of(P, r / P.nt), j};
     case HK_ARR:
-      return {-1, j, kmin_of(P, j / P.nt), j};
+      return {-1 - r, j, kmin_of(P, j / P.nt), j};
     case HK_PX:
       return {j + 1, j, kmin_of(P, (j + 1) / P.nt), j};
     case HK_PD:
@@ -295,6 +296,7 @@ __device__ __forceinline__ void chain_publish(int* f, int publisher = 0) {
 
 // ----------------------------------------------------------- tile movement
 typedef double cdbl2 __attribute__((ext_vector_type(2)));
+typedef double cdbl2u __attribute__((ext_vector_type(2), aligned(8)));  // any double address
 
 // Thread t holds rows (t >> 5) + 8q (q = 0..7), columns 2*(t & 31) .. +1 of a
 // 64x64 tile: each wave load instruction covers two whole 512-byte rows.
@@ -304,13 +306,10 @@ struct TileRegs16 {
 
 __device__ __forceinline__ void tile_load16(const CTile& t, TileRegs16& x) {
   const int rs = threadIdx.x >> 5, c = (threadIdx.x & 31) * 2;
-  const bool fast = t.rows == CT && t.cols == CT &&
-                    ((reinterpret_cast<uintptr_t>(t.p) & 15) == 0) && ((t.ld & 1) == 0);
-  if (fast) {
+  if (t.rows == CT && t.cols == CT) {
 #pragma unroll
     for (int q = 0; q < 8; ++q)
-      x.v[q] = *reinterpret_cast<const cdbl2*>(
-          __builtin_assume_aligned(t.p + (int64_t)(rs + 8 * q) * t.ld + c, 16));
+      x.v[q] = *reinterpret_cast<const cdbl2u*>(t.p + (int64_t)(rs + 8 * q) * t.ld + c);
   } else {
 #pragma unroll
     for (int q = 0; q < 8; ++q) {
@@ -444,27 +443,26 @@ __device__ __forceinline__ void cacc_to_lds(const f64x4 (&acc)[2][2], double* X,
             acc[i][j][r];
 }
 
-// Store a tile staged in LDS (X[row * pitch + col]) to memory.  Full,
-// 16-byte aligned tiles: each thread reads its 8 row pairs (rows rs + 8q,
-// columns c, c + 1) first and then issues 16-byte stores; other tiles go
-// element by element.
+// Store a tile staged in LDS (X[row * pitch + col]) to memory: each thread
+// reads its 8 row pairs (rows rs + 8q, columns c, c + 1) first and then issues
+// the stores, 16 bytes each for full tiles.
 __device__ __forceinline__ void lds_tile_store(const double* X, int pitch, const CTile& t) {
-  const int tid = threadIdx.x;
-  if (t.rows == CT && t.cols == CT && (t.ld & 1) == 0 &&
-      (reinterpret_cast<uintptr_t>(t.p) & 15) == 0) {
-    const int rs = tid >> 5, c = (tid & 31) * 2;
-    cdbl2 v[8];
+  const int rs = threadIdx.x >> 5, c = (threadIdx.x & 31) * 2;
+  cdbl2 v[8];
+#pragma unroll
+  for (int q = 0; q < 8; ++q) {
+    v[q].x = X[(rs + 8 * q) * pitch + c];
+    v[q].y = X[(rs + 8 * q) * pitch + c + 1];
+  }
+  double* dst = t.p + (int64_t)rs * t.ld + c;
+  if (t.rows == CT && t.cols == CT) {
+#pragma unroll
+    for (int q = 0; q < 8; ++q) *reinterpret_cast<cdbl2u*>(dst + (int64_t)(8 * q) * t.ld) = v[q];
+  } else {
 #pragma unroll
     for (int q = 0; q < 8; ++q) {
-      v[q].x = X[(rs + 8 * q) * pitch + c];
-      v[q].y = X[(rs + 8 * q) * pitch + c + 1];
-    }
-#pragma unroll
-    for (int q = 0; q < 8; ++q) *reinterpret_cast<cdbl2*>(t.p + (int64_t)(rs + 8 * q) * t.ld + c) = v[q];
-  } else {
-    for (int idx = tid; idx < CT * CT; idx += CH_THREADS) {
-      const int row = idx >> 6, col = idx & 63;
-      if (row < t.rows && col < t.cols) t.p[(int64_t)row * t.ld + col] = X[row * pitch + col];
+      if (rs + 8 * q < t.rows && c < t.cols) dst[(int64_t)(8 * q) * t.ld] = v[q].x;
+      if (rs + 8 * q < t.rows && c + 1 < t.cols) dst[(int64_t)(8 * q) * t.ld + 1] = v[q].y;
     }
   }
 }
@@ -478,8 +476,8 @@ __device__ __forceinline__ void tile_zero(const CTile& t) {
 }
 
 // ------------------------------------------------------------ helper work
-// acc -= sum over the contribution range (A = factor tile (ra,k) or arrow
-// tile k, B = factor tile (jb,k)); operands prefetched one product ahead.
+// acc -= sum over the contribution range (A = factor tile (ra,k) or an arrow
+// tile of column k, B = factor tile (jb,k)); operands prefetched one product ahead.
 // TAG gives each kernel its own copy of the non-inlined workers, so that
 // each copy sees a single kind of descriptor pointer (kernel argument or
 // global array) and is optimised for it.
@@ -488,7 +486,7 @@ __device__ __forceinline__ void helper_products(const PobtafChain& P, const Cont
                                                 double sgn, bool lower_only, double* XA,
                                                 double* XB, ACC (&acc)[2][2]) {
   TileRegs16 ra, rb;
-  auto tileA = [&](int k) { return cr.ra < 0 ? tile_arrow(P, k) : tile_g(P, cr.ra, k); };
+  auto tileA = [&](int k) { return cr.ra < 0 ? tile_arrow(P, k, -1 - cr.ra) : tile_g(P, cr.ra, k); };
   __shared__ int s_ready;
   chain_wait(P, factor_flag(P, cr.ra, cr.k0), factor_flag(P, cr.jb, cr.k0));
   tile_load16(tileA(cr.k0), ra);
@@ -565,251 +563,6 @@ __device__ __forceinline__ void helper_solve(const PobtafChain& P, int j, double
 }
 
 // ------------------------------------------------------------- chain work
-// LDS plan of the chain workgroup: S [64][65] (potrf, then L(g+1,g) staged
-// K-contiguous with pitch 65 for the next step's update), Xs [64][65]
-// (Linv(g)), Ws [64][17] (trtri scratch).
-template <int TAG>
-__device__ __forceinline__ void chain_run(const PobtafChain& P, double* S, double* Xs, double* Ws) {
-  const int tid = threadIdx.x;
-  double (*S2)[TT_LD] = reinterpret_cast<double (*)[TT_LD]>(S);
-  double (*X2)[TT_LD] = reinterpret_cast<double (*)[TT_LD]>(Xs);
-  double (*W2)[WS_LD] = reinterpret_cast<double (*)[WS_LD]>(Ws);
-  const int lane = tid & 63, wave = tid >> 6;
-  const int wm = (wave >> 1) * 32, wn = (wave & 1) * 32;
-  const int li = lane & 15, lk = lane >> 4;
-  // Linv tiles keep zeros above their 16x16 block diagonal from here on
-  // (full-tile inversions never write there; ragged ones clear it).
-  for (int idx = tid; idx < CT * TT_LD; idx += CH_THREADS) Xs[idx] = 0.0;
-  __syncthreads();
-  // PD(g+1) is usually ready when the chain waits for PX(g): it is waited
-  // for together with PX(g) and loaded into registers (pd_next) then, so
-  // that the next step starts without the load latency.
-  f64x4 pd_next[2][2];
-  bool have_pd = false;
-  __shared__ int s_early;
-  // L(g+1,g) is stored at the end of step g but published during step g+1,
-  // after its syrk products have read the tile from LDS: the publish
-  // (every wave's store wait, a barrier, the release) then replaces the
-  // barrier that follows the products instead of adding one, and the
-  // release runs on wave 3, which has no work in the first panel of the
-  // tile factorization that follows.
-  int pending = -1;  // step whose L(g+1,g) stores are not yet published
-  constexpr int PUBLISHER = 3 * 64;
-  for (int g = 0; g < P.NT; ++g) {
-    const CTile dt = tile_g(P, g, g);
-    f64x4 acc[2][2];
-    if (have_pd) {
-#pragma unroll
-      for (int i = 0; i < 2; ++i)
-#pragma unroll
-        for (int j = 0; j < 2; ++j) acc[i][j] = pd_next[i][j];
-    } else {
-      if (g > 0) chain_wait(P, P.hflags + t_pd(P, g), nullptr);
-      cacc_load(dt, acc);
-    }
-    have_pd = false;
-    if (g > 0 && P.f32) {
-      f32x4 a32[2][2];
-      cacc32_zero(a32);
-      if (wn <= wm) {
-#pragma unroll 4
-        for (int kk = 0; kk < CT; kk += 4) {
-          const double a0 = -S[(wm + li) * TT_LD + kk + lk];
-          const double a1 = -S[(wm + 16 + li) * TT_LD + kk + lk];
-          const double b0 = S[(wn + li) * TT_LD + kk + lk];
-          const double b1 = S[(wn + 16 + li) * TT_LD + kk + lk];
-          a32[0][0] = mfma_acc(a0, b0, a32[0][0]);
-          a32[0][1] = mfma_acc(a0, b1, a32[0][1]);
-          a32[1][0] = mfma_acc(a1, b0, a32[1][0]);
-          a32[1][1] = mfma_acc(a1, b1, a32[1][1]);
-        }
-      }
-      if (pending >= 0) chain_publish(P.cflags + 2 * pending + 1, PUBLISHER);
-      pending = -1;
-      acc32_add(a32, acc, S, TT_LD);
-    } else if (g > 0) {
-      // acc -= L(g,g-1) L(g,g-1)^T, with L(g,g-1) in S as S[row][k]
-      if (wn <= wm) {
-#pragma unroll 4
-        for (int kk = 0; kk < CT; kk += 4) {
-          const double a0 = -S[(wm + li) * TT_LD + kk + lk];
-          const double a1 = -S[(wm + 16 + li) * TT_LD + kk + lk];
-          const double b0 = S[(wn + li) * TT_LD + kk + lk];
-          const double b1 = S[(wn + 16 + li) * TT_LD + kk + lk];
-          acc[0][0] = mfma_f64(a0, b0, acc[0][0]);
-          acc[0][1] = mfma_f64(a0, b1, acc[0][1]);
-          acc[1][0] = mfma_f64(a1, b0, acc[1][0]);
-          acc[1][1] = mfma_f64(a1, b1, acc[1][1]);
-        }
-      }
-      if (pending >= 0)
-        chain_publish(P.cflags + 2 * pending + 1, PUBLISHER);  // includes the barrier
-      else
-        __syncthreads();
-      pending = -1;
-    }
-    cacc_to_lds(acc, S, TT_LD);
-    __syncthreads();
-    const int m = dt.rows;
-    const bool sub = g + 1 < band_end(P, g);
-    const bool pre = sub && g + 1 < P.NT;
-    const int* f_px = P.hflags + t_px(P, g);
-    const int* f_pd = pre ? P.hflags + t_pd(P, g + 1) : f_px;
-    // Full tiles: the inverse Linv(g) is formed by 16-row block rows while
-    // the tile is factored.  Its diagonal blocks X_II come with the panels;
-    // the rest of block row I needs only panels 0 .. I, so waves 2 and 3
-    // form X_IJ = -X_II sum_K L_IK X_KJ (MFMA) of block rows 1 and 2 while
-    // wave 0 factors panels 2 and 3; block row 3 follows the factorization.
-    // PX(g) and PD(g+1) are normally published while the tile is factored.
-    // Wave 1 checks their flags while wave 0 factors the last panel and, if
-    // both are set, acquires; every thread then loads its parts of the two
-    // tiles after its L(g,g) stores (which would otherwise queue behind the
-    // loads), and the loads land during the rest of the inversion.
-    {
-      const int64_t row0 = (int64_t)(g / P.nt) * P.b + (int64_t)(g % P.nt) * CT;
-      if (m == CT) {
-        lds_potrf_t<CT>(S2, X2, CT, P.info, row0, [&](int p) {
-          if (p == 16 && wave == 2) wave_trtri_offdiag(S2, X2, &X2[16][16], TT_LD, 1, 0);
-          if (p == 32) {
-            if (wave == 1) {
-              int ok = sub ? (__hip_atomic_load(f_px, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) &
-                              __hip_atomic_load(f_pd, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT))
-                           : 0;
-              ok = __builtin_amdgcn_readfirstlane(ok);
-              if (ok) __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
-              if (lane == 0) s_early = ok;
-            } else if (wave == 2) {
-              wave_trtri_offdiag(S2, X2, &X2[32][32], TT_LD, 2, 1);
-            } else {
-              wave_trtri_offdiag(S2, X2, &X2[32][32], TT_LD, 2, 0);
-            }
-          }
-        });
-      } else {
-        if (tid == 0) s_early = 0;
-        lds_potrf_t<0>(S2, X2, m, P.info, row0);
-      }
-    }
-    const int early = s_early;
-    // L(g,g) to memory with its upper triangle zero.  Full tiles: each
-    // thread reads its 8 row pairs from LDS first, then issues 16-byte
-    // stores (rows rs + 8q, columns c, c + 1).
-    const int rs = tid >> 5, c2 = (tid & 31) * 2;
-    if (m == CT && (dt.ld & 1) == 0 && (reinterpret_cast<uintptr_t>(dt.p) & 15) == 0) {
-      cdbl2 v[8];
-#pragma unroll
-      for (int q = 0; q < 8; ++q) {
-        const int rr = rs + 8 * q;
-        v[q].x = (c2 <= rr) ? S2[rr][c2] : 0.0;
-        v[q].y = (c2 + 1 <= rr) ? S2[rr][c2 + 1] : 0.0;
-      }
-#pragma unroll
-      for (int q = 0; q < 8; ++q)
-        *reinterpret_cast<cdbl2*>(dt.p + (int64_t)(rs + 8 * q) * dt.ld + c2) = v[q];
-    } else {
-      for (int idx = tid; idx < CT * CT; idx += CH_THREADS) {
-        const int rr = idx >> 6, cc = idx & 63;
-        if (rr < m && cc < m) dt.p[(int64_t)rr * dt.ld + cc] = (cc <= rr) ? S2[rr][cc] : 0.0;
-      }
-    }
-    const CTile xt = tile_g(P, g + 1, g);
-    TileRegs16 rx;
-    if (early) {
-      tile_load16(xt, rx);
-      if (pre) cacc_load(tile_g(P, g + 1, g + 1), pd_next);
-    }
-    // Otherwise each wave reads both flags again now and checks them after
-    // the Linv publish: when both were set it only acquires, without the
-    // poll's round trip.
-    int seen = 0;
-    if (sub && !early)
-      seen = __hip_atomic_load(f_px, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) &
-             __hip_atomic_load(f_pd, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    if (m == CT) {
-      // block row 3: X_32, X_31, X_30
-      if (wave < 3) wave_trtri_offdiag(S2, X2, &X2[48][48], TT_LD, 3, 2 - wave);
-      __syncthreads();
-    } else {
-      lds_trtri<false>(S2, X2, W2, m);
-    }
-    double* li_out = P.linv + (int64_t)g * CT * CT;
-    {
-      cdbl2 v[8];
-#pragma unroll
-      for (int q = 0; q < 8; ++q) {
-        v[q].x = X2[rs + 8 * q][c2];
-        v[q].y = X2[rs + 8 * q][c2 + 1];
-      }
-#pragma unroll
-      for (int q = 0; q < 8; ++q)
-        *reinterpret_cast<cdbl2*>(li_out + (rs + 8 * q) * CT + c2) = v[q];
-    }
-    // Linv(g) is published before the sub-diagonal solve: the helpers'
-    // solves of column g (TRSM(g+2,g) feeds PX(g+1), which the next step
-    // waits for) start while the chain finishes this step.
-    chain_publish(P.cflags + 2 * g);
-    if (!sub) continue;
-    // L(g+1,g) = PX(g) * Linv(g)^T.  Each thread loads only its own parts of
-    // the two tiles, so the waves acquire independently; the barrier after
-    // the staging below orders the LDS.
-    if (!early) {
-      if (__builtin_amdgcn_readfirstlane(seen))
-        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
-      else
-        wave_wait(P, f_px, pre ? f_pd : nullptr);
-      tile_load16(xt, rx);
-      if (pre) cacc_load(tile_g(P, g + 1, g + 1), pd_next);
-    }
-    have_pd = pre;
-    {
-      // S[m][k] = X(m, k) (pitch 65 rows are 8-byte aligned only: scalar stores)
-      const int rs = tid >> 5, c = (tid & 31) * 2;
-#pragma unroll
-      for (int q = 0; q < 8; ++q) {
-        S[(rs + 8 * q) * TT_LD + c] = rx.v[q].x;
-        S[(rs + 8 * q) * TT_LD + c + 1] = rx.v[q].y;
-      }
-    }
-    __syncthreads();
-    cacc_zero(acc);
-    if (P.f32) {
-      f32x4 a32[2][2];
-      cacc32_zero(a32);
-#pragma unroll 4
-      for (int kk = 0; kk < CT; kk += 4) {
-        const double a0 = S[(wm + li) * TT_LD + kk + lk];
-        const double a1 = S[(wm + 16 + li) * TT_LD + kk + lk];
-        const double b0 = Xs[(wn + li) * TT_LD + kk + lk];  // Linv(n, k)
-        const double b1 = Xs[(wn + 16 + li) * TT_LD + kk + lk];
-        a32[0][0] = mfma_acc(a0, b0, a32[0][0]);
-        a32[0][1] = mfma_acc(a0, b1, a32[0][1]);
-        a32[1][0] = mfma_acc(a1, b0, a32[1][0]);
-        a32[1][1] = mfma_acc(a1, b1, a32[1][1]);
-      }
-      acc32_add(a32, acc, S, TT_LD);
-    } else {
-#pragma unroll 4
-      for (int kk = 0; kk < CT; kk += 4) {
-        const double a0 = S[(wm + li) * TT_LD + kk + lk];
-        const double a1 = S[(wm + 16 + li) * TT_LD + kk + lk];
-        const double b0 = Xs[(wn + li) * TT_LD + kk + lk];  // Linv(n, k)
-        const double b1 = Xs[(wn + 16 + li) * TT_LD + kk + lk];
-        acc[0][0] = mfma_f64(a0, b0, acc[0][0]);
-        acc[0][1] = mfma_f64(a0, b1, acc[0][1]);
-        acc[1][0] = mfma_f64(a1, b0, acc[1][0]);
-        acc[1][1] = mfma_f64(a1, b1, acc[1][1]);
-      }
-    }
-    __syncthreads();  // S no longer read as X
-    cacc_to_lds(acc, S, TT_LD);  // keep L(g+1,g) as S[row][k]
-    __syncthreads();
-    lds_tile_store(S, TT_LD, xt);
-    pending = g;
-  }
-  if (pending >= 0) chain_publish(P.cflags + 2 * pending + 1, PUBLISHER);
-}
-
-
 // Columns p .. p + 15 of the factored tile S to memory by the calling wave,
 // zeros above the diagonal.
 __device__ __forceinline__ void chain_store_panel(const double (*S)[TT_LD], int p, const CTile& t) {
@@ -822,16 +575,8 @@ __device__ __forceinline__ void chain_store_panel(const double (*S)[TT_LD], int 
     v[q].y = c + 1 <= r ? S[r][c + 1] : 0.0;
   }
   double* dst = t.p + (int64_t)(lane >> 3) * t.ld + c;
-  if ((t.ld & 1) == 0 && (reinterpret_cast<uintptr_t>(t.p) & 15) == 0) {
 #pragma unroll
-    for (int q = 0; q < 8; ++q) *reinterpret_cast<cdbl2*>(dst + 8 * q * t.ld) = v[q];
-  } else {
-#pragma unroll
-    for (int q = 0; q < 8; ++q) {
-      dst[8 * q * t.ld] = v[q].x;
-      dst[8 * q * t.ld + 1] = v[q].y;
-    }
-  }
+  for (int q = 0; q < 8; ++q) *reinterpret_cast<cdbl2u*>(dst + (int64_t)(8 * q) * t.ld) = v[q];
 }
 
 // Rows r0 .. r0 + 15 of Ps (64 x 64, K-contiguous) <- Ps Linv^T, by the calling
@@ -868,20 +613,28 @@ __device__ __forceinline__ void chain_blk(int wave, int i, int& rb, int& cb) {
   cb = wave == 0 ? (i == 2 ? 1 : 0) : (wave == 3 ? i + 2 : i);
 }
 
-// The calling wave's blocks of tile t (full tile), in the accumulator layout
-// of ACC.
+// The calling wave's blocks of the diagonal tile t, in the accumulator layout
+// of ACC; a ragged tile continues with the identity.
 template <typename ACC>
 __device__ __forceinline__ void chain_pd_load(const CTile& t, int wave, f64x4 (&pd)[3]) {
   const int lane = threadIdx.x & 63;
+  auto each = [&](auto&& value) {
 #pragma unroll
-  for (int i = 0; i < 3; ++i) {
-    if (i >= chain_nblk(wave)) break;
-    int rb, cb;
-    chain_blk(wave, i, rb, cb);
+    for (int i = 0; i < 3; ++i) {
+      if (i >= chain_nblk(wave)) break;
+      int rb, cb;
+      chain_blk(wave, i, rb, cb);
 #pragma unroll
-    for (int r = 0; r < 4; ++r)
-      pd[i][r] = t.p[(int64_t)(16 * rb + acc_row(ACC{}, lane, r)) * t.ld + 16 * cb + acc_col(lane)];
-  }
+      for (int r = 0; r < 4; ++r)
+        pd[i][r] = value(16 * rb + acc_row(ACC{}, lane, r), 16 * cb + acc_col(lane));
+    }
+  };
+  if (t.rows == CT)
+    each([&](int row, int col) { return t.p[(int64_t)row * t.ld + col]; });
+  else
+    each([&](int row, int col) {
+      return row < t.rows && col < t.rows ? t.p[(int64_t)row * t.ld + col] : (row == col ? 1.0 : 0.0);
+    });
 }
 
 // The calling wave's blocks of Sn <- pd - Ps Ps^T.
@@ -927,9 +680,8 @@ __device__ __forceinline__ void chain_syrk(const double* Ps, const f64x4 (&pd)[3
   }
 }
 
-// ------------------------------------------------------- fused chain step
-// Chain schedule for matrices whose diagonal tiles are all full (b % 64 ==
-// 0).  Step g starts with D(g,g) fully updated in S and:
+// ------------------------------------------------------------- chain step
+// Step g starts with D(g,g) fully updated in S and:
 //   1. factors it (wave 0 factors the 16-column panels; waves 1-3 update the
 //      trailing columns and form block rows 1 and 2 of Linv(g) beside them;
 //      the diagonal blocks of Linv(g) come with the panels);
@@ -941,11 +693,65 @@ __device__ __forceinline__ void chain_syrk(const double* Ps, const f64x4 (&pd)[3
 // L(g+1,g) is released at the start of step g+1, whose first panel only wave
 // 0 works on.  In the mixed mode the products of steps 3 and 4 round their
 // operands to FP32 and accumulate in FP32; the PD(g+1) term stays FP64.
+// A ragged tile (the last of a block when b % 64 != 0) runs padded with the
+// identity to 64: PX comes with zeros past its rows and columns, so the
+// padding stays what it is through steps 3 and 4, and only the 16-column
+// panels that hold columns of the matrix are factored (chain_factor_ragged).
+// Measured against a schedule of their own with ragged tile routines: n = 100,
+// b = 130, a = 0 4.26 (5.22) ms, n = 8, b = 96, a = 12 248 (354) us.
+// Arrows of more than one tile add helper tasks only: n = 24, b = 200, a = 70
+// 1.39 ms, 3.9 ms launch per tile.
 // LDS: two D buffers [64][65] (D(g,g) -> L(g,g), and D(g+1,g+1)), Xs
 // [64][65] (Linv(g)), Ps [64][65] (PX(g) -> L(g+1,g), row-major =
 // K-contiguous).
+//
+// chain_factor_ragged: L(g,g) of m < 64 columns in S, Linv(g) in X2 (the
+// identity past m), L(g,g) to memory; wave 3 looks at the flags of PX(g) and
+// PD(g+1) meanwhile.  Returns with every wave past the last write of X2.
 template <int TAG>
-__device__ __forceinline__ void chain_run_fused(const PobtafChain& P, double* Sa, double* Sb,
+__device__ __forceinline__ void chain_factor_ragged(const PobtafChain& P, double (*S2)[TT_LD],
+                                                    double (*X2)[TT_LD], int m, int64_t row0,
+                                                    const CTile& dt, bool sub, const int* f_px,
+                                                    const int* f_pd, int* s_early) {
+  const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int pe = (m + PW - 1) / PW * PW;  // columns factored
+  for (int idx = pe * CT + tid; idx < CT * CT; idx += CH_THREADS)
+    X2[idx / CT][idx % CT] = idx / CT == idx % CT ? 1.0 : 0.0;
+#pragma unroll 1
+  for (int p = 0; p < pe; p += PW) {
+    if (wave == 0) {
+      WavePanel16<true> w;
+      w.factor(S2, p, TT);
+      w.finish(S2, p, &X2[p][p], TT_LD, P.info, row0);
+    }
+    __syncthreads();
+    if (p + PW < pe) {
+      lds_syrk_cols(S2, p, p + PW, pe, 0, 4);
+      __syncthreads();
+    }
+  }
+#pragma unroll 1
+  for (int I = 1; I < pe / PW; ++I) {
+    if (wave < I) wave_trtri_offdiag(S2, X2, &X2[PW * I][PW * I], TT_LD, I, wave);
+    __syncthreads();
+  }
+  if (wave == 3) {
+    int ok = sub ? (__hip_atomic_load(f_px, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) &
+                    __hip_atomic_load(f_pd, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT))
+                 : 0;
+    ok = __builtin_amdgcn_readfirstlane(ok);
+    if (ok) __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
+    if ((tid & 63) == 0) *s_early = ok;
+  }
+  for (int idx = tid; idx < m * CT; idx += CH_THREADS) {
+    const int r = idx / CT, c = idx % CT;
+    if (c < m) dt.p[(int64_t)r * dt.ld + c] = c <= r ? S2[r][c] : 0.0;
+  }
+  __syncthreads();
+}
+
+template <int TAG>
+__device__ __forceinline__ void chain_run(const PobtafChain& P, double* Sa, double* Sb,
                                                 double* Xs, double* Ps) {
   const int tid = threadIdx.x;
   double (*X2)[TT_LD] = reinterpret_cast<double (*)[TT_LD]>(Xs);
@@ -957,6 +763,9 @@ __device__ __forceinline__ void chain_run_fused(const PobtafChain& P, double* Sa
     f64x4 acc[2][2];
     cacc_load(tile_g(P, 0, 0), acc);  // D(0,0) has no updates
     cacc_to_lds(acc, Sa, TT_LD);
+    __syncthreads();
+    const int m0 = cmin(CT, P.b);
+    if (tid >= m0 && tid < CT) Sa[tid * TT_LD + tid] = 1.0;
   }
   __syncthreads();
   __shared__ int s_early;
@@ -982,7 +791,8 @@ __device__ __forceinline__ void chain_run_fused(const PobtafChain& P, double* Sa
     //    finished panels beside it; PX(g) and PD(g+1) flags checked by wave 1
     //    during the last panel
     const int64_t row0 = (int64_t)(g / P.nt) * P.b + (int64_t)(g % P.nt) * CT;
-    lds_potrf_t<CT>(S2, X2, CT, P.info, row0, [&](int p) {
+    const int m = dt.rows;
+    if (m == CT) lds_potrf_t<CT>(S2, X2, CT, P.info, row0, [&](int p) {
       if (p < 32) {
         if (wave == 3) chain_store_panel(S2, p, dt);
         if (p == 16 && wave == 2) wave_trtri_offdiag(S2, X2, &X2[16][16], TT_LD, 1, 0);
@@ -1000,6 +810,8 @@ __device__ __forceinline__ void chain_run_fused(const PobtafChain& P, double* Sa
         wave_trtri_offdiag(S2, X2, &X2[32][32], TT_LD, 2, wave == 2 ? 1 : 0);
       }
     });
+    else
+      chain_factor_ragged<TAG>(P, S2, X2, m, row0, dt, sub, f_px, f_pd, &s_early);
     const int early = s_early;
     chain_trace(P, g, 1);
     // PX(g) and PD(g+1), if both were published during the factorization: the
@@ -1023,11 +835,13 @@ __device__ __forceinline__ void chain_run_fused(const PobtafChain& P, double* Sa
     };
     if (early) load_px();
     // 2. Linv block row 3; the last panel of L(g,g) and Linv(g) to memory
-    if (wave >= 1)
-      wave_trtri_offdiag(S2, X2, &X2[48][48], TT_LD, 3, wave - 1);
-    else
-      chain_store_panel(S2, 48, dt);
-    __syncthreads();
+    if (m == CT) {
+      if (wave >= 1)
+        wave_trtri_offdiag(S2, X2, &X2[48][48], TT_LD, 3, wave - 1);
+      else
+        chain_store_panel(S2, 48, dt);
+      __syncthreads();
+    }
     double* li_out = P.linv + (int64_t)g * CT * CT;
     {
       cdbl2 v[8];
@@ -1035,6 +849,13 @@ __device__ __forceinline__ void chain_run_fused(const PobtafChain& P, double* Sa
       for (int q = 0; q < 8; ++q) {
         v[q].x = X2[rs + 8 * q][c2];
         v[q].y = X2[rs + 8 * q][c2 + 1];
+      }
+      if (m < CT) {  // zeros past a ragged tile's rows and columns
+#pragma unroll
+        for (int q = 0; q < 8; ++q) {
+          if (rs + 8 * q >= m || c2 >= m) v[q].x = 0.0;
+          if (rs + 8 * q >= m || c2 + 1 >= m) v[q].y = 0.0;
+        }
       }
 #pragma unroll
       for (int q = 0; q < 8; ++q) *reinterpret_cast<cdbl2*>(li_out + (rs + 8 * q) * CT + c2) = v[q];
@@ -1100,14 +921,30 @@ __device__ __forceinline__ void chain_helper_task(const PobtafChain& P, int task
   f64x4 acc[2][2];
   if (kind == HK_TIP) {
     cacc_load({P.T, P.a, P.a, P.a}, acc);
-    for (int i = 0; i < P.n; ++i) {
-      chain_wait(P, P.hflags + t_tippc(P, i), nullptr);
-      f64x4 pi[2][2];
-      cacc_load({P.tipp + (int64_t)i * P.a * P.a, P.a, P.a, P.a}, pi);
+    // four products a round: one round trip for their loads
+    for (int i0 = 0; i0 < P.n; i0 += 4) {
+      f64x4 pi[4][2][2];
+      if (tid == 0) {
+        long long spins = 0;
+        for (int i = i0; i < i0 + 4 && i < P.n; ++i)
+          if (!chain_poll(P, P.hflags + t_tippc(P, i), spins)) {
+            __hip_atomic_store(P.info, -1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            break;
+          }
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
+      }
+      __syncthreads();
 #pragma unroll
-      for (int x = 0; x < 2; ++x)
+      for (int u = 0; u < 4; ++u)
+        if (i0 + u < P.n) cacc_load({P.tipp + (int64_t)(i0 + u) * P.a * P.a, P.a, P.a, P.a}, pi[u]);
 #pragma unroll
-        for (int y = 0; y < 2; ++y) acc[x][y] -= pi[x][y];
+      for (int u = 0; u < 4; ++u)
+        if (i0 + u < P.n) {
+#pragma unroll
+          for (int x = 0; x < 2; ++x)
+#pragma unroll
+            for (int y = 0; y < 2; ++y) acc[x][y] -= pi[u][x][y];
+        }
     }
     double (*S2)[TT_LD] = reinterpret_cast<double (*)[TT_LD]>(lds);
     cacc_to_lds(acc, lds, TT_LD);
@@ -1135,9 +972,9 @@ __device__ __forceinline__ void chain_helper_task(const PobtafChain& P, int task
     cacc_zero(acc);
     for (int c = 0; c < P.nt; ++c) {
       const int k = i * P.nt + c;
-      chain_wait(P, P.hflags + t_arr(P, k), nullptr);
+      chain_wait(P, P.hflags + t_arr(P, k, 0), nullptr);
       TileRegs16 x;
-      tile_load16(tile_arrow(P, k), x);
+      tile_load16(tile_arrow(P, k, 0), x);
       __syncthreads();
       tile_store16(x, XA);
       __syncthreads();
@@ -1151,7 +988,7 @@ __device__ __forceinline__ void chain_helper_task(const PobtafChain& P, int task
   if (kind == HK_TRSM)
     out = tile_g(P, r, j);
   else if (kind == HK_ARR)
-    out = tile_arrow(P, j);
+    out = tile_arrow(P, j, r);
   else if (kind == HK_PX)
     out = tile_g(P, j + 1, j);
   else
@@ -1174,11 +1011,11 @@ __device__ __forceinline__ void chain_helper_task(const PobtafChain& P, int task
   if (kind == HK_PX && (j + 1) / P.nt == j / P.nt) tile_zero(tile_mirror(P, j + 1, j));
 }
 
-// LDS of the single-matrix kernel: the helper plan (XA, XB) or the chain's
-// (S, Xs, Ws; fused: two D buffers, Xs, Ps), whichever is larger.
+// LDS: the helper plan (XA, XB) or the chain's (two D buffers, Xs, Ps),
+// whichever is larger.
 constexpr int CH_LDS_HELPER = 2 * CT * KP + CT * WS_LD;
-constexpr int CH_LDS_FUSED = 4 * CT * TT_LD;
-constexpr int CH_LDS = CH_LDS_HELPER > CH_LDS_FUSED ? CH_LDS_HELPER : CH_LDS_FUSED;
+constexpr int CH_LDS_CHAIN = 4 * CT * TT_LD;
+constexpr int CH_LDS = CH_LDS_HELPER > CH_LDS_CHAIN ? CH_LDS_HELPER : CH_LDS_CHAIN;
 
 __global__ void __launch_bounds__(CH_THREADS) pobtaf_chain_kernel(PobtafChain P) {
   __shared__ __attribute__((aligned(16))) double lds[CH_LDS];
@@ -1192,10 +1029,7 @@ __global__ void __launch_bounds__(CH_THREADS) pobtaf_chain_kernel(PobtafChain P)
     // the chain runs latency-bound code: keep helpers off its CU
     if (tid == 0)
       __hip_atomic_store(P.chain_cu, 1 + hw_cu_key(), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    if (P.fused)
-      chain_run_fused<0>(P, lds, lds + CT * TT_LD, lds + 2 * CT * TT_LD, lds + 3 * CT * TT_LD);
-    else
-      chain_run<0>(P, lds, lds + CT * TT_LD, lds + 2 * CT * TT_LD);
+    chain_run<0>(P, lds, lds + CT * TT_LD, lds + 2 * CT * TT_LD, lds + 3 * CT * TT_LD);
     return;
   }
   const int my_cu = 1 + hw_cu_key();
@@ -1236,10 +1070,7 @@ __global__ void __launch_bounds__(CH_THREADS) pobtaf_chain_multi_kernel(const Po
   if (first < nmat) {
     if (tid == 0) __hip_atomic_store(cu_busy + my_key, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     const PobtafChain& P = Ps[first];
-    if (P.fused)
-      chain_run_fused<1>(P, lds, lds + CT * TT_LD, lds + 2 * CT * TT_LD, lds + 3 * CT * TT_LD);
-    else
-      chain_run<1>(P, lds, lds + CT * TT_LD, lds + 2 * CT * TT_LD);
+    chain_run<1>(P, lds, lds + CT * TT_LD, lds + 2 * CT * TT_LD, lds + 3 * CT * TT_LD);
     return;
   }
   if (tid == 0)

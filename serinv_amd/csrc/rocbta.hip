@@ -501,14 +501,15 @@ SiLayout si_layout(int64_t n, int64_t b, int64_t a) {
 
 struct AfLayout {
   size_t tinv, counter, claim, chain_cu, hflags, cflags, linv, tipp, save_d, save_r, save_t, total;
-  int nt, NT, slots, nstages, ntasks;
+  int nt, na, NT, slots, nstages, ntasks;
 };
 
 AfLayout af_layout(int64_t n, int64_t b, int64_t a) {
   AfLayout l{};
   l.nt = (int)((b + CT - 1) / CT);
   l.NT = (int)(n * l.nt);
-  l.slots = 5 + 2 * l.nt;
+  l.na = (int)((a + CT - 1) / CT);
+  l.slots = chain_slots(l.nt, l.na);
   l.nstages = l.NT + 2;
   l.ntasks = l.nstages * l.slots;
   size_t off = 0;
@@ -548,11 +549,10 @@ int device_cus() {
 }
 
 // ROCBTA_POBTAF_ALGO=loop forces the launch-per-tile path (used by tests to
-// cover both paths); default: the persistent chain kernel whenever it applies.
-bool pobtaf_use_chain(int64_t a) {
+// cover both paths); default: the persistent chain kernel.
+bool pobtaf_use_chain() {
   const char* e = getenv("ROCBTA_POBTAF_ALGO");
-  if (e && strcmp(e, "loop") == 0) return false;
-  return a <= CT;
+  return !(e && strcmp(e, "loop") == 0);
 }
 
 // info = 0 where it names a row of the last block or of the tip (rows past
@@ -562,9 +562,8 @@ __global__ void clear_info_above_kernel(int* info, int64_t first_open) {
 }
 
 // T = T0 - sum_{i < nblk} tipp[i], summed in block order (the order the
-// chain's tip task uses).  The chain forms only the lower part of each
-// symmetric tipp[i] (its upper-right 32 x 32 quadrant stays zero), so both
-// (r, s) and (s, r) take the lower entry.
+// chain's tip task uses).  Only the lower part of each symmetric tipp[i] is
+// formed, so both (r, s) and (s, r) take the lower entry.  T may be T0.
 __global__ void tip_open_kernel(double* T, const double* T0, const double* tipp, int a, int nblk) {
   const int aa = a * a;
   for (int idx = blockIdx.x * blockDim.x + threadIdx.x; idx < aa; idx += gridDim.x * blockDim.x) {
@@ -587,7 +586,7 @@ PobtafChain chain_params(int64_t n, int64_t b, int64_t a, double* D, double* L, 
   P.b = (int)b;
   P.a = (int)a;
   P.nt = lay.nt;
-  P.ha = a > 0 ? 1 : 0;
+  P.na = lay.na;
   P.NT = lay.NT;
   P.slots = lay.slots;
   P.nstages = lay.nstages;
@@ -604,10 +603,6 @@ PobtafChain chain_params(int64_t n, int64_t b, int64_t a, double* D, double* L, 
   P.info = info;
   P.spin_limit = 1ll << 22;
   P.f32 = g_mixed ? 1 : 0;
-  // ROCBTA_CHAIN=classic keeps the step-after-step chain schedule
-  const char* e = getenv("ROCBTA_CHAIN");
-  const bool classic = e && strcmp(e, "classic") == 0;
-  P.fused = (!classic && b % CT == 0) ? 1 : 0;
   P.trace = nullptr;
   return P;
 }
@@ -653,8 +648,8 @@ int pobtaf_chain(int64_t n, int64_t b, int64_t a, double* D, double* L, double* 
     RB_CHECK(hipStreamSynchronize(s));
     RB_CHECK(hipMemcpy(h.data(), P.trace, nev * sizeof(long long), hipMemcpyDeviceToHost));
     if (FILE* f = fopen(trace_path, "a")) {
-      fprintf(f, "# chain trace n=%lld b=%lld a=%lld NT=%d fused=%d\n", (long long)n, (long long)b,
-              (long long)a, P.NT, P.fused);
+      fprintf(f, "# chain trace n=%lld b=%lld a=%lld NT=%d\n", (long long)n, (long long)b,
+              (long long)a, P.NT);
       for (int g = 0; g < P.NT; ++g) {
         for (int e = 0; e < CHAIN_TRACE_EV; ++e) fprintf(f, "%lld ", h[(size_t)CHAIN_TRACE_EV * g + e]);
         fprintf(f, "\n");
@@ -1362,9 +1357,25 @@ int rocbta_dpobtaf(int64_t n, int64_t b, int64_t a, double* D, double* L, double
   const int bi = (int)b, ai = (int)a;
   const int64_t bb = b * b, ab = a * b;
   if (!factorize_last_block && n == 1) return ROCBTA_OK;  // no block row to eliminate
-  if (pobtaf_use_chain(a)) {
+  if (pobtaf_use_chain()) {
     char* ws = (char*)workspace;
-    if (factorize_last_block) return pobtaf_chain(n, b, a, D, L, R, T, info, ws, lay, s);
+    // Arrows of more than one tile: the launch leaves the tip alone and
+    // T - sum_{i < nblk} L_{t,i} L_{t,i}^T takes one batched product after it.
+    double* tipp = (double*)(ws + lay.tipp);
+    auto tip_products = [&](int64_t nblk) -> int {
+      GemmList pr;
+      push_term(pr.add(tipp, a, ai, ai, 0.0, TRI_LOWER, (int)nblk, a * a),
+                term(R, b, false, R, b, true, bi, 1.0, TRI_NONE, TRI_NONE, ab, ab));
+      return run_gemms(pr, s);
+    };
+    if (factorize_last_block) {
+      int rc = pobtaf_chain(n, b, a, D, L, R, T, info, ws, lay, s);
+      if (rc || lay.na <= 1) return rc;
+      if ((rc = tip_products(n))) return rc;
+      tip_open_kernel<<<cdiv(a * a, 256), 256, 0, s>>>(T, T, tipp, ai, (int)n);
+      RB_CHECK(hipGetLastError());
+      return factor_block_column(T, a, ai, {}, n * b, info, tinv, s);
+    }
     // pobtaf.py:143-159 leaves D_{n-1}, R_{n-1} and T Schur-updated but not
     // factored.  The chain factors them too; they are rebuilt afterwards
     // from the values given: D_{n-1} - L_{n-1,n-2} L_{n-1,n-2}^T, R_{n-1} -
@@ -1394,8 +1405,8 @@ int rocbta_dpobtaf(int64_t n, int64_t b, int64_t a, double* D, double* L, double
     rc = run_gemms(upd, s);
     if (rc) return rc;
     if (a > 0) {
-      tip_open_kernel<<<cdiv(a * a, 256), 256, 0, s>>>(T, st, (double*)(ws + lay.tipp), ai,
-                                                      (int)(n - 1));
+      if (lay.na > 1 && (rc = tip_products(n - 1))) return rc;
+      tip_open_kernel<<<cdiv(a * a, 256), 256, 0, s>>>(T, st, tipp, ai, (int)(n - 1));
       RB_CHECK(hipGetLastError());
     }
     return ROCBTA_OK;
@@ -1725,7 +1736,11 @@ int rocbta_dpobtas(int64_t n, int64_t b, int64_t a, const double* D, const doubl
 }
 
 int64_t rocbta_dag_selfcheck(int64_t n, int64_t b, int64_t a) {
-  if (bad_shape(n, b, a) || a > CT) return -1;
+  return a > CT ? -1 : rocbta_dag_selfcheck_arrows(n, b, a);
+}
+
+int64_t rocbta_dag_selfcheck_arrows(int64_t n, int64_t b, int64_t a) {
+  if (bad_shape(n, b, a)) return -1;
   const AfLayout lay = af_layout(n, b, a);
   double* const base = reinterpret_cast<double*>(uintptr_t(1) << 40);
   int* const fbase = reinterpret_cast<int*>(uintptr_t(1) << 44);
@@ -1770,19 +1785,19 @@ int64_t rocbta_dag_selfcheck(int64_t n, int64_t b, int64_t a) {
     if (kind == HK_TIPP) {
       if (t != t_tippc(P, j)) ++bad;
       for (int c = 0; c < P.nt; ++c)
-        if (!wait_ok(P.hflags + t_arr(P, j * P.nt + c), t)) ++bad;
+        if (!wait_ok(P.hflags + t_arr(P, j * P.nt + c, 0), t)) ++bad;
       continue;
     }
     int back = -1;
     if (kind == HK_TRSM) back = t_trsm(P, r, j);
-    if (kind == HK_ARR) back = t_arr(P, j);
+    if (kind == HK_ARR) back = t_arr(P, j, r);
     if (kind == HK_PX) back = t_px(P, j);
     if (kind == HK_PD) back = t_pd(P, j);
     if (back != t) ++bad;
     if (kind == HK_TRSM && !(r >= j + 2 && r < band_end(P, j))) ++bad;
     const ContribRange cr = chain_contribs(P, kind, r, j);
     for (int k = cr.k0; k < cr.k1; ++k) {
-      const CTile ta = cr.ra < 0 ? tile_arrow(P, k) : tile_g(P, cr.ra, k);
+      const CTile ta = cr.ra < 0 ? tile_arrow(P, k, -1 - cr.ra) : tile_g(P, cr.ra, k);
       if (!tile_ok(ta) || !tile_ok(tile_g(P, cr.jb, k))) ++bad;
       if (!wait_ok(factor_flag(P, cr.ra, k), t) || !wait_ok(factor_flag(P, cr.jb, k), t)) ++bad;
       if (cr.ra >= 0 && !(cr.ra > k)) ++bad;
@@ -1790,7 +1805,7 @@ int64_t rocbta_dag_selfcheck(int64_t n, int64_t b, int64_t a) {
     }
     if ((kind == HK_TRSM || kind == HK_ARR) && !wait_ok(P.cflags + 2 * j, t)) ++bad;
     CTile out = kind == HK_TRSM ? tile_g(P, r, j)
-                : kind == HK_ARR ? tile_arrow(P, j)
+                : kind == HK_ARR ? tile_arrow(P, j, r)
                 : kind == HK_PX  ? tile_g(P, j + 1, j)
                                  : tile_g(P, j, j);
     if (!tile_ok(out)) ++bad;
@@ -1814,7 +1829,7 @@ int64_t rocbta_dag_selfcheck(int64_t n, int64_t b, int64_t a) {
   }
   // every lower band tile is produced exactly once (chain or helper)
   int64_t expect = 0;
-  for (int j = 0; j < P.NT; ++j) expect += std::max(0, band_end(P, j) - (j + 2)) + (P.ha ? 1 : 0);
+  for (int j = 0; j < P.NT; ++j) expect += std::max(0, band_end(P, j) - (j + 2)) + P.na;
   int64_t got = 0;
   for (int t = 0; t < P.ntasks; ++t) {
     int r, j;
