@@ -26,8 +26,12 @@
 // PD(g) (stage g-1) and PX(g) (stage g), so no wait can cycle.  Every wait is
 // bounded: an overrun sets info = -1 and makes all later waits return.
 //
-// Memory ordering: tiles are published with an agent-scope release before
-// the flag store; waiters poll relaxed and issue one agent-scope acquire.
+// Memory ordering: helpers publish a tile with an agent-scope release before
+// the flag store.  The chain's tiles are written through (agent-scope stores),
+// each wave adding its share to the flag once its own stores are complete: no
+// barrier and no cache write-back on the chain's path.  A tile is ready when
+// its flag holds CH_READY; waiters poll relaxed and issue one agent-scope
+// acquire.
 #pragma once
 #include "common.hpp"
 #include "tile_f64.hpp"
@@ -37,6 +41,7 @@ namespace rocbta {
 constexpr int CT = 64;          // tile size
 constexpr int CH_THREADS = 256;
 constexpr int KP = CT + 2;      // pitch of K-contiguous LDS tiles (doubles)
+constexpr int CH_READY = 12;    // flag of a published tile
 
 struct PobtafChain {
   double* D;
@@ -69,7 +74,7 @@ struct PobtafChain {
 };
 
 // Timeline events of chain step g (diagnostic builds of a run):
-//   0 step start, 1 factorization done, 2 Linv(g) released, PX(g)/PD(g+1)
+//   0 step start, 1 factorization done, 2 Linv(g) complete, PX(g)/PD(g+1)
 //   staged, 3 L(g+1,g) complete, 5 step end, 6 PX(g) published (by its helper), 7 L(g+2,g) published (by its helper).
 constexpr int CHAIN_TRACE_EV = 8;
 __device__ __forceinline__ void chain_trace(const PobtafChain& P, int g, int e) {
@@ -240,8 +245,11 @@ __host__ __device__ __forceinline__ ContribRange chain_contribs(const PobtafChai
 }
 
 // ---------------------------------------------------------------- flags
+__device__ __forceinline__ bool chain_ready(const int* f) {
+  return __hip_atomic_load(f, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) >= CH_READY;
+}
 __device__ __forceinline__ bool chain_poll(const PobtafChain& P, const int* f, long long& spins) {
-  while (__hip_atomic_load(f, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == 0) {
+  while (!chain_ready(f)) {
     if (++spins > P.spin_limit) return false;
     if ((spins & 255) == 0 &&
         __hip_atomic_load(P.info, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) < 0)
@@ -284,14 +292,21 @@ __device__ __forceinline__ void wave_stores_done() { __builtin_amdgcn_s_waitcnt(
 // The explicit wait after thread 0's release fence keeps the flag store
 // behind the completion of the L2 write-back: with the counters already
 // drained, the compiler otherwise emits no wait between the two.
-__device__ __forceinline__ void chain_publish(int* f, int publisher = 0) {
+__device__ __forceinline__ void chain_publish(int* f) {
   wave_stores_done();
   __syncthreads();
-  if ((int)threadIdx.x == publisher) {
+  if (threadIdx.x == 0) {
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "agent");
     wave_stores_done();
-    __hip_atomic_store(f, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    __hip_atomic_store(f, CH_READY, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
   }
+}
+
+// The calling wave's share of a tile that several waves write through.
+__device__ __forceinline__ void chain_wave_done(int* f, int share) {
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // also keeps the stores above it
+  if ((threadIdx.x & 63) == 0)
+    __hip_atomic_fetch_add(f, share, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
 // ----------------------------------------------------------- tile movement
@@ -467,6 +482,48 @@ __device__ __forceinline__ void lds_tile_store(const double* X, int pitch, const
   }
 }
 
+// 16 bytes written through to where every XCD reads them (agent scope).  The
+// wait state keeps the data registers until the store has taken them.
+__device__ __forceinline__ void store_through(double* p, const cdbl2& v) {
+  asm volatile("global_store_dwordx4 %0, %1, off sc1\n\ts_nop 0" : : "v"(p), "v"(v) : "memory");
+}
+
+// Rows r0 .. r0 + NR - 1 (NR even) of the LDS tile X to tile t by the calling
+// wave, written through; zeros past row and column mc of t (mc = 64: none).
+template <int NR>
+__device__ __forceinline__ void chain_store_rows(const double* X, int pitch, int r0, const CTile& t,
+                                                 int mc = CT) {
+  const int lane = fresh_lane(), rs = r0 + (lane >> 5), c = 2 * (lane & 31);
+  cdbl2 v[NR / 2];
+#pragma unroll
+  for (int q = 0; q < NR / 2; ++q) {
+    const double* x = X + (rs + 2 * q) * pitch + c;
+    v[q].x = x[0];
+    v[q].y = x[1];
+  }
+  if (mc < CT) {
+#pragma unroll
+    for (int q = 0; q < NR / 2; ++q) {
+      if (rs + 2 * q >= mc || c >= mc) v[q].x = 0.0;
+      if (rs + 2 * q >= mc || c + 1 >= mc) v[q].y = 0.0;
+    }
+  }
+  __builtin_amdgcn_sched_barrier(0);  // all reads before the first store
+  double* dst = t.p + (int64_t)rs * t.ld + c;
+  if (t.rows == CT && t.cols == CT) {
+#pragma unroll
+    for (int q = 0; q < NR / 2; ++q) store_through(dst + (int64_t)(2 * q) * t.ld, v[q]);
+  } else {
+#pragma unroll
+    for (int q = 0; q < NR / 2; ++q) {
+      double* d = dst + (int64_t)(2 * q) * t.ld;
+      if (rs + 2 * q >= t.rows) continue;
+      if (c < t.cols) __hip_atomic_store(d, v[q].x, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      if (c + 1 < t.cols) __hip_atomic_store(d + 1, v[q].y, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    }
+  }
+}
+
 // Zero a whole tile (used for the strict-upper tiles of the D blocks).
 __device__ __forceinline__ void tile_zero(const CTile& t) {
   for (int idx = threadIdx.x; idx < CT * CT; idx += CH_THREADS) {
@@ -476,6 +533,49 @@ __device__ __forceinline__ void tile_zero(const CTile& t) {
 }
 
 // ------------------------------------------------------------ helper work
+// Rows r0 .. r0 + 15 of Ps (64 x 64, K-contiguous, pitch LD) <- Ps Linv^T, by the calling
+// wave, in place: column block J takes K < 16 J + 16 (Linv is lower
+// triangular), 40 MFMA steps on four accumulators, each operand of Ps read
+// once.  ACC f64x4: FP64 MFMA; f32x4: FP32 products.
+template <typename ACC, int LD>
+__device__ __forceinline__ void chain_trsm_rows(double* Ps, const double* Linv, int r0) {
+  const int lane = fresh_lane(), li = lane & 15, lk = lane >> 4;
+  ACC c[4];
+#pragma unroll
+  for (int J = 0; J < 4; ++J) c[J] = ACC{0, 0, 0, 0};
+  const double* pa = Ps + (r0 + li) * LD + lk;
+  const double* pb = Linv + li * LD + lk;
+  // operands of 16 k at a time, read while the previous 16 are multiplied
+  double a[2][4], b[2][4][4];
+  auto fetch = [&](int buf, int K) {
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+      a[buf][u] = pa[16 * K + 4 * u];
+#pragma unroll
+      for (int J = 0; J < 4; ++J)
+        if (J >= K) b[buf][u][J] = pb[16 * J * LD + 16 * K + 4 * u];
+    }
+  };
+  fetch(0, 0);
+#pragma unroll
+  for (int K = 0; K < 4; ++K) {
+    if (K < 3) fetch((K + 1) & 1, K + 1);
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int u = 0; u < 4; ++u)
+#pragma unroll
+      for (int J = 0; J < 4; ++J)
+        if (J >= K) c[J] = mfma_acc(a[K & 1][u], b[K & 1][u][J], c[J]);
+    __builtin_amdgcn_sched_barrier(0);
+  }
+  __builtin_amdgcn_wave_barrier();
+#pragma unroll
+  for (int J = 0; J < 4; ++J)
+#pragma unroll
+    for (int r = 0; r < 4; ++r)
+      Ps[(r0 + acc_row(c[J], lane, r)) * LD + 16 * J + acc_col(lane)] = (double)c[J][r];
+}
+
 // acc -= sum over the contribution range (A = factor tile (ra,k) or an arrow
 // tile of column k, B = factor tile (jb,k)); operands prefetched one product ahead.
 // TAG gives each kernel its own copy of the non-inlined workers, so that
@@ -488,9 +588,14 @@ __device__ __forceinline__ void helper_products(const PobtafChain& P, const Cont
   TileRegs16 ra, rb;
   auto tileA = [&](int k) { return cr.ra < 0 ? tile_arrow(P, k, -1 - cr.ra) : tile_g(P, cr.ra, k); };
   __shared__ int s_ready;
-  chain_wait(P, factor_flag(P, cr.ra, cr.k0), factor_flag(P, cr.jb, cr.k0));
-  tile_load16(tileA(cr.k0), ra);
-  tile_load16(tile_g(P, cr.jb, cr.k0), rb);
+  // each operand is loaded as soon as it is there
+  auto wait_load = [&](int k) {
+    chain_wait(P, factor_flag(P, cr.ra, k), nullptr);
+    tile_load16(tileA(k), ra);
+    if (!(cr.ra == cr.jb)) chain_wait(P, factor_flag(P, cr.jb, k), nullptr);
+    tile_load16(tile_g(P, cr.jb, k), rb);
+  };
+  wait_load(cr.k0);
   for (int k = cr.k0;; ++k) {
     const bool more = k + 1 < cr.k1;
     __syncthreads();  // previous product done with XA / XB
@@ -502,9 +607,7 @@ __device__ __forceinline__ void helper_products(const PobtafChain& P, const Cont
     // not held behind the wait for it.
     if (threadIdx.x == 0) {
       int ready = 0;
-      if (more &&
-          __hip_atomic_load(factor_flag(P, cr.ra, k + 1), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) &&
-          __hip_atomic_load(factor_flag(P, cr.jb, k + 1), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) {
+      if (more && chain_ready(factor_flag(P, cr.ra, k + 1)) && chain_ready(factor_flag(P, cr.jb, k + 1))) {
         __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
         ready = 1;
       }
@@ -519,9 +622,7 @@ __device__ __forceinline__ void helper_products(const PobtafChain& P, const Cont
     mfma_abt(XA, XB, acc, sgn, lower_only);
     if (!more) break;
     if (!pre) {
-      chain_wait(P, factor_flag(P, cr.ra, k + 1), factor_flag(P, cr.jb, k + 1));
-      tile_load16(tileA(k + 1), ra);
-      tile_load16(tile_g(P, cr.jb, k + 1), rb);
+      wait_load(k + 1);
     }
   }
   __syncthreads();
@@ -541,158 +642,182 @@ __device__ __forceinline__ void helper_accumulate(const PobtafChain& P, const Co
   }
 }
 
-// out = acc * Linv(j)^T
-template <int TAG>
+// XA <- acc * Linv(j)^T, rows 16w .. 16w + 15 by wave w (complete for that wave).
 __device__ __forceinline__ void helper_solve(const PobtafChain& P, int j, double* XA, double* XB,
-                             f64x4 (&acc)[2][2]) {
+                                             const f64x4 (&acc)[2][2]) {
   chain_wait(P, P.cflags + 2 * j, nullptr);
   TileRegs16 rl;
   tile_load16({P.linv + (int64_t)j * CT * CT, CT, CT, CT}, rl);
   cacc_to_lds(acc, XA, KP);  // A[m][k] = acc(m, k)
   tile_store16(rl, XB);      // B[n][k] = Linv(n, k)
   __syncthreads();
-  cacc_zero(acc);
-  if (P.f32) {
-    f32x4 a32[2][2];
-    cacc32_zero(a32);
-    mfma_abt(XA, XB, a32, 1.0, false);
-    acc32_add(a32, acc, XA, KP);
-  } else {
-    mfma_abt(XA, XB, acc, 1.0, false);
-  }
+  if (P.f32)
+    chain_trsm_rows<f32x4, KP>(XA, XB, 16 * wave_id());
+  else
+    chain_trsm_rows<f64x4, KP>(XA, XB, 16 * wave_id());
+  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
 }
 
 // ------------------------------------------------------------- chain work
-// Columns p .. p + 15 of the factored tile S to memory by the calling wave,
-// zeros above the diagonal.
-__device__ __forceinline__ void chain_store_panel(const double (*S)[TT_LD], int p, const CTile& t) {
-  const int lane = threadIdx.x & 63, c = p + (lane & 7) * 2;
-  cdbl2 v[8];
+// Rows r0 .. r0 + NR - 1 (NR even) of the LDS tile X to tile t by the calling
+// wave; LOWER: zeros above the diagonal (t full).
+template <int NR, bool LOWER>
+__device__ __forceinline__ void chain_store_plain(const double* X, int r0, const CTile& t) {
+  const int lane = fresh_lane(), rs = r0 + (lane >> 5), c = 2 * (lane & 31);
+  cdbl2 v[NR / 2];
 #pragma unroll
-  for (int q = 0; q < 8; ++q) {
-    const int r = (lane >> 3) + 8 * q;
-    v[q].x = c <= r ? S[r][c] : 0.0;
-    v[q].y = c + 1 <= r ? S[r][c + 1] : 0.0;
+  for (int q = 0; q < NR / 2; ++q) {
+    const double* x = X + (rs + 2 * q) * TT_LD + c;
+    v[q].x = x[0];
+    v[q].y = x[1];
   }
-  double* dst = t.p + (int64_t)(lane >> 3) * t.ld + c;
+  if (LOWER) {
 #pragma unroll
-  for (int q = 0; q < 8; ++q) *reinterpret_cast<cdbl2u*>(dst + (int64_t)(8 * q) * t.ld) = v[q];
-}
-
-// Rows r0 .. r0 + 15 of Ps (64 x 64, K-contiguous) <- Ps Linv^T, by the calling
-// wave, in place: column block J takes K < 16 J + 16 (Linv is lower
-// triangular), 40 MFMA steps on four accumulators, each operand of Ps read
-// once.  ACC f64x4: FP64 MFMA; f32x4: FP32 products.
-template <typename ACC>
-__device__ __forceinline__ void chain_trsm_rows(double* Ps, const double (*X2)[TT_LD], int r0) {
-  const int lane = threadIdx.x & 63, li = lane & 15, lk = lane >> 4;
-  ACC c[4];
-#pragma unroll
-  for (int J = 0; J < 4; ++J) c[J] = ACC{0, 0, 0, 0};
-  const double* pa = Ps + (r0 + li) * TT_LD + lk;
-  const double* pb = &X2[li][lk];
-#pragma unroll
-  for (int kk = 0; kk < CT; kk += 4) {
-    const double av = pa[kk];
-#pragma unroll
-    for (int J = kk / 16; J < 4; ++J) c[J] = mfma_acc(av, pb[16 * J * TT_LD + kk], c[J]);
-  }
-  __builtin_amdgcn_wave_barrier();
-#pragma unroll
-  for (int J = 0; J < 4; ++J)
-#pragma unroll
-    for (int r = 0; r < 4; ++r)
-      Ps[(r0 + acc_row(c[J], lane, r)) * TT_LD + 16 * J + acc_col(lane)] = (double)c[J][r];
-}
-
-// The ten lower 16 x 16 blocks of a 64-tile dealt to the four waves (3, 3, 2,
-// 2): block i of the calling wave, i < chain_nblk().
-__device__ __forceinline__ int chain_nblk(int wave) { return wave < 2 ? 3 : 2; }
-__device__ __forceinline__ void chain_blk(int wave, int i, int& rb, int& cb) {
-  rb = wave == 0 ? (i > 0 ? 1 : 0) : (wave == 1 ? 2 : 3);
-  cb = wave == 0 ? (i == 2 ? 1 : 0) : (wave == 3 ? i + 2 : i);
-}
-
-// The calling wave's blocks of the diagonal tile t, in the accumulator layout
-// of ACC; a ragged tile continues with the identity.
-template <typename ACC>
-__device__ __forceinline__ void chain_pd_load(const CTile& t, int wave, f64x4 (&pd)[3]) {
-  const int lane = threadIdx.x & 63;
-  auto each = [&](auto&& value) {
-#pragma unroll
-    for (int i = 0; i < 3; ++i) {
-      if (i >= chain_nblk(wave)) break;
-      int rb, cb;
-      chain_blk(wave, i, rb, cb);
-#pragma unroll
-      for (int r = 0; r < 4; ++r)
-        pd[i][r] = value(16 * rb + acc_row(ACC{}, lane, r), 16 * cb + acc_col(lane));
+    for (int q = 0; q < NR / 2; ++q) {
+      if (c > rs + 2 * q) v[q].x = 0.0;
+      if (c + 1 > rs + 2 * q) v[q].y = 0.0;
     }
-  };
-  if (t.rows == CT)
-    each([&](int row, int col) { return t.p[(int64_t)row * t.ld + col]; });
-  else
-    each([&](int row, int col) {
-      return row < t.rows && col < t.rows ? t.p[(int64_t)row * t.ld + col] : (row == col ? 1.0 : 0.0);
-    });
-}
-
-// The calling wave's blocks of Sn <- pd - Ps Ps^T.
-template <typename ACC>
-__device__ __forceinline__ void chain_syrk(const double* Ps, const f64x4 (&pd)[3], int wave,
-                                           double* Sn) {
-  const int lane = threadIdx.x & 63, li = lane & 15, lk = lane >> 4;
-  const int nblk = chain_nblk(wave);
-  ACC acc[3];
-  const double* pa[3];
-  const double* pb[3];
-#pragma unroll
-  for (int i = 0; i < 3; ++i) {
-    int rb, cb;
-    chain_blk(wave, i, rb, cb);
-    pa[i] = Ps + (16 * rb + li) * TT_LD + lk;
-    pb[i] = Ps + (16 * cb + li) * TT_LD + lk;
-    acc[i] = ACC{0, 0, 0, 0};
-    if constexpr (sizeof(ACC) == sizeof(f64x4)) acc[i] = pd[i];
   }
-  if (nblk == 3) {
+  __builtin_amdgcn_sched_barrier(0);  // all reads before the first store
+  double* dst = t.p + (int64_t)rs * t.ld + c;
+  if (LOWER || (t.rows == CT && t.cols == CT)) {
 #pragma unroll
-    for (int kk = 0; kk < CT; kk += 4)
-#pragma unroll
-      for (int i = 0; i < 3; ++i) acc[i] = mfma_acc(-pa[i][kk], pb[i][kk], acc[i]);
+    for (int q = 0; q < NR / 2; ++q) *reinterpret_cast<cdbl2u*>(dst + (int64_t)(2 * q) * t.ld) = v[q];
   } else {
 #pragma unroll
-    for (int kk = 0; kk < CT; kk += 4)
-#pragma unroll
-      for (int i = 0; i < 2; ++i) acc[i] = mfma_acc(-pa[i][kk], pb[i][kk], acc[i]);
-  }
-#pragma unroll
-  for (int i = 0; i < 3; ++i) {
-    if (i >= nblk) break;
-    int rb, cb;
-    chain_blk(wave, i, rb, cb);
-#pragma unroll
-    for (int r = 0; r < 4; ++r) {
-      double v = (double)acc[i][r];
-      if constexpr (sizeof(ACC) != sizeof(f64x4)) v += pd[i][r];
-      Sn[(16 * rb + acc_row(acc[i], lane, r)) * TT_LD + 16 * cb + acc_col(lane)] = v;
+    for (int q = 0; q < NR / 2; ++q) {
+      double* d = dst + (int64_t)(2 * q) * t.ld;
+      if (rs + 2 * q < t.rows && c < t.cols) d[0] = v[q].x;
+      if (rs + 2 * q < t.rows && c + 1 < t.cols) d[1] = v[q].y;
     }
   }
+}
+
+// N 16 x 16 blocks (I[i], J[i]) of X2 to the Linv tile at p, written through.
+template <int N>
+__device__ __forceinline__ void chain_store_blocks(const double (*X2)[TT_LD], const int (&I)[N],
+                                                   const int (&J)[N], double* p) {
+  const int lane = fresh_lane(), row = lane >> 3, col = 2 * (lane & 7);
+  cdbl2 v[N][2];
+#pragma unroll
+  for (int i = 0; i < N; ++i)
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+      const double* x = &X2[16 * I[i] + 8 * h + row][16 * J[i] + col];
+      v[i][h].x = x[0];
+      v[i][h].y = x[1];
+    }
+  __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+  for (int i = 0; i < N; ++i)
+#pragma unroll
+    for (int h = 0; h < 2; ++h)
+      store_through(p + (16 * I[i] + 8 * h + row) * CT + 16 * J[i] + col, v[i][h]);
+}
+
+// A whole tile in one wave: lane l holds rows 2q + l / 32, columns 2 (l % 32)
+// and the next.  Ragged tiles continue with zeros, or with the identity.
+struct WaveTile {
+  cdbl2 v[32];
+};
+__device__ __forceinline__ void wave_tile_load(const CTile& t, bool ident, WaveTile& x) {
+  const int lane = fresh_lane(), r0 = lane >> 5, c = (lane & 31) * 2;
+  const double* src = t.p + (int64_t)r0 * t.ld + c;
+  if (t.rows == CT && t.cols == CT) {
+#pragma unroll
+    for (int q = 0; q < 32; ++q) x.v[q] = *reinterpret_cast<const cdbl2u*>(src + (int64_t)(2 * q) * t.ld);
+  } else {
+#pragma unroll
+    for (int q = 0; q < 32; ++q) {
+      const int r = 2 * q + r0;
+      const bool in = r < t.rows;
+      x.v[q].x = in && c < t.cols ? src[(int64_t)(2 * q) * t.ld] : (ident && r == c ? 1.0 : 0.0);
+      x.v[q].y = in && c + 1 < t.cols ? src[(int64_t)(2 * q) * t.ld + 1] : (ident && r == c + 1 ? 1.0 : 0.0);
+    }
+  }
+}
+__device__ __forceinline__ void wave_tile_store(const WaveTile& x, double* X) {
+  const int lane = fresh_lane(), r0 = lane >> 5, c = (lane & 31) * 2;
+#pragma unroll
+  for (int q = 0; q < 32; ++q) {
+    X[(2 * q + r0) * TT_LD + c] = x.v[q].x;
+    X[(2 * q + r0) * TT_LD + c + 1] = x.v[q].y;
+  }
+}
+
+// N 16 x 16 blocks of Sn -= Ps Ps^T by the calling wave: rows rb[i], columns cb[i].
+template <typename ACC, int N>
+__device__ __forceinline__ void chain_syrk(const double* Ps, double* Sn, const int (&rb)[N],
+                                           const int (&cb)[N]) {
+  const int lane = fresh_lane(), li = lane & 15, lk = lane >> 4;
+  constexpr bool wide = sizeof(ACC) == sizeof(f64x4);
+  ACC acc[N];
+  double* c[N];
+#pragma unroll
+  for (int i = 0; i < N; ++i) {
+    c[i] = Sn + (16 * rb[i] + acc_row(ACC{}, lane, 0)) * TT_LD + 16 * cb[i] + acc_col(lane);
+    acc[i] = ACC{0, 0, 0, 0};
+    if constexpr (wide) {
+#pragma unroll
+      for (int r = 0; r < 4; ++r) acc[i][r] = c[i][4 * r * TT_LD];
+    }
+  }
+  double a[2][4][N], b[2][4][N];
+  auto fetch = [&](int buf, int K) {
+#pragma unroll
+    for (int u = 0; u < 4; ++u)
+#pragma unroll
+      for (int i = 0; i < N; ++i) {
+        a[buf][u][i] = Ps[(16 * rb[i] + li) * TT_LD + 16 * K + 4 * u + lk];
+        b[buf][u][i] = Ps[(16 * cb[i] + li) * TT_LD + 16 * K + 4 * u + lk];
+      }
+  };
+  fetch(0, 0);
+#pragma unroll
+  for (int K = 0; K < 4; ++K) {
+    if (K < 3) fetch((K + 1) & 1, K + 1);
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int u = 0; u < 4; ++u)
+#pragma unroll
+      for (int i = 0; i < N; ++i) acc[i] = mfma_acc(-a[K & 1][u][i], b[K & 1][u][i], acc[i]);
+    __builtin_amdgcn_sched_barrier(0);
+  }
+#pragma unroll
+  for (int i = 0; i < N; ++i)
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      if constexpr (wide)
+        c[i][4 * r * TT_LD] = acc[i][r];
+      else
+        c[i][r * TT_LD] += (double)acc[i][r];
+    }
 }
 
 // ------------------------------------------------------------- chain step
-// Step g starts with D(g,g) fully updated in S and:
-//   1. factors it (wave 0 factors the 16-column panels; waves 1-3 update the
-//      trailing columns and form block rows 1 and 2 of Linv(g) beside them;
-//      the diagonal blocks of Linv(g) come with the panels);
-//   2. completes Linv(g) (block row 3), stores it and releases it: the helpers
-//      wait for it first;
-//   3. with PX(g) staged in Ps, L(g+1,g) = PX(g) Linv(g)^T, 16 rows per wave;
-//   4. D(g+1,g+1) = PD(g+1) - L(g+1,g) L(g+1,g)^T on its lower 16 x 16
-//      blocks, into the other D buffer.
-// L(g+1,g) is released at the start of step g+1, whose first panel only wave
-// 0 works on.  In the mixed mode the products of steps 3 and 4 round their
-// operands to FP32 and accumulate in FP32; the PD(g+1) term stays FP64.
+// Step g starts with the first 16 columns of D(g,g) updated in S, and:
+//   1. factors it.  Wave 0 factors the 16-column panels.  Beside them waves 1-3
+//      finish the update of the other columns by L(g,g-1) and apply the panels
+//      to them; wave 3 forms block rows 1 and 2 of Linv(g) (its diagonal
+//      blocks come with the panels) and the products of row 3; waves 1 and 2
+//      store L(g-1,g-1) and, during the last panel, look whether PX(g) and
+//      PD(g+1) are published and load them if so;
+//   2. wave 3 completes Linv(g) while waves 1 and 2 wait for PX(g) and PD(g+1)
+//      if need be and put them in Ps and the other D buffer;
+//   3. L(g+1,g) = PX(g) Linv(g)^T, 16 rows per wave; Linv(g) is flagged after
+//      it, or before it if PX(g) was late: its stores have landed by then;
+//   4. the first 16 columns of D(g+1,g+1) = PD(g+1) - L(g+1,g) L(g+1,g)^T;
+//      L(g+1,g), stored meanwhile, is released beside the next first panel.
+// On the path are the four panels (8 us), 12 MFMA steps of the block row, 40 of
+// the solve, 16 of the update, and four barriers.  Stores and flag reads stay
+// off it: a wave that waits for either holds the next barrier up, so wave 0
+// has none, and no store precedes a look in the same phase.  In the mixed mode
+// the products of steps 3 and 4 round their operands to FP32 and accumulate in
+// FP32; the PD(g+1) term stays FP64.
+// Measured, median step at b = 64 / 256 / 1024: 12.1 / 12.7 / 13.9 us; with
+// whole update and release between the steps 14.2 / 14.2 / 15.1 us.  From b = 256
+// on PX(g) arrives about when the panels end: the helpers' path from Linv(g)
+// over L(g+2,g) to PX(g+1) is as long as the chain's.
 // A ragged tile (the last of a block when b % 64 != 0) runs padded with the
 // identity to 64: PX comes with zeros past its rows and columns, so the
 // padding stays what it is through steps 3 and 4, and only the 16-column
@@ -705,15 +830,16 @@ __device__ __forceinline__ void chain_syrk(const double* Ps, const f64x4 (&pd)[3
 // [64][65] (Linv(g)), Ps [64][65] (PX(g) -> L(g+1,g), row-major =
 // K-contiguous).
 //
-// chain_factor_ragged: L(g,g) of m < 64 columns in S, Linv(g) in X2 (the
-// identity past m), L(g,g) to memory; wave 3 looks at the flags of PX(g) and
-// PD(g+1) meanwhile.  Returns with every wave past the last write of X2.
-template <int TAG>
-__device__ __forceinline__ void chain_factor_ragged(const PobtafChain& P, double (*S2)[TT_LD],
-                                                    double (*X2)[TT_LD], int m, int64_t row0,
-                                                    const CTile& dt, bool sub, const int* f_px,
-                                                    const int* f_pd, int* s_early) {
-  const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+// chain_factor_ragged: L(g,g) of m < 64 columns in S and in memory, Linv(g) in
+// X2 (the identity past m).  start() and rest() run on waves 1-3 and
+// store_prev() on waves 1 and 2 beside the first panel, look() there beside the
+// last.  Ends with a barrier.
+template <typename START, typename REST, typename PREV, typename LOOK>
+__device__ __forceinline__ void chain_factor_ragged(double (*S2)[TT_LD], double (*X2)[TT_LD], int m,
+                                                    int* info, int64_t row0, const CTile& dt,
+                                                    const START& start, const REST& rest,
+                                                    const PREV& store_prev, const LOOK& look) {
+  const int tid = threadIdx.x, wave = wave_id();
   const int pe = (m + PW - 1) / PW * PW;  // columns factored
   for (int idx = pe * CT + tid; idx < CT * CT; idx += CH_THREADS)
     X2[idx / CT][idx % CT] = idx / CT == idx % CT ? 1.0 : 0.0;
@@ -722,7 +848,14 @@ __device__ __forceinline__ void chain_factor_ragged(const PobtafChain& P, double
     if (wave == 0) {
       WavePanel16<true> w;
       w.factor(S2, p, TT);
-      w.finish(S2, p, &X2[p][p], TT_LD, P.info, row0);
+      w.finish(S2, p, &X2[p][p], TT_LD, info, row0);
+    } else {
+      if (p == 0) {
+        start();
+        rest();
+        if (wave < 3) store_prev();
+      }
+      if (p + PW >= pe && wave < 3) look(3);
     }
     __syncthreads();
     if (p + PW < pe) {
@@ -735,29 +868,18 @@ __device__ __forceinline__ void chain_factor_ragged(const PobtafChain& P, double
     if (wave < I) wave_trtri_offdiag(S2, X2, &X2[PW * I][PW * I], TT_LD, I, wave);
     __syncthreads();
   }
-  if (wave == 3) {
-    int ok = sub ? (__hip_atomic_load(f_px, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) &
-                    __hip_atomic_load(f_pd, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT))
-                 : 0;
-    ok = __builtin_amdgcn_readfirstlane(ok);
-    if (ok) __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
-    if ((tid & 63) == 0) *s_early = ok;
-  }
   for (int idx = tid; idx < m * CT; idx += CH_THREADS) {
     const int r = idx / CT, c = idx % CT;
     if (c < m) dt.p[(int64_t)r * dt.ld + c] = c <= r ? S2[r][c] : 0.0;
   }
-  __syncthreads();
 }
 
 template <int TAG>
-__device__ __forceinline__ void chain_run(const PobtafChain& P, double* Sa, double* Sb,
-                                                double* Xs, double* Ps) {
+__device__ __forceinline__ void chain_run(const PobtafChain& P, double* Sa, double* Sb, double* Xs,
+                                          double* Ps) {
   const int tid = threadIdx.x;
   double (*X2)[TT_LD] = reinterpret_cast<double (*)[TT_LD]>(Xs);
-  const int lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int rs = tid >> 5, c2 = (tid & 31) * 2;
-  constexpr int PUB = 64;  // wave 1, lane 0: runs the releases
+  const int lane = tid & 63, wave = wave_id();
   for (int idx = tid; idx < CT * TT_LD; idx += CH_THREADS) Xs[idx] = 0.0;
   {
     f64x4 acc[2][2];
@@ -768,142 +890,139 @@ __device__ __forceinline__ void chain_run(const PobtafChain& P, double* Sa, doub
     if (tid >= m0 && tid < CT) Sa[tid * TT_LD + tid] = 1.0;
   }
   __syncthreads();
-  __shared__ int s_early;
-  int pending = -1;  // step whose L(g+1,g) stores wait for their release
+  __shared__ int s_have[2];
+  bool pending = false;  // L(g,g-1) is in Ps: update, store and flag open
   double* S = Sa;
   double* Sn = Sb;
   for (int g = 0; g < P.NT; ++g) {
     double (*S2)[TT_LD] = reinterpret_cast<double (*)[TT_LD]>(S);
     const CTile dt = tile_g(P, g, g);
-    const bool sub = g + 1 < band_end(P, g);
-    const int* f_px = P.hflags + t_px(P, g);
-    const int* f_pd = sub ? P.hflags + t_pd(P, g + 1) : f_px;
-    if (pending >= 0 && tid == PUB) {
-      // every wave waited for its L(g,g-1) stores before the barrier that
-      // ended the previous step
-      __builtin_amdgcn_fence(__ATOMIC_RELEASE, "agent");
-      wave_stores_done();
-      __hip_atomic_store(P.cflags + 2 * pending + 1, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    }
-    pending = -1;
-    chain_trace(P, g, 0);
-    // 1. factorization with Linv block rows 1 and 2 and the stores of
-    //    finished panels beside it; PX(g) and PD(g+1) flags checked by wave 1
-    //    during the last panel
-    const int64_t row0 = (int64_t)(g / P.nt) * P.b + (int64_t)(g % P.nt) * CT;
     const int m = dt.rows;
-    if (m == CT) lds_potrf_t<CT>(S2, X2, CT, P.info, row0, [&](int p) {
-      if (p < 32) {
-        if (wave == 3) chain_store_panel(S2, p, dt);
-        if (p == 16 && wave == 2) wave_trtri_offdiag(S2, X2, &X2[16][16], TT_LD, 1, 0);
-      } else if (wave == 1) {
-        chain_store_panel(S2, 32, dt);
-        // a few looks: a flag set while the panel runs saves the wait after it
-        int ok = 0;
-        for (int look = 0; sub && !ok && look < 3; ++look)
-          ok = __builtin_amdgcn_readfirstlane(
-              __hip_atomic_load(f_px, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) &
-              __hip_atomic_load(f_pd, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT));
-        if (ok) __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
-        if (lane == 0) s_early = ok;
-      } else {
-        wave_trtri_offdiag(S2, X2, &X2[32][32], TT_LD, 2, wave == 2 ? 1 : 0);
-      }
-    });
-    else
-      chain_factor_ragged<TAG>(P, S2, X2, m, row0, dt, sub, f_px, f_pd, &s_early);
-    const int early = s_early;
-    chain_trace(P, g, 1);
-    // PX(g) and PD(g+1), if both were published during the factorization: the
-    // loads land during step 2
-    const CTile xt = tile_g(P, g + 1, g);
-    TileRegs16 rx;
-    f64x4 pd[3];
-    auto load_px = [&]() {
-      tile_load16(xt, rx);
+    const bool sub = g + 1 < band_end(P, g);
+    int* const f_linv = P.cflags + 2 * g;
+    double* const linv = P.linv + (int64_t)g * CT * CT;
+    chain_trace(P, g, 0);
+    // 1. factorization
+    WaveTile wt;        // waves 1, 2: PX(g), PD(g+1)
+    bool have = false;
+    const int* const f_tile = !sub ? nullptr : P.hflags + (wave == 1 ? t_px(P, g) : t_pd(P, g + 1));
+    auto load_tile = [&]() { wave_tile_load(tile_g(P, g + 1, g + (wave - 1)), wave == 2, wt); };
+    auto syrk = [&](double* X, int rb, int cb) {
+      const int r[1] = {rb}, c[1] = {cb};
       if (P.f32)
-        chain_pd_load<f32x4>(tile_g(P, g + 1, g + 1), wave, pd);
+        chain_syrk<f32x4, 1>(Ps, X, r, c);
       else
-        chain_pd_load<f64x4>(tile_g(P, g + 1, g + 1), wave, pd);
+        chain_syrk<f64x4, 1>(Ps, X, r, c);
     };
-    auto stage_px = [&]() {  // pitch 65: 8-byte stores
-#pragma unroll
-      for (int q = 0; q < 8; ++q) {
-        Ps[(rs + 8 * q) * TT_LD + c2] = rx.v[q].x;
-        Ps[(rs + 8 * q) * TT_LD + c2 + 1] = rx.v[q].y;
+    auto start = [&]() {
+      if (!pending) return;
+      if (wave == 3) {  // every wave has waited for its rows of L(g,g-1)
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "agent");
+        chain_wave_done(P.cflags + 2 * g - 1, CH_READY);
       }
+      syrk(S, wave, 1);
     };
-    if (early) load_px();
-    // 2. Linv block row 3; the last panel of L(g,g) and Linv(g) to memory
+    // blocks (2,2), (3,2), (3,3): after the update of the same blocks by panel 0,
+    // which the same waves have
+    auto rest = [&]() {
+      if (pending) syrk(S, wave == 1 ? 2 : 3, wave == 3 ? 3 : 2);
+    };
+    // waves 1, 2: L(g-1,g-1), still in the other D buffer
+    auto store_prev = [&]() {
+      if (!pending) return;
+      const CTile pt = tile_g(P, g - 1, g - 1);
+      if (pt.rows == CT) chain_store_plain<32, true>(Sn, 32 * (wave - 1), pt);
+    };
+    WaveTrtriRow<3> row3;  // wave 3
+    auto look = [&](int looks) {
+      // a few looks: a flag set while the panel runs saves the wait after it
+      const bool had = have;
+      for (int k = 0; sub && !have && k < looks; ++k)
+        have = __builtin_amdgcn_readfirstlane((int)chain_ready(f_tile)) != 0;
+      if (have && !had) {
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
+        load_tile();
+      }
+      if (lane == 0) s_have[wave - 1] = have;
+    };
+    const int64_t row0 = (int64_t)(g / P.nt) * P.b + (int64_t)(g % P.nt) * CT;
     if (m == CT) {
-      if (wave >= 1)
-        wave_trtri_offdiag(S2, X2, &X2[48][48], TT_LD, 3, wave - 1);
-      else
-        chain_store_panel(S2, 48, dt);
-      __syncthreads();
-    }
-    double* li_out = P.linv + (int64_t)g * CT * CT;
-    {
-      cdbl2 v[8];
-#pragma unroll
-      for (int q = 0; q < 8; ++q) {
-        v[q].x = X2[rs + 8 * q][c2];
-        v[q].y = X2[rs + 8 * q][c2 + 1];
-      }
-      if (m < CT) {  // zeros past a ragged tile's rows and columns
-#pragma unroll
-        for (int q = 0; q < 8; ++q) {
-          if (rs + 8 * q >= m || c2 >= m) v[q].x = 0.0;
-          if (rs + 8 * q >= m || c2 + 1 >= m) v[q].y = 0.0;
+      lds_potrf_t<CT>(S2, X2, CT, P.info, row0, [&](int p) {
+        if (p < 0) {
+          start();
+        } else if (p == 0) {
+          rest();
+        } else if (p == 16) {
+          if (wave < 3) {
+            store_prev();
+          } else {
+            WaveTrtriRow<1> row1;
+            row1.products(S2, X2);
+            row1.finish(X2);
+            const int I[3] = {0, 1, 1}, J[3] = {0, 0, 1};
+            chain_store_blocks<3>(X2, I, J, linv);
+          }
+        } else {
+          if (wave < 3) {
+            look(3);
+          } else {
+            WaveTrtriRow<2> row2;
+            row2.products(S2, X2);
+            row2.finish(X2);
+            row3.products(S2, X2);
+            const int I[3] = {2, 2, 2}, J[3] = {0, 1, 2};
+            chain_store_blocks<3>(X2, I, J, linv);
+          }
         }
-      }
-#pragma unroll
-      for (int q = 0; q < 8; ++q) *reinterpret_cast<cdbl2*>(li_out + (rs + 8 * q) * CT + c2) = v[q];
+      });
+    } else {
+      chain_factor_ragged(S2, X2, m, P.info, row0, dt, start, rest, store_prev, look);
     }
+    pending = sub;
+    chain_trace(P, g, 1);
+    // 2. Linv(g) complete, PX(g) in Ps, PD(g+1) in Sn
+    if (m < CT) {
+      chain_store_rows<16>(Xs, TT_LD, 16 * wave, {linv, CT, CT, CT}, m);
+    } else if (wave == 3) {
+      row3.finish(X2);
+      const int I[4] = {3, 3, 3, 3}, J[4] = {0, 1, 2, 3};
+      chain_store_blocks<4>(X2, I, J, linv);
+    }
+    // Linv(g) is stored by wave 3, a ragged tile's by all waves
+    const bool fetch = wave == 1 || wave == 2, stores = m < CT || wave == 3;
+    const int share = m < CT ? CH_READY / 4 : CH_READY;
+    const bool wait = !sub || fetch || !(s_have[0] && s_have[1]);
+    if (stores && wait) chain_wave_done(f_linv, share);
     if (!sub) {  // last diagonal tile of the matrix
-      chain_publish(P.cflags + 2 * g);
+      if (m == CT && wave < 2) chain_store_plain<32, true>(S, 32 * wave, dt);
       continue;
     }
-    if (early) stage_px();
-    wave_stores_done();
+    if (fetch) {
+      if (!have) {
+        wave_wait(P, f_tile, nullptr);
+        load_tile();
+      }
+      wave_tile_store(wt, wave == 1 ? Ps : Sn);
+    }
     __syncthreads();
-    if (tid == PUB) {
-      __builtin_amdgcn_fence(__ATOMIC_RELEASE, "agent");
-      wave_stores_done();
-      __hip_atomic_store(P.cflags + 2 * g, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    }
-    if (!early) {
-      wave_wait(P, f_px, f_pd);
-      load_px();
-      stage_px();
-      __syncthreads();
-    }
     chain_trace(P, g, 2);
     // 3. L(g+1,g), wave w: rows 16w .. 16w + 15
     if (P.f32)
-      chain_trsm_rows<f32x4>(Ps, X2, 16 * wave);
+      chain_trsm_rows<f32x4, TT_LD>(Ps, Xs, 16 * wave);
     else
-      chain_trsm_rows<f64x4>(Ps, X2, 16 * wave);
+      chain_trsm_rows<f64x4, TT_LD>(Ps, Xs, 16 * wave);
+    if (stores && !wait) chain_wave_done(f_linv, share);
+    chain_store_plain<16, false>(Ps, 16 * wave, tile_g(P, g + 1, g));
     __syncthreads();  // L(g+1,g) complete in Ps
     chain_trace(P, g, 3);
-    lds_tile_store(Ps, TT_LD, xt);
-    pending = g;
-    // 4. D(g+1,g+1) into Sn
-    if (P.f32)
-      chain_syrk<f32x4>(Ps, pd, wave, Sn);
-    else
-      chain_syrk<f64x4>(Ps, pd, wave, Sn);
+    // 4. the first 16 columns of D(g+1,g+1)
+    syrk(Sn, wave, 0);
     wave_stores_done();  // L(g+1,g): released at the start of step g+1
     __syncthreads();
     chain_trace(P, g, 5);
     double* t = S;
     S = Sn;
     Sn = t;
-  }
-  if (pending >= 0 && tid == PUB) {
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "agent");
-    wave_stores_done();
-    __hip_atomic_store(P.cflags + 2 * pending + 1, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
   }
 }
 
@@ -996,12 +1115,15 @@ __device__ __forceinline__ void chain_helper_task(const PobtafChain& P, int task
   cacc_load(out, acc);
   const ContribRange cr = chain_contribs(P, kind, r, j);
   helper_accumulate<TAG>(P, cr, -1.0, kind == HK_PD, XA, XB, acc);
-  if (kind == HK_TRSM || kind == HK_ARR) helper_solve<TAG>(P, j, XA, XB, acc);
-  __syncthreads();  // the last product is done with XA
-  cacc_to_lds(acc, XA, KP);
-  __syncthreads();
-  lds_tile_store(XA, KP, out);
-  chain_publish(P.hflags + task);
+  if (kind == HK_TRSM || kind == HK_ARR) {
+    helper_solve(P, j, XA, XB, acc);
+  } else {
+    __syncthreads();  // the last product is done with XA
+    cacc_to_lds(acc, XA, KP);
+    __syncthreads();
+  }
+  chain_store_rows<16>(XA, KP, 16 * wave_id(), out);
+  chain_wave_done(P.hflags + task, CH_READY / 4);
   if (kind == HK_PX) chain_trace(P, j, 6);
   if (kind == HK_TRSM && r == j + 2) chain_trace(P, j, 7);
   // The strict-upper mirror of a lower D-block tile is zero in the factor.

@@ -40,6 +40,19 @@ struct TileBatch {
   int grid_begin;   // list launches: first workgroup of this entry
 };
 
+// Wave of the calling lane as a scalar: branches on it are scalar branches, and
+// what one wave keeps in registers does not count in another wave's branch.
+__device__ __forceinline__ int wave_id() { return __builtin_amdgcn_readfirstlane(threadIdx.x >> 6); }
+
+// Lane index as a new value at each call: addresses formed from it are computed
+// where they are used.  In a long loop the compiler otherwise forms all of
+// them once before it and runs out of registers.
+__device__ __forceinline__ int fresh_lane() {
+  int l = threadIdx.x & 63;
+  asm volatile("" : "+v"(l));
+  return l;
+}
+
 __device__ __forceinline__ double readlane_f64(double v, int lane) {
   const uint64_t u = __builtin_bit_cast(uint64_t, v);
   const uint32_t lo = __builtin_amdgcn_readlane((uint32_t)u, lane);
@@ -235,7 +248,7 @@ template <bool INV>
 struct WavePanel16 {
   double d[PW], r[PW], pv;
   __device__ __forceinline__ void factor(double (*S)[TT_LD], int p, int m) {
-    const int lane = threadIdx.x & 63, li = lane & 15;
+    const int lane = fresh_lane(), li = lane & 15;
     const int row = p + lane;
     const double* sd = &S[p + li][p];
     const double* sr = &S[row < m ? row : p + li][p];
@@ -253,7 +266,7 @@ struct WavePanel16 {
   }
   __device__ __forceinline__ void finish(double (*S)[TT_LD], int p, double* Xp, int ldx, int* info,
                                          int64_t row0) {
-    const int lane = threadIdx.x & 63;
+    const int lane = fresh_lane();
     if (lane < 16) {
       if (INV) {
 #pragma unroll
@@ -309,7 +322,7 @@ __device__ __forceinline__ void lds_syrk_update(double (*S)[TT_LD], int p, int w
 // diagonal).
 __device__ __forceinline__ void lds_syrk_cols(double (*S)[TT_LD], int p, int c0, int c1,
                                               int wave0, int nw) {
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int lane = fresh_lane(), wave = wave_id();
   const int li = lane & 15, lk = lane >> 4;
   int t = 0;
   for (int cb = c0 / 16; cb < c1 / 16; ++cb)
@@ -344,17 +357,21 @@ struct NoIdle {
 // next panel is factored (wave 0), while waves 1-3 apply panel p to the
 // columns beyond it.  Full tiles also leave the inverses of the four diagonal
 // blocks in X's (each written with its panel), and after the update beside a
-// panel, waves 1-3 run idle(p) while wave 0 factors panel p + 16; panels 0 ..
-// p and their blocks' inverses are final by then.  The call ends with a barrier
+// panel, waves 1-3 run idle(p) while wave 0 factors panel p + 16, from p = -16
+// on; panels 0 .. p and their blocks' inverses are final by then.  Columns 16
+// .. 63 of S may be completed by idle(-16).  The call ends with a barrier
 // after the last of them.  MFIX = 0 handles any m <= 64 and leaves X alone.
 template <int MFIX, typename IDLE = NoIdle>
 __device__ __forceinline__ void lds_potrf_t(double (*S)[TT_LD], double (*X)[TT_LD], int m_rt,
                                             int* info, int64_t row0, IDLE idle = IDLE()) {
   const int m = MFIX ? MFIX : m_rt;
-  const int wave = threadIdx.x >> 6;
+  const int wave = wave_id();
   if (MFIX == TT) {
     WavePanel16<true> w;
-    if (wave == 0) w.factor(S, 0, TT);
+    if (wave == 0)
+      w.factor(S, 0, TT);
+    else
+      idle(-PW);
     __syncthreads();
 #pragma unroll
     for (int p = 0; p + PW < TT; p += PW) {
@@ -459,7 +476,7 @@ __device__ __forceinline__ void wave_diag_inv16(const double (*S)[TT_LD], double
 // of k-step r of the second, so W never leaves the registers.
 __device__ __forceinline__ void wave_trtri_offdiag(const double (*S)[TT_LD], double (*Xs)[TT_LD],
                                                    const double* XI, int ldi, int I, int J) {
-  const int lane = threadIdx.x & 63, li = lane & 15, lk = lane >> 4;
+  const int lane = fresh_lane(), li = lane & 15, lk = lane >> 4;
   f64x4 w = {0.0, 0.0, 0.0, 0.0};
   for (int K = J; K < I; ++K)
 #pragma unroll
@@ -473,6 +490,55 @@ __device__ __forceinline__ void wave_trtri_offdiag(const double (*S)[TT_LD], dou
 #pragma unroll
   for (int r = 0; r < 4; ++r) Xs[I * 16 + acc_row_f64(lane, r)][J * 16 + acc_col(lane)] = -x[r];
 }
+
+// Blocks 0 .. I - 1 of block row I of X = L^{-1} by the calling wave, as
+// wave_trtri_offdiag with X_II in Xs, in two parts: the products W_J = sum_K
+// L_IK X_KJ need block row I of L up to column I - 1 only, so they can run
+// while block (I, I) is factored.  All operands are read before the first MFMA
+// and the chains of dependent MFMAs run interleaved.
+template <int I>
+struct WaveTrtriRow {
+  f64x4 w[I];
+  __device__ __forceinline__ void products(const double (*S)[TT_LD], const double (*Xs)[TT_LD]) {
+    const int lane = fresh_lane(), li = lane & 15, lk = lane >> 4;
+    double a[I][4], b[I][I][4];
+#pragma unroll
+    for (int k = 0; k < I; ++k)
+#pragma unroll
+      for (int u = 0; u < 4; ++u) {
+        a[k][u] = S[I * 16 + li][k * 16 + 4 * u + lk];
+#pragma unroll
+        for (int j = 0; j <= k; ++j) b[j][k][u] = Xs[k * 16 + 4 * u + lk][j * 16 + li];
+      }
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int j = 0; j < I; ++j) w[j] = f64x4{0.0, 0.0, 0.0, 0.0};
+#pragma unroll
+    for (int k = 0; k < I; ++k)
+#pragma unroll
+      for (int u = 0; u < 4; ++u)
+#pragma unroll
+        for (int j = 0; j <= k; ++j) w[j] = mfma_f64(a[k][u], b[j][k][u], w[j]);
+  }
+  __device__ __forceinline__ void finish(double (*Xs)[TT_LD]) const {
+    const int lane = fresh_lane(), li = lane & 15, lk = lane >> 4;
+    double xi[4];
+#pragma unroll
+    for (int r = 0; r < 4; ++r) xi[r] = Xs[16 * I + li][16 * I + 4 * r + lk];
+    f64x4 x[I];
+#pragma unroll
+    for (int j = 0; j < I; ++j) x[j] = f64x4{0.0, 0.0, 0.0, 0.0};
+#pragma unroll
+    for (int r = 0; r < 4; ++r)
+#pragma unroll
+      for (int j = 0; j < I; ++j) x[j] = mfma_f64(xi[r], w[j][r], x[j]);
+#pragma unroll
+    for (int j = 0; j < I; ++j)
+#pragma unroll
+      for (int r = 0; r < 4; ++r)
+        Xs[I * 16 + acc_row_f64(lane, r)][j * 16 + acc_col(lane)] = -x[j][r];
+  }
+};
 
 // ZERO = false: the caller guarantees that the blocks of Xs strictly above
 // the 16x16 block diagonal already hold zeros (they are never written here).
