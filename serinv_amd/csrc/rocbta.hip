@@ -884,8 +884,16 @@ BsLayout bs_layout(int64_t n, int64_t b, int64_t a, int64_t r) {
 template <int CW>
 int launch_block_sweep(BlockSweepP P, hipStream_t s) {
   const int rw = bs_rw(CW, P.trans);
-  P.G = (int)std::min<int64_t>(std::min<int64_t>((P.b + rw - 1) / rw, BS_MAX_G), device_cus());
-  if (P.trans == 0)
+  const int ngroups = (P.b + rw - 1) / rw;
+  P.G = std::min(std::min(ngroups, BS_MAX_G), device_cus());
+  // a workgroup per row group and the rows of a phase in registers: the form
+  // that loads a phase ahead
+  const bool reg = P.G == ngroups && P.b <= BS_KU * BS_THREADS;
+  if (reg && P.trans == 0)
+    pobtas_block_reg_kernel<CW, 0><<<P.G, BS_THREADS, 0, s>>>(P);
+  else if (reg)
+    pobtas_block_reg_kernel<CW, 1><<<P.G, BS_THREADS, 0, s>>>(P);
+  else if (P.trans == 0)
     pobtas_block_kernel<CW, 0><<<P.G, BS_THREADS, 0, s>>>(P);
   else
     pobtas_block_kernel<CW, 1><<<P.G, BS_THREADS, 0, s>>>(P);

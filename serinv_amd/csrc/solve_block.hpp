@@ -253,6 +253,85 @@ __device__ __forceinline__ void bs_emit(const BlockSweepP& P, double* buf, int i
   }
 }
 
+// Workgroup 0: y_t = Tinv (b_t - sum_w part_w)   (partial: b_t - sum only)
+template <int CW>
+__device__ __forceinline__ void bs_tip_solve(const BlockSweepP& P, double* tip) {
+  const int tid = threadIdx.x, n = P.n, b = P.b, a = P.a;
+  for (int idx = tid; idx < a * CW; idx += BS_THREADS) {
+    const int m = idx / CW, c = idx % CW;
+    double s = 0.0;
+    // sixteen workgroups' sums a round trip, added in workgroup order
+    for (int w0 = 0; w0 < P.G; w0 += 16) {
+      double part[16];
+      long long spins = 0;
+      for (bool empty = true; empty;) {
+        empty = false;
+#pragma unroll
+        for (int u = 0; u < 16; ++u) {
+          const unsigned long long v =
+              w0 + u < P.G ? sw_ld(P.tpart + (int64_t)(w0 + u) * a * CW + idx) : 0ull;
+          part[u] = __longlong_as_double((long long)v);
+          empty |= v == SW_EMPTY;
+        }
+        if (empty && !bs_spin(P, spins)) {
+#pragma unroll
+          for (int u = 0; u < 16; ++u) part[u] = 0.0;
+          break;
+        }
+      }
+#pragma unroll
+      for (int u = 0; u < 16; ++u) s += part[u];
+    }
+    const double bv = (c < P.r) ? P.B[((int64_t)n * b + m) * P.ldb + c] : 0.0;
+    tip[idx] = bv - s;
+  }
+  __syncthreads();
+  for (int idx = tid; idx < a * CW; idx += BS_THREADS) {
+    const int m = idx / CW, c = idx % CW;
+    double v = tip[idx];
+    if (!P.partial) {
+      v = 0.0;
+      for (int mm = 0; mm <= m; ++mm) v = fma(P.Tinv[(int64_t)m * a + mm], tip[mm * CW + c], v);
+    }
+    if (c < P.r) P.B[((int64_t)n * b + m) * P.ldb + c] = v;
+  }
+}
+
+// x_t: solved by workgroup 0 and published (or the given B rows if
+// partial); every workgroup keeps it in LDS
+template <int CW>
+__device__ __forceinline__ void bs_tip_back(const BlockSweepP& P, double* xt) {
+  const int tid = threadIdx.x, n = P.n, b = P.b, a = P.a;
+  if (a > 0) {
+    if (!P.partial) {
+      if (blockIdx.x == 0) {
+        for (int idx = tid; idx < a * CW; idx += BS_THREADS) {
+          const int m = idx / CW, c = idx % CW;
+          double v = 0.0;
+          for (int mm = m; mm < a; ++mm)
+            v = fma(P.Tinv[(int64_t)mm * a + m],
+                    (c < P.r) ? P.B[((int64_t)n * b + mm) * P.ldb + c] : 0.0, v);
+          xt[idx] = v;
+        }
+        __syncthreads();  // every read of the tip rows of B precedes the writes
+        for (int idx = tid; idx < a * CW; idx += BS_THREADS) {
+          const int m = idx / CW, c = idx % CW;
+          if (c < P.r) P.B[((int64_t)n * b + m) * P.ldb + c] = xt[idx];
+          sw_st(P.tipbuf + idx, xt[idx]);
+        }
+      } else {
+        for (int idx = tid; idx < a * CW; idx += BS_THREADS) xt[idx] = bs_take(P, P.tipbuf + idx);
+      }
+    } else {
+      for (int idx = tid; idx < a * CW; idx += BS_THREADS) {
+        const int m = idx / CW, c = idx % CW;
+        xt[idx] = (c < P.r) ? P.B[((int64_t)n * b + m) * P.ldb + c] : 0.0;
+      }
+    }
+    __syncthreads();
+  }
+}
+
 template <int CW, int TRANS>
 __global__ void __launch_bounds__(BS_THREADS) pobtas_block_kernel(BlockSweepP P) {
   constexpr int RW = bs_rw(CW, TRANS);
@@ -329,58 +408,11 @@ __global__ void __launch_bounds__(BS_THREADS) pobtas_block_kernel(BlockSweepP P)
       if (idx < a * CW) sw_st(P.tpart + (int64_t)blockIdx.x * a * CW + idx, tacc[u]);
     }
     if (blockIdx.x != 0) return;
-    // workgroup 0: y_t = Tinv (b_t - sum_w part_w)   (partial: b_t - sum only)
-    double* tip = S.xt;
-    for (int idx = tid; idx < a * CW; idx += BS_THREADS) {
-      const int m = idx / CW, c = idx % CW;
-      double s = 0.0;
-      for (int w = 0; w < P.G; ++w) s += bs_take(P, P.tpart + (int64_t)w * a * CW + idx);
-      const double bv = (c < P.r) ? P.B[((int64_t)n * b + m) * P.ldb + c] : 0.0;
-      tip[idx] = bv - s;
-    }
-    __syncthreads();
-    for (int idx = tid; idx < a * CW; idx += BS_THREADS) {
-      const int m = idx / CW, c = idx % CW;
-      double v = tip[idx];
-      if (!P.partial) {
-        v = 0.0;
-        for (int mm = 0; mm <= m; ++mm) v = fma(P.Tinv[(int64_t)m * a + mm], tip[mm * CW + c], v);
-      }
-      if (c < P.r) P.B[((int64_t)n * b + m) * P.ldb + c] = v;
-    }
+    bs_tip_solve<CW>(P, S.xt);
     return;
   }
   // -------------------------------------------------------------- backward
-  // x_t: solved by workgroup 0 and published (or the given B rows if
-  // partial); every workgroup keeps it in LDS
-  if (a > 0) {
-    if (!P.partial) {
-      if (blockIdx.x == 0) {
-        for (int idx = tid; idx < a * CW; idx += BS_THREADS) {
-          const int m = idx / CW, c = idx % CW;
-          double v = 0.0;
-          for (int mm = m; mm < a; ++mm)
-            v = fma(P.Tinv[(int64_t)mm * a + m],
-                    (c < P.r) ? P.B[((int64_t)n * b + mm) * P.ldb + c] : 0.0, v);
-          S.xt[idx] = v;
-        }
-        __syncthreads();  // every read of the tip rows of B precedes the writes
-        for (int idx = tid; idx < a * CW; idx += BS_THREADS) {
-          const int m = idx / CW, c = idx % CW;
-          if (c < P.r) P.B[((int64_t)n * b + m) * P.ldb + c] = S.xt[idx];
-          sw_st(P.tipbuf + idx, S.xt[idx]);
-        }
-      } else {
-        for (int idx = tid; idx < a * CW; idx += BS_THREADS) S.xt[idx] = bs_take(P, P.tipbuf + idx);
-      }
-    } else {
-      for (int idx = tid; idx < a * CW; idx += BS_THREADS) {
-        const int m = idx / CW, c = idx % CW;
-        S.xt[idx] = (c < P.r) ? P.B[((int64_t)n * b + m) * P.ldb + c] : 0.0;
-      }
-    }
-    __syncthreads();
-  }
+  bs_tip_back<CW>(P, S.xt);
   for (int i = n - 1; i >= 0; --i) {
     const bool skip = P.partial && i == n - 1;  // x_{n-1} is the given B block
     for (int g = blockIdx.x; g < ngroups; g += P.G) {
@@ -442,6 +474,239 @@ __global__ void __launch_bounds__(BS_THREADS) pobtas_block_kernel(BlockSweepP P)
       bs_emit<CW, RW>(P, P.sbuf, i, k0, S.out, true);
       __syncthreads();
     }
+  }
+}
+
+// ------------------------------------------------ one row group per workgroup
+// The sweep for b <= BS_KU * BS_THREADS where every row group has a workgroup of
+// its own: the rows of a phase's matrix fit in registers and are loaded one
+// phase ahead, behind the polls of the phase before (loads complete in order,
+// so a load issued before a poll would delay it), together with the right-hand
+// side and the arrow entries of the rows.  A phase then costs the round trip
+// of the published values, the products and the reduction, which adds the
+// waves' lanes by half-exchanges and row rotations and needs one barrier.
+// Every poll round asks for all values of a thread at once.
+// Bound by that round trip (about 1.5 us).  Measured, N + C: BSR_FIGS
+template <int N>
+__device__ __forceinline__ double row_ror_add(double x) {
+  const unsigned long long u = (unsigned long long)__double_as_longlong(x);
+  const int lo = __builtin_amdgcn_update_dpp(0, (int)(unsigned)u, 0x120 + N, 0xf, 0xf, true);
+  const int hi = __builtin_amdgcn_update_dpp(0, (int)(u >> 32), 0x120 + N, 0xf, 0xf, true);
+  return x + __longlong_as_double(((long long)hi << 32) | (unsigned)lo);
+}
+// Lanes with bit BIT (32 or 16) of their index clear: a's sum over lane pairs
+// that differ in it; the others: b's.
+template <int BIT>
+__device__ __forceinline__ double half_exchange_add(double a, double b) {
+  const bool up = (threadIdx.x & BIT) != 0;
+  return (up ? b : a) + __shfl_xor(up ? a : b, BIT, 64);
+}
+
+// Sum of each of the NV values over the workgroup, in a fixed order: thread t
+// < NV returns value t.  red: 4 * NV doubles; contains one barrier, and red may
+// be written again after the next one.
+template <int NV>
+__device__ __forceinline__ double bs_sum(const double (&acc)[NV], double* red) {
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  double h[NV / 4];
+#pragma unroll
+  for (int j = 0; j < NV / 4; ++j) {
+    const double x = half_exchange_add<32>(acc[j], acc[j + NV / 2]);
+    const double y = half_exchange_add<32>(acc[j + NV / 4], acc[j + NV / 2 + NV / 4]);
+    h[j] = half_exchange_add<16>(x, y);
+  }
+#pragma unroll
+  for (int j = 0; j < NV / 4; ++j) {
+    h[j] = row_ror_add<8>(h[j]);
+    h[j] = row_ror_add<4>(h[j]);
+    h[j] = row_ror_add<2>(h[j]);
+    h[j] = row_ror_add<1>(h[j]);
+  }
+  if ((lane & 15) == 0) {
+    const int v0 = (lane >> 5) * (NV / 2) + ((lane >> 4) & 1) * (NV / 4);
+#pragma unroll
+    for (int j = 0; j < NV / 4; ++j) red[wave * NV + v0 + j] = h[j];
+  }
+  __syncthreads();
+  const int t = threadIdx.x < NV ? threadIdx.x : 0;
+  return ((red[t] + red[NV + t]) + red[2 * NV + t]) + red[3 * NV + t];
+}
+
+template <int CW, int TRANS>
+__global__ void __launch_bounds__(BS_THREADS) pobtas_block_reg_kernel(BlockSweepP P) {
+  constexpr int RW = bs_rw(CW, TRANS), NV = RW * CW, TU = BS_TIPMAX / BS_THREADS;
+  __shared__ double red[2][4 * NV];
+  __shared__ double ysh[NV];
+  __shared__ double xt[BS_TIPMAX];
+  const int tid = threadIdx.x;
+  const int b = P.b, n = P.n, a = P.a;
+  const int k0 = blockIdx.x * RW;
+  const int64_t bb = (int64_t)b * b;
+  const int q_ = tid / CW, c_ = tid % CW;
+  const bool out_thread = tid < NV && k0 + q_ < b && c_ < P.r;
+  const int64_t out_off = (int64_t)(k0 + q_) * P.ldb + c_;  // within a block's rows of B
+
+  auto load_rows = [&](double (&m)[BS_KU][RW], const double* M, int jlo, int jhi) {
+#pragma unroll
+    for (int u = 0; u < BS_KU; ++u) {
+      const int j = jlo + tid + u * BS_THREADS;
+#pragma unroll
+      for (int q = 0; q < RW; ++q)
+        m[u][q] = (j < jhi && k0 + q < b) ? M[(int64_t)(k0 + q) * b + j] : 0.0;
+    }
+  };
+  // published values of the thread's reduction indices, all asked for at once
+  auto poll = [&](double (&x)[BS_KU][CW], const double* src, int jlo, int jhi) {
+    long long spins = 0;
+    for (;;) {
+      bool empty = false;
+#pragma unroll
+      for (int u = 0; u < BS_KU; ++u) {
+        const int j = jlo + tid + u * BS_THREADS;
+#pragma unroll
+        for (int c = 0; c < CW; ++c) {
+          const unsigned long long v = (j < jhi && c < P.r) ? sw_ld(src + (int64_t)j * CW + c) : 0ull;
+          x[u][c] = __longlong_as_double((long long)v);
+          empty |= v == SW_EMPTY;
+        }
+      }
+      if (!empty) return;
+      if (!bs_spin(P, spins)) {
+#pragma unroll
+        for (int u = 0; u < BS_KU; ++u)
+#pragma unroll
+          for (int c = 0; c < CW; ++c) x[u][c] = 0.0;
+        return;
+      }
+    }
+  };
+  auto products = [&](const double (&m)[BS_KU][RW], const double (&x)[BS_KU][CW], double (&acc)[NV]) {
+#pragma unroll
+    for (int u = 0; u < BS_KU; ++u)
+#pragma unroll
+      for (int q = 0; q < RW; ++q)
+#pragma unroll
+        for (int c = 0; c < CW; ++c) acc[q * CW + c] = fma(m[u][q], x[u][c], acc[q * CW + c]);
+  };
+  auto zero = [&](double (&acc)[NV]) {
+#pragma unroll
+    for (int v = 0; v < NV; ++v) acc[v] = 0.0;
+  };
+  // R_i[m][k0 .. k0 + RW - 1] of the thread's tip entries (m, c)
+  auto load_arrow = [&](double (&rr)[TU][RW], int i) {
+#pragma unroll
+    for (int u = 0; u < TU; ++u) {
+      const int idx = tid + u * BS_THREADS, m = TRANS ? idx : idx / CW;
+#pragma unroll
+      for (int q = 0; q < RW; ++q)
+        rr[u][q] = (m < a && k0 + q < b) ? P.R[((int64_t)i * a + m) * b + k0 + q] : 0.0;
+    }
+  };
+  auto publish = [&](double* buf, int i, double v, bool to_b) {
+    if (!out_thread) return;
+    sw_st(buf + ((int64_t)i * b + k0) * CW + tid, v);
+    if (to_b) P.B[(int64_t)i * b * P.ldb + out_off] = v;
+  };
+  auto rhs = [&](int i) { return out_thread ? P.B[(int64_t)i * b * P.ldb + out_off] : 0.0; };
+
+  double ma[BS_KU][RW], mb[BS_KU][RW], x[BS_KU][CW], rr[TU][RW], acc[NV];
+  double bv = 0.0;
+  if (TRANS == 0) {
+    double tacc[TU] = {};
+    // tip: b_t -= R_i y_i over the workgroup's rows, a phase late (y in ysh)
+    auto tip = [&]() {
+#pragma unroll
+      for (int u = 0; u < TU; ++u) {
+        const int c = (tid + u * BS_THREADS) % CW;
+#pragma unroll
+        for (int q = 0; q < RW; ++q) tacc[u] = fma(rr[u][q], ysh[q * CW + c], tacc[u]);
+      }
+    };
+    const int nsolve = P.partial ? n - 1 : n;
+    bv = rhs(0);
+    load_rows(mb, P.Linv, 0, min(b, k0 + RW));
+    for (int i = 0; i < n; ++i) {
+      // phase A: t_i = b_i - L_{i,i-1} y_{i-1}
+      zero(acc);
+      if (i > 0) {
+        poll(x, P.sbuf + (int64_t)(i - 1) * b * CW, 0, b);
+        if (i < nsolve) load_rows(mb, P.Linv + i * bb, 0, min(b, k0 + RW));
+        asm volatile("" ::: "memory");  // the loads are issued here
+        products(ma, x, acc);
+      }
+      const double s = bs_sum<NV>(acc, red[0]);
+      if (i > 0 && a > 0) tip();
+      publish(P.tbuf, i, bv - s, i >= nsolve);
+      if (i >= nsolve) continue;
+      // phase B: y_i = Linv_i t_i (t rows 0 .. k0 + RW - 1)
+      zero(acc);
+      poll(x, P.tbuf + (int64_t)i * b * CW, 0, min(b, k0 + RW));
+      if (i + 1 < n) {
+        load_rows(ma, P.L + i * bb, 0, b);
+        bv = rhs(i + 1);
+      }
+      if (a > 0) load_arrow(rr, i);
+      asm volatile("" ::: "memory");
+      products(mb, x, acc);
+      const double y = bs_sum<NV>(acc, red[1]);
+      publish(P.sbuf, i, y, true);
+      if (tid < NV) ysh[tid] = out_thread ? y : 0.0;
+    }
+    if (a == 0) return;
+    __syncthreads();
+    if (nsolve == n) tip();  // (partial: the last solved block's share was added above)
+    // publish this workgroup's tip partial sums
+#pragma unroll
+    for (int u = 0; u < TU; ++u) {
+      const int idx = tid + u * BS_THREADS;
+      if (idx < a * CW) sw_st(P.tpart + (int64_t)blockIdx.x * a * CW + idx, tacc[u]);
+    }
+    if (blockIdx.x != 0) return;
+    bs_tip_solve<CW>(P, xt);
+    return;
+  }
+  bs_tip_back<CW>(P, xt);
+  const bool open = P.partial != 0;  // x_{n-1} is the given B block
+  if (open) {
+    publish(P.sbuf, n - 1, rhs(n - 1), false);
+    if (n == 1) return;
+  }
+  const int i0 = open ? n - 2 : n - 1;
+  bv = rhs(i0);
+  if (i0 + 1 < n) load_rows(ma, P.L + i0 * bb, 0, b);
+  if (a > 0) load_arrow(rr, i0);
+  for (int i = i0; i >= 0; --i) {
+    // phase A: s_i = y_i - L_{i+1,i}^T x_{i+1} - R_i^T x_t (P.L holds L^T)
+    zero(acc);
+    if (a > 0) {
+#pragma unroll
+      for (int u = 0; u < TU; ++u) {
+        const int m = tid + u * BS_THREADS;
+        if (m < a) {
+#pragma unroll
+          for (int q = 0; q < RW; ++q)
+#pragma unroll
+            for (int c = 0; c < CW; ++c) acc[q * CW + c] = fma(rr[u][q], xt[m * CW + c], acc[q * CW + c]);
+        }
+      }
+    }
+    if (i + 1 < n) poll(x, P.sbuf + (int64_t)(i + 1) * b * CW, 0, b);
+    load_rows(mb, P.Linv + i * bb, k0, b);
+    asm volatile("" ::: "memory");
+    if (i + 1 < n) products(ma, x, acc);
+    const double s = bs_sum<NV>(acc, red[0]);
+    publish(P.tbuf, i, bv - s, false);
+    // phase B: x_i = Linv_i^T s_i (s rows k0 .. b - 1)
+    zero(acc);
+    poll(x, P.tbuf + (int64_t)i * b * CW, k0, b);
+    if (i > 0) {
+      load_rows(ma, P.L + (i - 1) * bb, 0, b);
+      bv = rhs(i - 1);
+      if (a > 0) load_arrow(rr, i - 1);
+    }
+    asm volatile("" ::: "memory");
+    products(mb, x, acc);
+    publish(P.sbuf, i, bs_sum<NV>(acc, red[1]), true);
   }
 }
 
