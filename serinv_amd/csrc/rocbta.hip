@@ -709,31 +709,38 @@ __global__ void fill_u64_kernel(unsigned long long* p, int64_t count, unsigned l
 }
 
 // Solve algorithm: the block-level sweep (precomputed diagonal-block
-// inverses, two dependent device-wide products per block row) for at most 4
+// inverses, two dependent device-wide products per block row) for few
 // right-hand sides, its wide form (64 columns per launch, MFMA tiles) for
-// more, the 64-row-tile sweep for blocks of one tile and what the others do
-// not fit, the launch-per-tile form for partial solves there.  Per block row
-// the block sweep takes 5.5 us at r = 1 and 8.5 us at r = 4 whatever b is, the
-// wide one 10 us, the tile sweep 4 to 7 us per 64-row tile.  Measured, N + C
-// at n = 64, b = 130, a = 16: r = 1 853 us against 1722 us for the tile sweep,
-// r = 4 1239 against 1959; b = 256, r = 8: wide 1469, block 1905, tile 3539.
+// more, the 64-row-tile sweep for small blocks and what the others do not fit,
+// the launch-per-tile form for partial solves there.  Measured, N + C in us:
+//                        block  wide  tiles
+//   n=8   b=96   r=2       236   224    272
+//   n=64  b=130  r=1 / 4 / 8    688 / 931 / 1358 block, 1762 / 1988 / 2715 tiles
+//   n=64  b=128  r=4       871   772   1331
+//   n=64  b=256  r=1       723   904
+//   n=64  b=256  r=4 / 8   985 / 1423 block, 907 / 908 wide, 3571 tiles (r=8)
+//   n=64  b=1024 r=4 / 8  3209 / 4195 block, 3399 / 3403 wide
+//   n=32  b=64   r=1       316          340
+//   n=64  b=64   r=4       787   603    678
+//   n=32  b=48   r=4       446          396
 // ROCBTA_POBTAS_ALGO = block | wide | sweep | loop forces one (tests cover
 // all four; block and wide fall back when the shape does not fit them).
 enum SolveAlgo { SOLVE_LOOP = 0, SOLVE_SWEEP = 1, SOLVE_BLOCK = 2, SOLVE_WIDE = 3 };
 // The block and wide sweeps need their inverses' launches first (about 40 us
-// a call): they are taken from this many tile steps saved on.  n = 8, b = 96
-// (8 saved): 236 us against 228 for the tile sweep at r = 4; b = 130 (16): 258
-// against 297.
-constexpr int BS_MIN_SAVED = 12;
+// a call): they are taken from this many tile steps saved on, for blocks of one
+// full tile from BS_MIN_N block rows on.
+constexpr int BS_MIN_SAVED = 8;
+constexpr int BS_MIN_N = 32;
 constexpr int BS_MIN_B = 256;   // and for these blocks always
 constexpr int BS_MAX_G = 1024;  // workgroups of the block sweep (tip partial sums sized for it)
 
 int bs_cw(int64_t r) { return r <= 1 ? 1 : (r <= 4 ? 4 : 8); }
 bool bs_fits(int64_t a, int64_t r) { return a * bs_cw(r) <= BS_TIPMAX; }
-// The block sweep re-reads the factor once per group of columns, and groups of
-// 8 cost it 13.6 us per block row, so it serves 5 to 8 columns only where the
-// wide one does not fit (b = 130, r = 8: 1839 us against 2673 for the tiles).
+// The block sweep re-reads the factor once per group of columns, so it serves 5
+// to 8 of them only where the wide one does not fit; from b = 513 on the wide
+// sweep's MFMA time makes it the slower one up to 4 columns.
 constexpr int BS_MAX_R = 8;
+constexpr int WD_FEW_B = 512;
 
 // The wide sweep: full solves with b a multiple of its 16-row tiles.
 bool wd_fits(int64_t b, int partial) { return !partial && b >= WD_CW && b % WD_T == 0; }
@@ -745,9 +752,11 @@ int pobtas_algo(int64_t n, int64_t b, int64_t a, int64_t r, int partial) {
     return wd_fits(b, partial) ? SOLVE_WIDE : (partial ? SOLVE_LOOP : SOLVE_SWEEP);
   if (e && strcmp(e, "sweep") == 0) return partial ? SOLVE_LOOP : SOLVE_SWEEP;
   if (e && strcmp(e, "block") == 0) return bs_fits(a, r) ? SOLVE_BLOCK : (partial ? SOLVE_LOOP : SOLVE_SWEEP);
-  if (b >= BS_MIN_B || n * (cdiv(b, SW_T) - 1) >= BS_MIN_SAVED) {
+  if (b > SW_T ? (b >= BS_MIN_B || n * (cdiv(b, SW_T) - 1) >= BS_MIN_SAVED)
+               : (b == SW_T && n >= BS_MIN_N)) {
     const bool wide = wd_fits(b, partial);
-    if (r <= (wide ? 4 : BS_MAX_R) && bs_fits(a, r)) return SOLVE_BLOCK;
+    if (wide && r > (b <= WD_FEW_B ? 1 : 4)) return SOLVE_WIDE;
+    if (r <= (b > SW_T ? BS_MAX_R : 1) && bs_fits(a, r)) return SOLVE_BLOCK;
     if (wide) return SOLVE_WIDE;
   }
   return partial ? SOLVE_LOOP : SOLVE_SWEEP;
@@ -1070,7 +1079,14 @@ int pobtas_wide(int64_t n, int64_t b, int64_t a, const double* D, const double* 
     RB_CHECK(hipGetLastError());
     const int nitems = (bi / WD_T) * ((rc_ + WD_T - 1) / WD_T);
     P.G = std::min(std::min(nitems, WD_MAX_G), device_cus());
-    if (trans)
+    // a workgroup per item and a phase's factor entries in registers: the form
+    // that loads a phase ahead
+    const bool reg = P.G == nitems && bi <= 16 * WD_NW * WD_NB;
+    if (reg && trans)
+      pobtas_wide_reg_kernel<1><<<P.G, WD_THREADS, 0, s>>>(P);
+    else if (reg)
+      pobtas_wide_reg_kernel<0><<<P.G, WD_THREADS, 0, s>>>(P);
+    else if (trans)
       pobtas_wide_kernel<1><<<P.G, WD_THREADS, 0, s>>>(P);
     else
       pobtas_wide_kernel<0><<<P.G, WD_THREADS, 0, s>>>(P);

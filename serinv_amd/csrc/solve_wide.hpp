@@ -204,6 +204,159 @@ __global__ void __launch_bounds__(WD_THREADS) pobtas_wide_kernel(WideSweepP P) {
   }
 }
 
+// The sweep where every item has a workgroup of its own and a wave's share of
+// the reduction is at most WD_NB groups (b <= 16 WD_NW WD_NB): the factor's
+// entries of a phase are held in registers and loaded a phase ahead, behind the
+// polls of the phase before (loads complete in order).  A poll that finds
+// values missing waits for one of them and then asks for all again: waiting
+// for each in turn cost a round trip per value.  Bound by two such round trips
+// and 1.8 + 0.9 us of MFMA (b = 1024) per block row.  Measured at n = 256, b =
+// 1024, r = 64: forward 3.4 (5.8 streamed) ms, backward 3.1 (4.2) ms.
+template <int TRANS>
+__global__ void __launch_bounds__(WD_THREADS) pobtas_wide_reg_kernel(WideSweepP P) {
+  __shared__ double red[2][WD_NW * 256];
+  const int b = P.b, n = P.n;
+  const int ntc = (P.r + WD_T - 1) / WD_T;
+  const int item = wd_item(blockIdx.x, (b / WD_T) * ntc);
+  const int k0 = (item / ntc) * WD_T, c0 = (item % ntc) * WD_T;
+  const int t = threadIdx.x, lane = t & 63, wave = __builtin_amdgcn_readfirstlane(t >> 6);
+  const int li = lane & 15, g4 = (lane >> 4) * 4;
+  const int64_t bb = (int64_t)b * b;
+  typedef double wdbl2u __attribute__((ext_vector_type(2), aligned(8)));
+
+  // lane offsets (bytes) to a wave-uniform address
+  // (recomputed where used: kept across the block rows, the addresses of a phase
+  // take more registers than there are)
+  auto fresh = [&]() {
+    int w = wave;
+    asm volatile("" : "+s"(w));
+    return w;
+  };
+  const uint32_t moff = TRANS ? ((uint32_t)g4 * b + k0 + li) * 8u : ((uint32_t)(k0 + li) * b + g4) * 8u;
+  const uint32_t voff = ((uint32_t)g4 * WD_CW + c0 + li) * 8u;
+  auto load_m = [&](double (&m)[WD_NB][4], const double* M, int jlo, int jhi) {
+    const int wv = fresh();
+#pragma unroll
+    for (int u = 0; u < WD_NB; ++u) {
+      const int j = jlo + 16 * (wv + WD_NW * u);
+      if (j >= jhi) break;
+      if (TRANS) {
+#pragma unroll
+        for (int s = 0; s < 4; ++s)
+          m[u][s] = *reinterpret_cast<const double*>(
+              reinterpret_cast<const char*>(M + (int64_t)(j + s) * b) + moff);
+      } else {
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {
+          const wdbl2u x = *reinterpret_cast<const wdbl2u*>(
+              reinterpret_cast<const char*>(M + j + 2 * h) + moff);
+          m[u][2 * h] = x.x;
+          m[u][2 * h + 1] = x.y;
+        }
+      }
+    }
+  };
+  // acc of the wave's part of the tile op(M) src: src polled and multiplied four
+  // groups at a time
+  constexpr int H = WD_NB / 2;
+  auto part = [&](const double (&m)[WD_NB][4], const double* src, int jlo, int jhi) {
+    const int wv = fresh();
+    long long spins = 0;
+    // lane u waits for one value of group u first: polling all of them takes
+    // 128 KiB per workgroup and round
+    {
+      const int j = jlo + 16 * (wv + WD_NW * lane);
+      if (lane < WD_NB && j < jhi)
+        while (sw_ld(src + (int64_t)(j + 15) * WD_CW + c0 + 15) == SW_EMPTY)
+          if (!wd_spin(P, spins)) break;
+    }
+    f64x4 acc = {0.0, 0.0, 0.0, 0.0};
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+      const int j0 = jlo + 16 * (wv + WD_NW * H * h);
+      if (j0 >= jhi) break;
+      double v[H][4];
+      for (;;) {
+        bool late = false;
+#pragma unroll
+        for (int u = 0; u < H; ++u) {
+          const int j = j0 + 16 * WD_NW * u;
+          const char* p = reinterpret_cast<const char*>(src + (int64_t)(j < jhi ? j : j0) * WD_CW);
+#pragma unroll
+          for (int s = 0; s < 4; ++s)
+            v[u][s] = __longlong_as_double((long long)sw_ld(
+                reinterpret_cast<const double*>(p + voff + (uint32_t)(s * WD_CW * 8))));
+        }
+#pragma unroll
+        for (int u = 0; u < H; ++u)
+#pragma unroll
+          for (int s = 0; s < 4; ++s)
+            late |= (unsigned long long)__double_as_longlong(v[u][s]) == SW_EMPTY;
+        if (!__any(late)) break;
+        if (!wd_spin(P, spins)) {
+#pragma unroll
+          for (int u = 0; u < H; ++u)
+#pragma unroll
+            for (int s = 0; s < 4; ++s) v[u][s] = 0.0;
+          break;
+        }
+      }
+#pragma unroll
+      for (int u = 0; u < H; ++u) {
+        if (j0 + 16 * WD_NW * u >= jhi) break;
+#pragma unroll
+        for (int s = 0; s < 4; ++s) acc = mfma_f64(m[H * h + u][s], v[u][s], acc);
+      }
+    }
+    return acc;
+  };
+  // thread t < 256: entry (t / 16, t % 16) of the waves' sum
+  auto sum = [&](const f64x4& acc, double* p) {
+#pragma unroll
+    for (int r = 0; r < 4; ++r) p[wave * 256 + acc_row_f64(lane, r) * 16 + acc_col(lane)] = acc[r];
+    __syncthreads();
+    double o = p[t & 255];
+#pragma unroll
+    for (int w = 1; w < WD_NW; ++w) o += p[w * 256 + (t & 255)];
+    return o;
+  };
+  const int row = (t >> 4) & 15, c = c0 + (t & 15);
+  const bool live = t < 256 && c < P.r;
+  auto rhs = [&](int i) {
+    return live ? P.B[((int64_t)i * b + k0 + row) * P.ldb + c] : 0.0;
+  };
+  const int jlo = TRANS ? k0 : 0, jhi = TRANS ? b : k0 + WD_T;
+
+  double m[WD_NB][4];
+  f64x4 acc = {0.0, 0.0, 0.0, 0.0};
+  double bv = rhs(TRANS ? n - 1 : 0);
+  load_m(m, P.Linv + (int64_t)(TRANS ? n - 1 : 0) * bb, jlo, jhi);
+#pragma unroll 1
+  for (int step = 0; step < n; ++step) {
+    const int i = TRANS ? n - 1 - step : step;
+    const int64_t grow = (int64_t)i * b + k0 + row;
+    // phase A: t_i = b_i - L_{i,i-1} y_{i-1}  /  s_i = y'_i - L_{i+1,i}^T x_{i+1}
+    double o = 0.0;
+    if (step > 0) {
+      acc = part(m, P.sbuf + (int64_t)(TRANS ? i + 1 : i - 1) * b * WD_CW, 0, b);
+      load_m(m, P.Linv + (int64_t)i * bb, jlo, jhi);
+      asm volatile("" ::: "memory");  // the loads are issued here
+      o = sum(acc, red[0]);
+    }
+    if (t < 256) sw_st(P.tbuf + grow * WD_CW + c, live ? bv - o : 0.0);
+    // phase B: y_i = Linv_i t_i (rows up to the tile's)  /  x_i = Linv_i^T s_i (from it on)
+    acc = part(m, P.tbuf + (int64_t)i * b * WD_CW, jlo, jhi);
+    if (step + 1 < n) {
+      load_m(m, P.L + (int64_t)(TRANS ? i - 1 : i) * bb, 0, b);
+      bv = rhs(TRANS ? i - 1 : i + 1);
+    }
+    asm volatile("" ::: "memory");
+    o = sum(acc, red[1]);
+    if (live) P.B[grow * P.ldb + c] = o;
+    if (t < 256) sw_st(P.sbuf + grow * WD_CW + c, live ? o : 0.0);
+  }
+}
+
 // Bt[m][c] = B0[m][c] - sum_{i < nblk} Pt[i][m][c] (fixed order), for the
 // forward tip right-hand side; m < a, c < r (row strides ldb, r).
 __global__ void wide_tip_reduce_kernel(double* out, const double* B0, int64_t ldb,

@@ -35,3 +35,21 @@ def test_block_solve_matches_oracle(gpu_device, monkeypatch, n, b, a, r, partial
         serinv_np.pobtas(D, L, R, T, B, trans=trans, partial=partial)
         algs.pobtas(d, l, rr, t, bb, trans=trans, partial=partial)
         assert relerr(to_host(bb)[0], B) < TOL, trans
+
+
+@pytest.mark.parametrize("n,b,a,r", [(31, 64, 3, 2), (32, 64, 3, 1), (32, 64, 0, 2), (7, 96, 12, 1), (8, 96, 12, 1),
+                                     (8, 96, 12, 2), (9, 65, 5, 8), (9, 65, 5, 9), (2, 512, 4, 2), (2, 528, 4, 4),
+                                     (2, 528, 4, 5), (32, 64, 600, 1)])
+def test_default_solve_matches_oracle(gpu_device, monkeypatch, n, b, a, r):
+    """The form the sizes select, on both sides of each line of the rule."""
+    import serinv_amd.algs as algs
+
+    monkeypatch.delenv("ROCBTA_POBTAS_ALGO", raising=False)
+    print(f"pobtas n={n} b={b} a={a} r={r}", flush=True)
+    D, L, R, T, B = bta_spd(n, b, a, seed=5600 + n + b + a + r, n_rhs=r)
+    serinv_np.pobtaf(D, L, R, T)
+    d, l, rr, t, bb = to_dev(gpu_device, D, L, R, T, B)
+    for trans in ("N", "C"):
+        serinv_np.pobtas(D, L, R, T, B, trans=trans)
+        algs.pobtas(d, l, rr, t, bb, trans=trans)
+        assert relerr(to_host(bb)[0], B) < TOL, trans

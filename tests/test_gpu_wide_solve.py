@@ -58,3 +58,11 @@ def test_wide_solve_default_selection(algs, gpu_device, monkeypatch):
     algs.pobtas(d, l, rr, t, bb, trans="N")
     algs.pobtas(d, l, rr, t, bb, trans="C")
     assert relerr(to_host(bb)[0], np.linalg.solve(A, B)) < 1e-11
+
+
+@pytest.mark.parametrize("n,b,a,r", [(3, 1024, 0, 5), (2, 1024, 8, 64), (3, 512, 5, 33), (2, 1040, 3, 64),
+                                     (2, 1040, 3, 9), (3, 144, 70, 16)])
+def test_wide_solve_forms(algs, gpu_device, monkeypatch, n, b, a, r):
+    """Both forms of the wide sweep at their edge: a phase's factor entries in
+    registers up to b = 1024 (one workgroup per 16 x 16 tile), streamed beyond."""
+    test_wide_solve_matches_oracle(algs, gpu_device, monkeypatch, n, b, a, r)
