@@ -176,7 +176,9 @@ template <bool AK, bool BK, typename ACC>
 __device__ __forceinline__ void gemm_wave(const double* A, int64_t lda, const double* B, int64_t ldb,
                                           int kb, int ke, int rows, int cols, int g0, int gs,
                                           ACC (&acc)[2][2]) {
-  const int full = rows >= GW && cols >= GW ? (ke - kb) / GK : 0;  // groups without checks
+  // groups without checks: full blocks whose lane offsets fit in 32 bits
+  const bool fits = lda < (1 << 24) && ldb < (1 << 24);
+  const int full = rows >= GW && cols >= GW && fits ? (ke - kb) / GK : 0;
   int g = g0;
   if (g < full) {
     const GStream sa = stream_at<AK>(A, lda), sb = stream_at<BK>(B, ldb);
