@@ -890,14 +890,17 @@ BsLayout bs_layout(int64_t n, int64_t b, int64_t a, int64_t r) {
   return l;
 }
 
+// A workgroup per row group and the rows of a phase in registers: the form
+// that loads a phase ahead and needs no transposes.
+bool bs_reg(int64_t b) {
+  return cdiv(b, bs_rw(1, 0)) <= std::min(BS_MAX_G, device_cus()) && b <= BS_KU * BS_THREADS;
+}
+
 template <int CW>
 int launch_block_sweep(BlockSweepP P, hipStream_t s) {
   const int rw = bs_rw(CW, P.trans);
-  const int ngroups = (P.b + rw - 1) / rw;
-  P.G = std::min(std::min(ngroups, BS_MAX_G), device_cus());
-  // a workgroup per row group and the rows of a phase in registers: the form
-  // that loads a phase ahead
-  const bool reg = P.G == ngroups && P.b <= BS_KU * BS_THREADS;
+  P.G = std::min(std::min(cdiv(P.b, rw), BS_MAX_G), device_cus());
+  const bool reg = bs_reg(P.b);
   if (reg && P.trans == 0)
     pobtas_block_reg_kernel<CW, 0><<<P.G, BS_THREADS, 0, s>>>(P);
   else if (reg)
@@ -922,8 +925,8 @@ int pobtas_block(int64_t n, int64_t b, int64_t a, const double* D, const double*
   RB_CHECK(hipGetLastError());
   double* Linv = (double*)(ws + lay.linv);
   double* Tinv = (double*)(ws + lay.tinv);
-  // Linv is read on and below the diagonal tiles only (the backward sweep
-  // reads it after the in-place transpose, on and above them)
+  // Linv is read on and below the diagonal tiles only (the streamed backward
+  // sweep reads it after the in-place transpose, on and above them)
   int rc = block_trtri(D, b, b * b, Linv, b, b * b, (int)b, (int)n, (double*)(ws + lay.w), s, true,
                        false);
   if (rc) return rc;
@@ -931,8 +934,9 @@ int pobtas_block(int64_t n, int64_t b, int64_t a, const double* D, const double*
     rc = block_trtri(T, a, 0, Tinv, a, a * a, (int)a, 1, (double*)(ws + lay.wt), s);
     if (rc) return rc;
   }
-  if (trans) {
-    // the backward sweep reads L_{i+1,i}^T and (the upper triangle of)
+  const bool transposed = trans && !bs_reg(b);
+  if (transposed) {
+    // the streamed backward sweep reads L_{i+1,i}^T and (the upper triangle of)
     // Linv_i^T by rows
     const int T = (int)((b + 63) / 64);
     for (int64_t z0 = 0; z0 < n; z0 += 65535) {
@@ -950,7 +954,7 @@ int pobtas_block(int64_t n, int64_t b, int64_t a, const double* D, const double*
     }
   }
   BlockSweepP P{};
-  P.L = trans ? (const double*)(ws + lay.lt) : L;
+  P.L = transposed ? (const double*)(ws + lay.lt) : L;
   P.R = R;
   P.Linv = Linv;
   P.Tinv = Tinv;

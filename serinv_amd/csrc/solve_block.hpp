@@ -18,10 +18,12 @@
 // forward, y_{n-1} = t_{n-1} and b_t -= sum_{i<n-1} R_i y_i is left unsolved;
 // backward, x_{n-1} and x_t are the given B rows.
 //
-// The backward sweep reads the transposes of L_{i+1,i} and Linv_i, written
-// beforehand (transpose_blocks_kernel), so that both directions read whole
-// matrix rows: with the factor's own layout every output row of the
-// backward products is a matrix column, read in 8-byte pieces.
+// The streamed form's backward sweep reads the transposes of L_{i+1,i} and
+// Linv_i, written beforehand (transpose_blocks_kernel), so that both directions
+// read whole matrix rows: with the factor's own layout every output row of the
+// backward products is a matrix column.  The form with a workgroup per row
+// group (pobtas_block_reg_kernel) reads the columns where they are, four at a
+// time, a phase ahead.
 //
 // Work split: the b rows of a block are cut into row groups of RW rows;
 // workgroup w owns row groups w, w + G, w + 2G, ... of every block (G
@@ -98,10 +100,10 @@ __global__ void __launch_bounds__(256) transpose_lower_to_upper_kernel(double* X
 }
 
 struct BlockSweepP {
-  const double* L;     // (n-1, b, b); backward: the transposes L_{i+1,i}^T
+  const double* L;     // (n-1, b, b); backward, streamed form: the transposes L_{i+1,i}^T
   const double* R;     // (n, a, b)
   const double* Linv;  // (n, b, b): inverses of the diagonal blocks (dense, zero above);
-                       // backward: their transposes (zero below)
+                       // backward, streamed form: their transposes (zero below)
   const double* Tinv;  // (a, a): inverse of the tip factor (zero above)
   double* B;           // right-hand sides, columns [0, r), row stride ldb
   int64_t ldb;
@@ -487,7 +489,8 @@ __global__ void __launch_bounds__(BS_THREADS) pobtas_block_kernel(BlockSweepP P)
 // waves' lanes by half-exchanges and row rotations and needs one barrier.
 // Every poll round asks for all values of a thread at once.
 // Bound by that round trip.  Measured, a sweep of n = 256, b = 1024, r = 1: 1.48
-// ms (1.79 streamed), n = 100, b = 130, r = 3: 0.55 (0.78) ms.
+// ms (1.79 streamed), n = 100, b = 130, r = 3: 0.55 (0.78) ms.  Backward without
+// the transposed copies, N + C at n = 256, b = 1024, r = 1: 10.1 (10.7) ms.
 template <int N>
 __device__ __forceinline__ double row_ror_add(double x) {
   const unsigned long long u = (unsigned long long)__double_as_longlong(x);
@@ -533,6 +536,8 @@ __device__ __forceinline__ double bs_sum(const double (&acc)[NV], double* red) {
   return ((red[t] + red[NV + t]) + red[2 * NV + t]) + red[3 * NV + t];
 }
 
+typedef double bsdbl2u __attribute__((ext_vector_type(2), aligned(8)));  // any double address
+
 template <int CW, int TRANS>
 __global__ void __launch_bounds__(BS_THREADS) pobtas_block_reg_kernel(BlockSweepP P) {
   constexpr int RW = bs_rw(CW, TRANS), NV = RW * CW, TU = BS_TIPMAX / BS_THREADS;
@@ -541,7 +546,11 @@ __global__ void __launch_bounds__(BS_THREADS) pobtas_block_reg_kernel(BlockSweep
   __shared__ double xt[BS_TIPMAX];
   const int tid = threadIdx.x;
   const int b = P.b, n = P.n, a = P.a;
-  const int k0 = blockIdx.x * RW;
+  // Backward reads the matrices by columns, RW of them: each XCD gets a contiguous
+  // range of row groups, so that the workgroups that share a 128-byte line
+  // find it in one L2.
+  const int gq = P.G / 8, gr = P.G % 8, gx = blockIdx.x % 8;
+  const int k0 = RW * (TRANS ? gx * gq + min(gx, gr) + (int)blockIdx.x / 8 : (int)blockIdx.x);
   const int64_t bb = (int64_t)b * b;
   const int q_ = tid / CW, c_ = tid % CW;
   const bool out_thread = tid < NV && k0 + q_ < b && c_ < P.r;
@@ -551,9 +560,21 @@ __global__ void __launch_bounds__(BS_THREADS) pobtas_block_reg_kernel(BlockSweep
 #pragma unroll
     for (int u = 0; u < BS_KU; ++u) {
       const int j = jlo + tid + u * BS_THREADS;
+      if (TRANS && k0 + RW <= b) {  // whole columns k0 .. k0 + RW - 1
+        const bsdbl2u* p = reinterpret_cast<const bsdbl2u*>(M + (int64_t)j * b + k0);
 #pragma unroll
-      for (int q = 0; q < RW; ++q)
-        m[u][q] = (j < jhi && k0 + q < b) ? M[(int64_t)(k0 + q) * b + j] : 0.0;
+        for (int q = 0; q < RW; q += 2) {
+          const bsdbl2u v = j < jhi ? p[q / 2] : bsdbl2u{0.0, 0.0};
+          m[u][q] = v.x;
+          m[u][q + 1] = v.y;
+        }
+      } else {
+#pragma unroll
+        for (int q = 0; q < RW; ++q)
+          m[u][q] = (j < jhi && k0 + q < b)
+                        ? (TRANS ? M[(int64_t)j * b + k0 + q] : M[(int64_t)(k0 + q) * b + j])
+                        : 0.0;
+      }
     }
   };
   // published values of the thread's reduction indices, all asked for at once
@@ -677,7 +698,7 @@ __global__ void __launch_bounds__(BS_THREADS) pobtas_block_reg_kernel(BlockSweep
   if (i0 + 1 < n) load_rows(ma, P.L + i0 * bb, 0, b);
   if (a > 0) load_arrow(rr, i0);
   for (int i = i0; i >= 0; --i) {
-    // phase A: s_i = y_i - L_{i+1,i}^T x_{i+1} - R_i^T x_t (P.L holds L^T)
+    // phase A: s_i = y_i - L_{i+1,i}^T x_{i+1} - R_i^T x_t
     zero(acc);
     if (a > 0) {
 #pragma unroll
