@@ -19,12 +19,15 @@
 // MFMA step takes 64 cycles on its SIMD, so a wave needs 4 KiB of operands per
 // 512 cycles, which the caches deliver without staging them in LDS, and the
 // waves run without a barrier until their blocks are summed.  Bound by the
-// L1's load path: two groups in flight at four waves per SIMD measured best
-// (three or four groups at two waves per SIMD: 640 against 581 us for sixteen
-// 1024^3 products).  Measured, against the LDS-staged 64-tile kernel before:
-// 64^3 4.5 (14) us, 512^3 10.7 (31) us, sixteen 1024^3 630 us = 54.6 TFLOP/s
-// (36.4 TFLOP/s); with both operands stored along their rows (A transposed)
-// 581 us = 59 TFLOP/s, 83% of what the MFMA pipes reach at the clock held.
+// MFMA pipes for large products (63 TFLOP/s is 88% of what they reach at the
+// clock held), by the L1's load path behind them and, for small ones, by the
+// round trips of a launch: two groups in flight at four waves per SIMD measured
+// best (three or four groups at two waves per SIMD: 640 against 581 us for
+// sixteen 1024^3 products).  Measured, against the LDS-staged 64-tile kernel before
+// (A and B as they are / B transposed / A transposed): 64^3 4.6 / 4.8 / 4.5
+// (9.5) us, 512^3 10.2 / 10.6 / 10.0 (26.5) us, 1024^3 46 / 49 / 44 (52 / 50 /
+// 51) us, sixteen 1024^3 551 / 578 / 544 (630 / 626 / 628) us; FP32 products,
+// sixteen 1024^3 429 / 486 / 402 (457 / 444 / 436) us.
 #pragma once
 #include "common.hpp"
 
@@ -45,11 +48,12 @@ struct GemmTerm {
   const double* B;
   int64_t lda, ldb;
   int64_t sA1, sA2, sB1, sB2;  // batch strides (elements) along batch dims 1 and 2
-  int K;
-  uint8_t transA, transB;
-  uint8_t triA;  // shape of op(A): TRI_LOWER => op(A)(m,k) = 0 for k > m
-  uint8_t triB;  // shape of op(B): TRI_LOWER => op(B)(k,n) = 0 for k < n
   double alpha;
+  // (whole words: scalar loads read no bytes)
+  int K;
+  int transA, transB;
+  int triA;  // shape of op(A): TRI_LOWER => op(A)(m,k) = 0 for k > m
+  int triB;  // shape of op(B): TRI_LOWER => op(B)(k,n) = 0 for k < n
 };
 
 struct GemmProblem {
@@ -91,14 +95,27 @@ typedef double dbl2u __attribute__((ext_vector_type(2), aligned(8)));  // any do
 //   k = k0 + 8 (s >> 1) + 2 lk + (s & 1),
 // the same for both operands (which of the four k of a step sits in which
 // lane group is free).  Either storage then takes four 16-byte loads per lane
-// and group: KC two per row (64 contiguous bytes per row and load), otherwise
-// one per k (256 contiguous bytes per k).
+// and group: one per k (256 contiguous bytes per k), or, KC, one per row of four
+// (128 contiguous bytes of eight rows), two adjacent lanes on one line, which then
+// trade (frag_trade).  What a load costs is the lines among neighbouring lanes:
+// with a row per lane, 64 bytes of sixteen rows a load, sixteen 1024^3 products
+// took 598 us with one operand stored this way and 892 us with both (551 and 578
+// so); with lanes four apart on one line it was 593 and 894 us.
 struct GFrag {
   double v[2][4];  // [sub-block][step]
 };
 
-// The loads address a wave-uniform pointer plus two 32-bit lane offsets
-// (bytes), so that a stream takes two registers per lane.
+// Lane index as a new value at each call: what is formed from it is computed
+// where it is used.  The compiler otherwise forms it once for all the loops
+// below, and then spills in them.
+__device__ __forceinline__ int gemm_lane() {
+  int l = threadIdx.x & 63;
+  asm volatile("" : "+v"(l));
+  return l;
+}
+
+// The loads address a wave-uniform pointer plus 32-bit lane offsets (bytes), so
+// that a stream takes at most two registers per lane.
 struct GStream {
   const char* p;  // wave-uniform, at k = 0 of the K range
   int64_t ld;     // bytes
@@ -107,13 +124,13 @@ struct GStream {
 
 template <bool KC>
 __device__ __forceinline__ GStream stream_at(const double* p, int64_t ld) {
-  const int lane = threadIdx.x & 63, li = lane & 15, lk = lane >> 4;
+  const int lane = gemm_lane(), li = lane & 15, lk = lane >> 4;
   GStream s;
   s.p = reinterpret_cast<const char*>(p);
   s.ld = ld * 8;
 #pragma unroll
   for (int i = 0; i < 2; ++i)
-    s.off[i] = KC ? (uint32_t)(2 * li + i) * (uint32_t)(ld * 8) + 16 * lk
+    s.off[i] = KC ? (uint32_t)(2 * (li & ~1)) * (uint32_t)(ld * 8) + 64 * (li & 1) + 16 * lk
                   : (uint32_t)(2 * lk + i) * (uint32_t)(ld * 8) + 16 * li;
   return s;
 }
@@ -121,15 +138,14 @@ __device__ __forceinline__ GStream stream_at(const double* p, int64_t ld) {
 template <bool KC>
 __device__ __forceinline__ void frag_load(const GStream& st, int k0, GFrag& f) {
   if (KC) {
+    // load t: row 4 (li / 2) + t, k = 8 (li % 2) + 2 lk and the next
     const char* p = st.p + (int64_t)k0 * 8;
 #pragma unroll
-    for (int i = 0; i < 2; ++i)
-#pragma unroll
-      for (int h = 0; h < 2; ++h) {
-        const dbl2u x = *reinterpret_cast<const dbl2u*>(p + st.off[i] + 64 * h);
-        f.v[i][2 * h] = x.x;
-        f.v[i][2 * h + 1] = x.y;
-      }
+    for (int t = 0; t < 4; ++t) {
+      const dbl2u x = *reinterpret_cast<const dbl2u*>(p + t * st.ld + st.off[0]);
+      f.v[t & 1][2 * (t >> 1)] = x.x;
+      f.v[t & 1][2 * (t >> 1) + 1] = x.y;
+    }
   } else {
 #pragma unroll
     for (int h = 0; h < 2; ++h) {
@@ -144,7 +160,54 @@ __device__ __forceinline__ void frag_load(const GStream& st, int k0, GFrag& f) {
   }
 }
 
-// The same with zeros past row r_ok and index k_ok (exclusive).
+// Even lanes keep x and get y from the odd neighbour's x; odd lanes keep y and
+// get x from the even neighbour's y.  One select per 32 bits, which takes one of
+// its operands from the other lane (as a lane read and a select each, B
+// transposed took 600 us); the wait states in front of a DPP read are written
+// out, since the compiler does not track them into an asm statement.
+#define ROCBTA_SEL(d, n, o, q) \
+  "v_cndmask_b32_dpp " d ", " n ", " o ", vcc quad_perm:[" q "] row_mask:0xf bank_mask:0xf\n\t"
+__device__ __forceinline__ void pair_trade(double& x0, double& x1, double& y0, double& y1) {
+  constexpr uint64_t even = 0x5555555555555555ull;
+  const uint64_t u[4] = {__builtin_bit_cast(uint64_t, x0), __builtin_bit_cast(uint64_t, x1),
+                         __builtin_bit_cast(uint64_t, y0), __builtin_bit_cast(uint64_t, y1)};
+  uint32_t x[4], y[4], a[4];
+#pragma unroll
+  for (int w = 0; w < 4; ++w) {
+    x[w] = (uint32_t)(u[w >> 1] >> (32 * (w & 1)));
+    y[w] = (uint32_t)(u[2 + (w >> 1)] >> (32 * (w & 1)));
+  }
+  asm("s_mov_b64 vcc, %12\n\ts_nop 0\n\t" ROCBTA_SEL("%0", "%4", "%8", "0,0,2,2")
+          ROCBTA_SEL("%1", "%5", "%9", "0,0,2,2") ROCBTA_SEL("%2", "%6", "%10", "0,0,2,2")
+              ROCBTA_SEL("%3", "%7", "%11", "0,0,2,2")
+      : "=&v"(a[0]), "=&v"(a[1]), "=&v"(a[2]), "=&v"(a[3])
+      : "v"(y[0]), "v"(y[1]), "v"(y[2]), "v"(y[3]), "v"(x[0]), "v"(x[1]), "v"(x[2]), "v"(x[3]),
+        "s"(even)
+      : "vcc");
+  asm("s_mov_b64 vcc, %8\n\ts_nop 0\n\t" ROCBTA_SEL("%0", "%4", "%0", "1,1,3,3")
+          ROCBTA_SEL("%1", "%5", "%1", "1,1,3,3") ROCBTA_SEL("%2", "%6", "%2", "1,1,3,3")
+              ROCBTA_SEL("%3", "%7", "%3", "1,1,3,3")
+      : "+&v"(y[0]), "+&v"(y[1]), "+&v"(y[2]), "+&v"(y[3])
+      : "v"(x[0]), "v"(x[1]), "v"(x[2]), "v"(x[3]), "s"(~even)
+      : "vcc");
+  x0 = __builtin_bit_cast(double, ((uint64_t)a[1] << 32) | a[0]);
+  x1 = __builtin_bit_cast(double, ((uint64_t)a[3] << 32) | a[2]);
+  y0 = __builtin_bit_cast(double, ((uint64_t)y[1] << 32) | y[0]);
+  y1 = __builtin_bit_cast(double, ((uint64_t)y[3] << 32) | y[2]);
+}
+#undef ROCBTA_SEL
+
+// A group as KC loaded it to the layout of the MFMA steps.
+template <bool KC>
+__device__ __forceinline__ void frag_trade(GFrag& f) {
+  if (!KC) return;
+#pragma unroll
+  for (int i = 0; i < 2; ++i)
+    pair_trade(f.v[i][0], f.v[i][1], f.v[i][2], f.v[i][3]);
+}
+
+// A group in the layout of the MFMA steps, zeros past row r_ok and index k_ok
+// (exclusive).
 template <bool KC>
 __device__ __forceinline__ void frag_load_edge(const double* p, int64_t ld, int k0, int r_ok,
                                                int k_ok, GFrag& f) {
@@ -193,6 +256,8 @@ __device__ __forceinline__ void gemm_wave(const double* A, int64_t lda, const do
 #pragma unroll
       for (int u = 0; u < GPF; ++u) {
         if (g >= full) break;
+        frag_trade<AK>(a[u]);
+        frag_trade<BK>(b[u]);
         frag_mfma(a[u], b[u], acc);
         if (g + GPF * gs < full) {
           frag_load<AK>(sa, kb + (g + GPF * gs) * GK, a[u]);
@@ -222,12 +287,16 @@ __device__ __forceinline__ void gemm_k_range(const GemmTerm& t, int m0, int n0, 
   if (t.triB == TRI_UPPER) kend = min(kend, n0 + GW);
 }
 
-// One term of the wave's block.
+// One term of the wave's block; `at`: groups dealt to the waves before.  Returns
+// whether the wave has one.
 template <typename ACC>
-__device__ __forceinline__ void gemm_term(const GemmTerm& t, int b1, int b2, int M, int N, int m0,
-                                          int n0, int g0, int gs, ACC (&acc)[2][2]) {
+__device__ __forceinline__ bool gemm_term(const GemmTerm& t, int b1, int b2, int M, int N, int m0,
+                                          int n0, int wk, int gs, int& at, ACC (&acc)[2][2]) {
   int kb, ke;
   gemm_k_range(t, m0, n0, kb, ke);
+  const int g0 = (wk - at) & (gs - 1);
+  at += max(ke - kb + GK - 1, 0) / GK;
+  if (kb + g0 * GK >= ke) return false;
   const double* A = t.A + b1 * t.sA1 + b2 * t.sA2 + (t.transA ? m0 : (int64_t)m0 * t.lda);
   const double* B = t.B + b1 * t.sB1 + b2 * t.sB2 + (t.transB ? (int64_t)n0 * t.ldb : n0);
   const int rows = M - m0, cols = N - n0;
@@ -239,43 +308,46 @@ __device__ __forceinline__ void gemm_term(const GemmTerm& t, int b1, int b2, int
     gemm_wave<false, false>(A, t.lda, B, t.ldb, kb, ke, rows, cols, g0, gs, acc);
   else
     gemm_wave<false, true>(A, t.lda, B, t.ldb, kb, ke, rows, cols, g0, gs, acc);
+  return true;
 }
 
-// Sum of the two terms over the wave's share of K, to its LDS block.  The
-// terms' alphas are not applied to the operands: the accumulators hold the
-// sum in units of the last term's alpha (term 0's partial sum is scaled by
-// the quotient when it is complete, exact for the +-1 in use), and the epilogue
-// multiplies by it.  A second term with alpha 0 is skipped.
+// Sum of the two terms over the wave's share of K, to its LDS block: the groups
+// of both are dealt in turn to the gs waves.  The terms' alphas are not applied
+// to the operands: the block holds the sum in units of the last term's alpha
+// (term 0's share is scaled by the quotient r0, exact for the +-1 in use), and the
+// epilogue multiplies by it.  A second term with alpha 0 is skipped.  Each term
+// starts from zero: with the accumulators carried from one to the next the
+// second one's loops spill (four 1024^3 problems of two terms with B transposed:
+// 432 us, 290 so).
 template <typename ACC>
-__device__ __forceinline__ void gemm_wave_block(const GemmProblem& P, bool two, double r0, int b1,
-                                                int b2, int m0, int n0, int g0, int gs, double* part) {
-  const int lane = threadIdx.x & 63;
-  ACC acc[2][2];
+__device__ __forceinline__ void gemm_wave_block(const GemmProblem& P, const GemmTerm& t0,
+                                                const GemmTerm& t1, bool two, double r0, int b1, int b2,
+                                                int m0, int n0, int wk, int gs, double* part) {
+  const bool in = m0 < P.M && n0 < P.N && P.nterms > 0;
+  int at = 0;
+  auto one = [&](const GemmTerm& term, int t) {
+    ACC acc[2][2];
 #pragma unroll
-  for (int i = 0; i < 2; ++i)
+    for (int i = 0; i < 2; ++i)
 #pragma unroll
-    for (int j = 0; j < 2; ++j) acc[i][j] = ACC{0, 0, 0, 0};
-  if (m0 < P.M && n0 < P.N && P.nterms > 0) {
-    gemm_term(P.t[0], b1, b2, P.M, P.N, m0, n0, g0, gs, acc);
-    if (two) {
-      if (r0 != 1.0) {
+      for (int j = 0; j < 2; ++j) acc[i][j] = ACC{0, 0, 0, 0};
+    const bool has = in && gemm_term(term, b1, b2, P.M, P.N, m0, n0, wk, gs, at, acc);
+    if (t && !has) return;
+    const int lane = gemm_lane();
 #pragma unroll
-        for (int i = 0; i < 2; ++i)
+    for (int i = 0; i < 2; ++i)
 #pragma unroll
-          for (int j = 0; j < 2; ++j) acc[i][j] *= r0;
+      for (int r = 0; r < 4; ++r) {
+        dbl2* p = reinterpret_cast<dbl2*>(part + (2 * acc_row(acc[i][0], lane, r) + i) * GP +
+                                          2 * acc_col(lane));
+        dbl2 x;
+        x.x = (double)acc[i][0][r];
+        x.y = (double)acc[i][1][r];
+        *p = t ? *p + x : x * r0;
       }
-      gemm_term(P.t[1], b1, b2, P.M, P.N, m0, n0, g0, gs, acc);
-    }
-  }
-#pragma unroll
-  for (int i = 0; i < 2; ++i)
-#pragma unroll
-    for (int r = 0; r < 4; ++r) {
-      dbl2 x;
-      x.x = (double)acc[i][0][r];
-      x.y = (double)acc[i][1][r];
-      *reinterpret_cast<dbl2*>(part + (2 * acc_row(acc[i][0], lane, r) + i) * GP + 2 * acc_col(lane)) = x;
-    }
+  };
+  one(t0, 0);
+  if (two) one(t1, 1);
 }
 
 // Tile `tile` (global index) of problem P: W x W blocks of 32 x 32, the K
@@ -311,20 +383,26 @@ __device__ __forceinline__ void gemm_tile(const GemmProblem& P, int tile, double
   const int m0 = tm * TS, n0 = tn * TS;
   if (P.uplo == TRI_LOWER && n0 > m0 + TS - 1) return;
   if (P.uplo == TRI_UPPER && m0 > n0 + TS - 1) return;
-  const bool two = P.nterms == 2 && P.t[1].alpha != 0.0;
-  const double a_ref = two ? P.t[1].alpha : P.t[0].alpha;
-  const double r0 = two ? P.t[0].alpha / a_ref : 1.0;
+  // read here, by scalar loads: after the first store (to LDS) they would be vector
+  // loads, a round trip each
+  const GemmTerm t0 = P.t[0], t1 = P.t[1];
+  const int M = P.M, N = P.N, uplo = P.uplo, mirror = P.mirror;
+  const int64_t ldc = P.ldc;
+  const double beta = P.beta;
+  double* const C = P.C + b1 * P.sC1 + b2 * P.sC2;
+  const bool two = P.nterms == 2 && t1.alpha != 0.0;
+  const double a_ref = two ? t1.alpha : t0.alpha;
+  const double r0 = two ? t0.alpha / a_ref : 1.0;
 
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int wk = wave % WK, wb = wave / WK, wm = m0 + GW * (wb / W), wn = n0 + GW * (wb % W);
   if (P.f32)
-    gemm_wave_block<f32x4>(P, two, r0, b1, b2, wm, wn, wk, WK, lds + wave * GW * GP);
+    gemm_wave_block<f32x4>(P, t0, t1, two, r0, b1, b2, wm, wn, wk, WK, lds + wave * GW * GP);
   else
-    gemm_wave_block<f64x4>(P, two, r0, b1, b2, wm, wn, wk, WK, lds + wave * GW * GP);
+    gemm_wave_block<f64x4>(P, t0, t1, two, r0, b1, b2, wm, wn, wk, WK, lds + wave * GW * GP);
   __syncthreads();  // every operand has been read: C may now be written
 
   // thread: two adjacent columns of W * W rows (one per 32 x 32 block)
-  double* C = P.C + b1 * P.sC1 + b2 * P.sC2;
   const int rr = threadIdx.x >> 4, cc = 2 * (threadIdx.x & 15);
 #pragma unroll
   for (int blk = 0; blk < W * W; ++blk) {
@@ -333,27 +411,27 @@ __device__ __forceinline__ void gemm_tile(const GemmProblem& P, int tile, double
 #pragma unroll
     for (int q = 1; q < WK; ++q) s += *reinterpret_cast<const dbl2*>(part + q * GW * GP);
     const int row = m0 + GW * (blk / W) + rr, col = n0 + GW * (blk % W) + cc;
-    double* c = C + (int64_t)row * P.ldc + col;
-    const bool full = row < P.M && col + 1 < P.N && P.uplo == TRI_NONE;
+    double* c = C + (int64_t)row * ldc + col;
+    const bool full = row < M && col + 1 < N && uplo == TRI_NONE;
     s *= a_ref;
     if (full) {
-      if (P.beta != 0.0) s += P.beta * (dbl2)*reinterpret_cast<const dbl2u*>(c);
+      if (beta != 0.0) s += beta * (dbl2)*reinterpret_cast<const dbl2u*>(c);
       *reinterpret_cast<dbl2u*>(c) = s;
     } else {
 #pragma unroll
       for (int e = 0; e < 2; ++e) {
-        if (row >= P.M || col + e >= P.N) continue;
-        if (P.uplo == TRI_LOWER && col + e > row) continue;
-        if (P.uplo == TRI_UPPER && col + e < row) continue;
+        if (row >= M || col + e >= N) continue;
+        if (uplo == TRI_LOWER && col + e > row) continue;
+        if (uplo == TRI_UPPER && col + e < row) continue;
         double v = e ? s.y : s.x;
-        if (P.beta != 0.0) v += P.beta * c[e];
+        if (beta != 0.0) v += beta * c[e];
         c[e] = v;
         if (e) s.y = v; else s.x = v;
       }
     }
-    if (P.mirror) *reinterpret_cast<dbl2*>(part) = s;
+    if (mirror) *reinterpret_cast<dbl2*>(part) = s;
   }
-  if (!P.mirror) return;
+  if (!mirror) return;
   // the transposed entries, read back from LDS so that they are stored by rows
   __syncthreads();
 #pragma unroll
@@ -361,11 +439,11 @@ __device__ __forceinline__ void gemm_tile(const GemmProblem& P, int tile, double
     const double* part = lds + blk * WK * GW * GP;
     // element (cc + e, rr) of the block goes to C[col of it][row of it]
     const int col = n0 + GW * (blk % W) + rr;
-    double* c = C + (int64_t)col * P.ldc;
+    double* c = C + (int64_t)col * ldc;
 #pragma unroll
     for (int e = 0; e < 2; ++e) {
       const int row = m0 + GW * (blk / W) + cc + e;
-      if (row < P.M && col < row) c[row] = part[(cc + e) * GP + rr];
+      if (row < M && col < row) c[row] = part[(cc + e) * GP + rr];
     }
   }
 }

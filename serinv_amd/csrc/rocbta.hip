@@ -86,8 +86,8 @@ GemmTerm term(const double* A, int64_t lda, bool tA, const double* B, int64_t ld
   t.K = K;
   t.transA = tA;
   t.transB = tB;
-  t.triA = (uint8_t)triA;
-  t.triB = (uint8_t)triB;
+  t.triA = triA;
+  t.triB = triB;
   t.alpha = alpha;
   return t;
 }
@@ -140,11 +140,12 @@ int device_cus();  // CUs of the current device (below)
 
 // Width (in 32s) of the output tiles of a launch: 1, with the K range split
 // over the eight waves of a workgroup, or 2, with it split in two.  Wide tiles
-// read each operand half as often from L2: sixteen 1024^3 products take 630
-// instead of 733 us.  A launch of fewer wide tiles than two rounds of
-// the CUs leaves more of them idle than that is worth: 10.7 against 25 us at
-// 512^3, 50 us both at 1024^3 (one wide tile per CU).  In-place problems need
-// the wide ones (aliasing contract of gemm_f64.hpp).
+// read each operand half as often from L2: sixteen 1024^3 products take 551
+// instead of 599 us.  A launch of fewer wide tiles than two rounds of
+// the CUs leaves more of them idle than that is worth: 10.2 against 23 us at
+// 512^3, 46 and 45 us at 1024^3 (one wide tile per CU), 66 against 88 us at
+// 1100^3.  In-place problems need the wide ones (aliasing contract of
+// gemm_f64.hpp).
 template <class V>
 int gemm_width(const V& probs) {
   int64_t wide = 0;
