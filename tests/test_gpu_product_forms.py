@@ -115,3 +115,34 @@ def test_transposed_operands_keep_up(gpu_device):
             best[name] = min(best.get(name, float("inf")), start.elapsed_time(end))
     print(f"ddbtasci permuted n={n} b={b} a={a}: {best}", flush=True)
     assert best["quadratic"] < 4.0 * best["plain"], best
+
+
+def test_ragged_edges_keep_up(gpu_device):
+    """FP32 products at block sizes that are no multiple of the tiles: the selected
+    inversion takes no longer with them than with FP64 ones (0.9 of its time; 1.3
+    where edge blocks waited for each of their loads)."""
+    import torch
+
+    import serinv_amd.algs as algs
+    from serinv_amd.mixed import pobtasi_mixed
+
+    n, b, a = 12, 1100, 32
+    gen = torch.Generator(device=gpu_device).manual_seed(64)
+    rand = lambda *s: torch.rand(s, dtype=torch.float64, device=gpu_device, generator=gen)  # noqa: E731
+    D, T = rand(n, b, b), rand(a, a)
+    D.diagonal(dim1=1, dim2=2).add_(3 * b + a)
+    T.diagonal().add_(n * b + a)
+    F = [D, rand(n - 1, b, b), rand(n, a, b), T]
+    algs.pobtaf(*F)
+    start, end = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+    best = {}
+    for _ in range(6):
+        for fn in (algs.pobtasi, pobtasi_mixed):
+            F1 = [x.clone() for x in F]
+            start.record()
+            fn(*F1)
+            end.record()
+            end.synchronize()
+            best[fn.__name__] = min(best.get(fn.__name__, float("inf")), start.elapsed_time(end))
+    print(f"selected inversion n={n} b={b} a={a}: {best}", flush=True)
+    assert best["pobtasi_mixed"] < 1.08 * best["pobtasi"], best
