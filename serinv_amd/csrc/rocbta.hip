@@ -746,8 +746,10 @@ constexpr int WD_FEW_B = 512;
 // The wide sweep: full solves with b a multiple of its 16-row tiles.
 bool wd_fits(int64_t b, int partial) { return !partial && b >= WD_CW && b % WD_T == 0; }
 
-int pobtas_algo(int64_t n, int64_t b, int64_t a, int64_t r, int partial) {
-  const char* e = getenv("ROCBTA_POBTAS_ALGO");
+const char* pobtas_forced() { return getenv("ROCBTA_POBTAS_ALGO"); }
+
+// e: pobtas_forced()
+int pobtas_algo(const char* e, int64_t n, int64_t b, int64_t a, int64_t r, int partial) {
   if (e && strcmp(e, "loop") == 0) return SOLVE_LOOP;
   if (e && strcmp(e, "wide") == 0)
     return wd_fits(b, partial) ? SOLVE_WIDE : (partial ? SOLVE_LOOP : SOLVE_SWEEP);
@@ -861,6 +863,12 @@ int pobtas_sweep(int64_t n, int64_t b, int64_t a, const double* D, const double*
   return ROCBTA_OK;
 }
 
+// A workgroup per row group and the rows of a phase in registers: the form
+// that loads a phase ahead and needs no transposes.
+bool bs_reg(int64_t b) {
+  return cdiv(b, bs_rw(1, 0)) <= std::min(BS_MAX_G, device_cus()) && b <= BS_KU * BS_THREADS;
+}
+
 struct BsLayout {
   size_t status, linv, lt, w, tinv, wt, sbuf, tbuf, tpart, tipbuf, total;
   int cw;
@@ -878,7 +886,8 @@ BsLayout bs_layout(int64_t n, int64_t b, int64_t a, int64_t r) {
   const int64_t ntb = (b + TT - 1) / TT, nta = (a + TT - 1) / TT;
   l.status = take(sizeof(int));
   l.linv = take((size_t)n * b * b * sizeof(double));
-  l.lt = take((size_t)std::max<int64_t>(n - 1, 1) * b * b * sizeof(double));  // backward: L^T
+  // the streamed backward sweep's L^T
+  l.lt = take(bs_reg(b) ? 0 : (size_t)std::max<int64_t>(n - 1, 1) * b * b * sizeof(double));
   // trtri scratch: 64-wide levels need ntb * 64^2 per block, halving b^2 / 4
   l.w = take((size_t)n * std::max<int64_t>(ntb * TT * TT, ntb * TT * ntb * TT / 4) * sizeof(double));
   l.tinv = take((size_t)a * a * sizeof(double));
@@ -889,12 +898,6 @@ BsLayout bs_layout(int64_t n, int64_t b, int64_t a, int64_t r) {
   l.tipbuf = take((size_t)a * l.cw * sizeof(double));
   l.total = off;
   return l;
-}
-
-// A workgroup per row group and the rows of a phase in registers: the form
-// that loads a phase ahead and needs no transposes.
-bool bs_reg(int64_t b) {
-  return cdiv(b, bs_rw(1, 0)) <= std::min(BS_MAX_G, device_cus()) && b <= BS_KU * BS_THREADS;
 }
 
 template <int CW>
@@ -1338,12 +1341,20 @@ size_t rocbta_workspace_bytes(int op, int64_t n, int64_t b, int64_t a, int64_t r
     case ROCBTA_OP_POBTASI:
       return si_layout(n, b, a).total;
     case ROCBTA_OP_POBTAS: {
-      // enough for the algorithm the shape selects (partial or not)
+      // Enough for the algorithms that the shape selects, partial or not, with this
+      // many columns and with fewer, which select others: one workspace serves a
+      // caller's widest right-hand side and its parts (of blocks from BS_MIN_B on,
+      // whose inverses the widest may do without, up to BS_MAX_R columns).
       const int64_t rr = std::max<int64_t>(r, 1);
       size_t need = sw_layout(n, b, a, rr).total;
-      if (pobtas_algo(n, b, a, rr, 0) == SOLVE_BLOCK || pobtas_algo(n, b, a, rr, 1) == SOLVE_BLOCK)
-        need = std::max(need, bs_layout(n, b, a, rr).total);
-      if (pobtas_algo(n, b, a, rr, 0) == SOLVE_WIDE) need = std::max(need, wd_layout(n, b, a).total);
+      const char* const forced = pobtas_forced();
+      for (const int64_t q : {(int64_t)1, (int64_t)4, (int64_t)BS_MAX_R, rr}) {
+        if (q > rr || (q < rr && rr > BS_MAX_R && b >= BS_MIN_B)) continue;
+        const int full = pobtas_algo(forced, n, b, a, q, 0);
+        if (full == SOLVE_BLOCK || pobtas_algo(forced, n, b, a, q, 1) == SOLVE_BLOCK)
+          need = std::max(need, bs_layout(n, b, a, q).total);
+        if (full == SOLVE_WIDE) need = std::max(need, wd_layout(n, b, a).total);
+      }
       return need;
     }
     case ROCBTA_OP_LOGDET:
@@ -1698,7 +1709,7 @@ int rocbta_dpobtas(int64_t n, int64_t b, int64_t a, const double* D, const doubl
   if (trans != 'N' && trans != 'T' && trans != 'C') return ROCBTA_ERR_ARG;
   if (r == 0) return ROCBTA_OK;
   hipStream_t s = (hipStream_t)stream;
-  const int algo = pobtas_algo(n, b, a, r, partial);
+  const int algo = pobtas_algo(pobtas_forced(), n, b, a, r, partial);
   if (algo == SOLVE_BLOCK) {
     if (!workspace || workspace_bytes < bs_layout(n, b, a, r).total) return ROCBTA_ERR_WORKSPACE;
     return pobtas_block(n, b, a, D, L, R, T, B, r, ldb, trans == 'N' ? 0 : 1, partial,
