@@ -346,7 +346,7 @@ int rocbta_batched_create(int nmat, const int64_t* n, const int64_t* b, const in
     chains[m] = chain_params(n[m], b[m], a[m], D[m], L[m], R[m], T[m], p->d_info + m, ws, q.lay);
     chains[m].tip_inv = a[m] > 0 ? (double*)(base + q.tipinv) : nullptr;
     zero.push_back({(double*)(ws + q.lay.counter),
-                    (int64_t)((q.lay.linv - q.lay.counter) / sizeof(double)), 0.0});
+                    (int64_t)((q.lay.flags_end - q.lay.counter) / sizeof(double)), 0.0});
     lds[m] = {D[m], a[m] > 0 ? T[m] : nullptr, n[m], b[m], a[m], p->d_logdet_out + m};
     if (solve) {
       SweepP P{};

@@ -501,7 +501,7 @@ SiLayout si_layout(int64_t n, int64_t b, int64_t a) {
 }
 
 struct AfLayout {
-  size_t tinv, counter, claim, chain_cu, hflags, cflags, linv, tipp, save_d, save_r, save_t, total;
+  size_t tinv, counter, claim, chain_cu, hflags, cflags, flags_end, linv, tipp, save_d, save_r, save_t, total;
   int nt, na, NT, slots, nstages, ntasks;
 };
 
@@ -519,14 +519,23 @@ AfLayout af_layout(int64_t n, int64_t b, int64_t a) {
     off = align256(off + bytes);
     return o;
   };
+  const size_t tipp_bytes = (size_t)n * a * a * sizeof(double);
   l.tinv = take(TT * TT * sizeof(double));
   l.counter = take(sizeof(int));
   l.claim = take(sizeof(int));
   l.chain_cu = take(sizeof(int));
   l.hflags = take((size_t)l.ntasks * sizeof(int));
   l.cflags = take((size_t)2 * l.NT * sizeof(int));
-  l.linv = take((size_t)l.NT * CT * CT * sizeof(double));
-  l.tipp = take((size_t)n * a * a * sizeof(double));
+  l.flags_end = off;
+  if (l.na > 1) {
+    // the tip products of wide arrows are formed after the launch, over its flags
+    l.tipp = l.counter;
+    off = std::max(off, align256(l.tipp + tipp_bytes));
+    l.linv = take((size_t)l.NT * CT * CT * sizeof(double));
+  } else {
+    l.linv = take((size_t)l.NT * CT * CT * sizeof(double));
+    l.tipp = take(tipp_bytes);
+  }
   // factorize_last_block = 0 on the chain: the last block, its arrow block
   // and the tip as given
   l.save_d = take((size_t)b * b * sizeof(double));
@@ -629,7 +638,7 @@ long long* chain_trace_buffer(size_t count) {
 int pobtaf_chain(int64_t n, int64_t b, int64_t a, double* D, double* L, double* R, double* T,
                  int* info, char* ws, const AfLayout& lay, hipStream_t s) {
   PobtafChain P = chain_params(n, b, a, D, L, R, T, info, ws, lay);
-  const int64_t nflag = (int64_t)((lay.linv - lay.counter) / sizeof(int));
+  const int64_t nflag = (int64_t)((lay.flags_end - lay.counter) / sizeof(int));
   fill_i32_kernel<<<(int)std::min<int64_t>(1024, (nflag + 255) / 256), 256, 0, s>>>(P.counter, nflag, 0);
   RB_CHECK(hipGetLastError());
   const char* trace_path = getenv("ROCBTA_CHAIN_TRACE");
