@@ -130,6 +130,8 @@ thread_local Recorder* g_rec = nullptr;
 // Set for the duration of a mixed-precision entry point: every GEMM problem
 // and the persistent factorization run their products in FP32.
 thread_local bool g_mixed = false;
+// GemmProblem::f32 of a problem that stays FP64 there.
+constexpr int GEMM_FP64 = -1;
 struct MixedScope {
   bool prev;
   explicit MixedScope(bool on) : prev(g_mixed) { g_mixed = on; }
@@ -175,7 +177,7 @@ int run_gemms(GemmList& list, hipStream_t s) {
     for (GemmProblem p : list.probs) {
       if (p.M <= 0 || p.N <= 0 || p.batch1 <= 0 || p.batch2 <= 0) continue;
       if (p.nterms == 0 && p.beta == 1.0) continue;
-      p.f32 = g_mixed ? 1 : 0;
+      p.f32 = g_mixed && p.f32 != GEMM_FP64 ? 1 : 0;
       ph.gemms.push_back(p);
     }
     return ROCBTA_OK;
@@ -197,7 +199,7 @@ int run_gemms(GemmList& list, hipStream_t s) {
   for (GemmProblem p : list.probs) {
     if (p.M <= 0 || p.N <= 0 || p.batch1 <= 0 || p.batch2 <= 0) continue;
     if (p.nterms == 0 && p.beta == 1.0) continue;
-    p.f32 = g_mixed ? 1 : 0;
+    p.f32 = g_mixed && p.f32 != GEMM_FP64 ? 1 : 0;
     const int64_t tiles = gemm_set_tiles(p, width);
     if (g.nprob == ROCBTA_MAX_PROBLEMS || (int64_t)g.total_tiles + tiles > (1ll << 30)) {
       int rc = flush();
@@ -1406,12 +1408,18 @@ int rocbta_dpobtaf(int64_t n, int64_t b, int64_t a, double* D, double* L, double
   const int bi = (int)b, ai = (int)a;
   const int64_t bb = b * b, ab = a * b;
   if (!factorize_last_block && n == 1) return ROCBTA_OK;  // no block row to eliminate
+  // The tip is FP64 in the mixed form too.
+  auto factor_tip = [&]() -> int {
+    MixedScope fp64(false);
+    return factor_block_column(T, a, ai, {}, n * b, info, tinv, s);
+  };
   if (pobtaf_use_chain()) {
     char* ws = (char*)workspace;
     // Arrows of more than one tile: the launch leaves the tip alone and
     // T - sum_{i < nblk} L_{t,i} L_{t,i}^T takes one batched product after it.
     double* tipp = (double*)(ws + lay.tipp);
     auto tip_products = [&](int64_t nblk) -> int {
+      MixedScope fp64(false);  // as inside the launch
       GemmList pr;
       push_term(pr.add(tipp, a, ai, ai, 0.0, TRI_LOWER, (int)nblk, a * a),
                 term(R, b, false, R, b, true, bi, 1.0, TRI_NONE, TRI_NONE, ab, ab));
@@ -1423,7 +1431,7 @@ int rocbta_dpobtaf(int64_t n, int64_t b, int64_t a, double* D, double* L, double
       if ((rc = tip_products(n))) return rc;
       tip_open_kernel<<<cdiv(a * a, 256), 256, 0, s>>>(T, T, tipp, ai, (int)n);
       RB_CHECK(hipGetLastError());
-      return factor_block_column(T, a, ai, {}, n * b, info, tinv, s);
+      return factor_tip();
     }
     // pobtaf.py:143-159 leaves D_{n-1}, R_{n-1} and T Schur-updated but not
     // factored.  The chain factors them too; they are rebuilt afterwards
@@ -1475,7 +1483,9 @@ int rocbta_dpobtaf(int64_t n, int64_t b, int64_t a, double* D, double* L, double
     if (a > 0) {
       push_term(upd.add(R + (i + 1) * ab, b, ai, bi, 1.0),
                 term(R + i * ab, b, false, Li, b, true, bi, -1.0));
-      push_term(upd.add(T, a, ai, ai, 1.0), term(R + i * ab, b, false, R + i * ab, b, true, bi, -1.0));
+      GemmProblem& tip = upd.add(T, a, ai, ai, 1.0);
+      tip.f32 = GEMM_FP64;
+      push_term(tip, term(R + i * ab, b, false, R + i * ab, b, true, bi, -1.0));
     }
     rc = run_gemms(upd, s);
     if (rc) return rc;
@@ -1489,10 +1499,12 @@ int rocbta_dpobtaf(int64_t n, int64_t b, int64_t a, double* D, double* L, double
     if (a > 0) {
       GemmList upd;
       const double* Rl = R + (n - 1) * ab;
-      push_term(upd.add(T, a, ai, ai, 1.0), term(Rl, b, false, Rl, b, true, bi, -1.0));
+      GemmProblem& tip = upd.add(T, a, ai, ai, 1.0);
+      tip.f32 = GEMM_FP64;
+      push_term(tip, term(Rl, b, false, Rl, b, true, bi, -1.0));
       rc = run_gemms(upd, s);
       if (rc) return rc;
-      rc = factor_block_column(T, a, ai, {}, n * b, info, tinv, s);
+      rc = factor_tip();
       if (rc) return rc;
     }
   }
