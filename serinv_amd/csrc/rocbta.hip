@@ -566,6 +566,13 @@ bool pobtaf_use_chain() {
   const char* e = getenv("ROCBTA_POBTAF_ALGO");
   return !(e && strcmp(e, "loop") == 0);
 }
+// With the last block left open the chain's steps of that block are done for
+// nothing and the block is rebuilt afterwards; under an arrow of more than one
+// tile the tip too takes launches of its own.  That many tile columns go launch
+// by launch.  Measured, launches / chain in us, a = 100: n=2 b=16 34 / 69, n=2 b=64
+// 46 / 76, n=2 b=128 82 / 102, n=3 b=64 78 / 88; n=4 b=64 108 / 99, n=3 b=128 (four
+// columns) 147 / 128.
+constexpr int64_t OPEN_LOOP_COLS = 2;
 
 // info = 0 where it names a row of the last block or of the tip (rows past
 // `first_open`), which factorize_last_block = 0 leaves unfactored.
@@ -1413,7 +1420,8 @@ int rocbta_dpobtaf(int64_t n, int64_t b, int64_t a, double* D, double* L, double
     MixedScope fp64(false);
     return factor_block_column(T, a, ai, {}, n * b, info, tinv, s);
   };
-  if (pobtaf_use_chain()) {
+  const bool few = !factorize_last_block && lay.na > 1 && (n - 1) * lay.nt <= OPEN_LOOP_COLS;
+  if (!few && pobtaf_use_chain()) {
     char* ws = (char*)workspace;
     // Arrows of more than one tile: the launch leaves the tip alone and
     // T - sum_{i < nblk} L_{t,i} L_{t,i}^T takes one batched product after it.
