@@ -730,57 +730,79 @@ __global__ void fill_u64_kernel(unsigned long long* p, int64_t count, unsigned l
 // Solve algorithm: the block-level sweep (precomputed diagonal-block
 // inverses, two dependent device-wide products per block row) for few
 // right-hand sides, its wide form (64 columns per launch, MFMA tiles) for
-// more, the 64-row-tile sweep for small blocks and what the others do not fit,
-// the launch-per-tile form for partial solves there.  Measured, N + C in us:
-//                        block  wide  tiles
-//   n=8   b=96   r=2       236   224    272
-//   n=64  b=130  r=1 / 4 / 8    688 / 931 / 1358 block, 1762 / 1988 / 2715 tiles
-//   n=64  b=128  r=4       871   772   1331
-//   n=64  b=256  r=1       723   904
-//   n=64  b=256  r=4 / 8   985 / 1423 block, 907 / 908 wide, 3571 tiles (r=8)
-//   n=64  b=1024 r=4 / 8  3209 / 4195 block, 3399 / 3403 wide
-//   n=32  b=64   r=1       316          340
-//   n=64  b=64   r=4       787   603    678
-//   n=32  b=48   r=4       446          396
+// more, the 64-row-tile sweep for small problems and what the others do not fit,
+// the launch-per-tile form for small partial solves.
 // ROCBTA_POBTAS_ALGO = block | wide | sweep | loop forces one (tests cover
 // all four; block and wide fall back when the shape does not fit them).
 enum SolveAlgo { SOLVE_LOOP = 0, SOLVE_SWEEP = 1, SOLVE_BLOCK = 2, SOLVE_WIDE = 3 };
-// The block and wide sweeps need their inverses' launches first (about 40 us
-// a call): they are taken from this many tile steps saved on, for blocks of one
-// full tile from BS_MIN_N block rows on.
-constexpr int BS_MIN_SAVED = 8;
-constexpr int BS_MIN_N = 32;
-constexpr int BS_MIN_B = 256;   // and for these blocks always
+constexpr int BS_MIN_B = 256;   // blocks whose inverses pay for any number of rows
 constexpr int BS_MAX_G = 1024;  // workgroups of the block sweep (tip partial sums sized for it)
+constexpr int BS_MAX_R = 8;     // columns: the block sweep reads the factor once per group of them
+constexpr int WD_FEW_B = 256;   // 2 to 4 columns take the wide sweep up to this block size
 
 int bs_cw(int64_t r) { return r <= 1 ? 1 : (r <= 4 ? 4 : 8); }
 bool bs_fits(int64_t a, int64_t r) { return a * bs_cw(r) <= BS_TIPMAX; }
-// The block sweep re-reads the factor once per group of columns, so it serves 5
-// to 8 of them only where the wide one does not fit; from b = 513 on the wide
-// sweep's MFMA time makes it the slower one up to 4 columns.
-constexpr int BS_MAX_R = 8;
-constexpr int WD_FEW_B = 512;
 
 // The wide sweep: full solves with b a multiple of its 16-row tiles.
 bool wd_fits(int64_t b, int partial) { return !partial && b >= WD_CW && b % WD_T == 0; }
+
+// Lines between the sweeps, for blocks of nt tiles, n of them, and arrows of na
+// tiles.  A tile step of the 64-row-tile sweep costs 8.6 us, N + C, with one
+// column (10 with 4, 13 with 8), a block row of the block sweep 7.6 (11), of the
+// wide one 8 to 9 us; the inverses cost launches, more of them for more tiles of a
+// block and of the tip.  Measured, N + C in us, tiles / block / wide:
+//   one column  n=3 b=65  a=8    117 / 108         n=2 b=130 a=8    117 / 136
+//               n=3 b=130 a=8    145 / 138         n=3 b=200 a=8    178 / 169
+//               n=4 b=65  a=70   166 / 172         n=6 b=65  a=70   198 / 188
+//               n=5 b=130 a=130  234 / 249         n=6 b=130 a=130  254 / 251
+//               n=16 b=65 a=300  423 / 434         n=24 b=65 a=300  566 / 500
+//               n=10 b=130 a=300 400 / 432         n=12 b=130 a=300 458 / 444
+//               n=8 b=64  a=64   131 / 133         n=12 b=64 a=64   166 / 160
+//               n=16 b=64 a=70   210 / 213         n=40 b=64 a=70   395 / 366
+//   4 columns   n=6 b=96  a=8    198 / 168 / 176   n=10 b=96 a=8    277 / 216 / 206
+//               n=4 b=256 a=8    218 / 160 / 170   n=128 b=256 a=8  - / 1682 / 1599
+//               n=128 b=320 a=8  - / 1927 / 1943   n=64 b=512 a=8   - / 1227 / 1312
+//               n=5 b=96  a=300  272 / - / 293     n=8 b=96  a=300  334 / - / 320
+//               n=3 b=256 a=300  275 / - / 287     n=4 b=256 a=300  311 / - / 300
+//               n=12 b=64 a=64   181 / - / 183     n=16 b=64 a=64   219 / - / 213
+//   16 columns  n=2 b=64  a=8    92 / - / 89       n=2 b=96  a=130  186 / - / 194
+//               n=3 b=128 a=70   178 / - / 166     n=4 b=96  a=300  305 / - / 299
+//   partial, one column, launches / block
+//               n=3 b=65  a=8    119 / 117         n=2 b=130 a=8    102 / 123
+//               n=2 b=64  a=8    61 / 76           n=4 b=64  a=8    119 / 84
+bool bs_pays(int64_t n, int64_t nt, int64_t na, int64_t r) {
+  if (nt == 1) return r <= 1 && n >= 10 * na * na;
+  return n >= 3 && 3 * (n - 3) * (nt - 1) >= 2 * (na * na - 1);
+}
+bool wd_pays(int64_t n, int64_t nt, int64_t na, int64_t r) {
+  if (r > 4) return n >= 2 && (n - 2) * nt >= na - 1;
+  if (nt == 1) return r > 1 && n >= 12 + 4 * na;
+  return n >= (r > 1 ? 1 : 2) * (4 + (na + 1) / (2 * (nt - 1)));
+}
 
 const char* pobtas_forced() { return getenv("ROCBTA_POBTAS_ALGO"); }
 
 // e: pobtas_forced()
 int pobtas_algo(const char* e, int64_t n, int64_t b, int64_t a, int64_t r, int partial) {
+  const bool block = bs_fits(a, r), wide = wd_fits(b, partial);
+  const int other = partial ? SOLVE_LOOP : SOLVE_SWEEP;
   if (e && strcmp(e, "loop") == 0) return SOLVE_LOOP;
-  if (e && strcmp(e, "wide") == 0)
-    return wd_fits(b, partial) ? SOLVE_WIDE : (partial ? SOLVE_LOOP : SOLVE_SWEEP);
-  if (e && strcmp(e, "sweep") == 0) return partial ? SOLVE_LOOP : SOLVE_SWEEP;
-  if (e && strcmp(e, "block") == 0) return bs_fits(a, r) ? SOLVE_BLOCK : (partial ? SOLVE_LOOP : SOLVE_SWEEP);
-  if (b > SW_T ? (b >= BS_MIN_B || n * (cdiv(b, SW_T) - 1) >= BS_MIN_SAVED)
-               : (b == SW_T && n >= BS_MIN_N)) {
-    const bool wide = wd_fits(b, partial);
-    if (wide && r > (b <= WD_FEW_B ? 1 : 4)) return SOLVE_WIDE;
-    if (r <= (b > SW_T ? BS_MAX_R : 1) && bs_fits(a, r)) return SOLVE_BLOCK;
-    if (wide) return SOLVE_WIDE;
+  if (e && strcmp(e, "wide") == 0) return wide ? SOLVE_WIDE : other;
+  if (e && strcmp(e, "sweep") == 0) return other;
+  if (e && strcmp(e, "block") == 0) return block ? SOLVE_BLOCK : other;
+  const int64_t nt = cdiv(b, SW_T), na = std::max(1, cdiv(a, SW_T));
+  const bool big = b >= BS_MIN_B;
+  if (b < SW_T) return other;
+  if (partial) {  // no tip inverse
+    const bool pays = nt > 1 ? n >= 3 && n * (nt - 1) >= 4 : n >= 4 && r <= 4;
+    return block && r <= BS_MAX_R && (big || pays) ? SOLVE_BLOCK : SOLVE_LOOP;
   }
-  return partial ? SOLVE_LOOP : SOLVE_SWEEP;
+  if (wide && r > 4 && ((big && r > BS_MAX_R) || wd_pays(n, nt, na, r))) return SOLVE_WIDE;
+  if (block && r <= BS_MAX_R && (big || bs_pays(n, nt, na, r))) {
+    const bool few = r > 1 && b <= WD_FEW_B && n * na >= 8 * (nt - 1);
+    return wide && few && wd_pays(n, nt, na, r) ? SOLVE_WIDE : SOLVE_BLOCK;
+  }
+  return wide && wd_pays(n, nt, na, r) ? SOLVE_WIDE : SOLVE_SWEEP;
 }
 
 // Inverses of the diagonal tiles of an m_total x m_total lower-triangular
@@ -952,7 +974,7 @@ int pobtas_block(int64_t n, int64_t b, int64_t a, const double* D, const double*
   int rc = block_trtri(D, b, b * b, Linv, b, b * b, (int)b, (int)n, (double*)(ws + lay.w), s, true,
                        false);
   if (rc) return rc;
-  if (a > 0) {
+  if (a > 0 && !partial) {
     rc = block_trtri(T, a, 0, Tinv, a, a * a, (int)a, 1, (double*)(ws + lay.wt), s);
     if (rc) return rc;
   }
@@ -1369,7 +1391,9 @@ size_t rocbta_workspace_bytes(int op, int64_t n, int64_t b, int64_t a, int64_t r
       for (const int64_t q : {(int64_t)1, (int64_t)4, (int64_t)BS_MAX_R, rr}) {
         if (q > rr || (q < rr && rr > BS_MAX_R && b >= BS_MIN_B)) continue;
         const int full = pobtas_algo(forced, n, b, a, q, 0);
-        if (full == SOLVE_BLOCK || pobtas_algo(forced, n, b, a, q, 1) == SOLVE_BLOCK)
+        // (where the wide sweep runs, fewer rows may select the block sweep)
+        if (full == SOLVE_BLOCK || pobtas_algo(forced, n, b, a, q, 1) == SOLVE_BLOCK ||
+            (full == SOLVE_WIDE && q <= BS_MAX_R && bs_fits(a, q) && bs_reg(b)))
           need = std::max(need, bs_layout(n, b, a, q).total);
         if (full == SOLVE_WIDE) need = std::max(need, wd_layout(n, b, a).total);
       }
