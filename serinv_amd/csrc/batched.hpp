@@ -442,7 +442,7 @@ int rocbta_batched_create(int nmat, const int64_t* n, const int64_t* b, const in
     pl.tile_grid = grid;
     if (pl.ntile) pl.tile_off = dtake(ph.tiles.size() * sizeof(TileBatch));
     int64_t tiles = 0;
-    pl.gemm_width = p->gemm512 ? 1 : gemm_width(ph.gemms);
+    pl.gemm_width = p->gemm512 && !gemm_in_place(ph.gemms) ? 1 : gemm_width(ph.gemms);
     for (GemmProblem& g : ph.gemms) {
       g.tile_begin = (int)tiles;
       tiles += gemm_set_tiles(g, pl.gemm_width);

@@ -149,11 +149,17 @@ int device_cus();  // CUs of the current device (below)
 // 1100^3.  In-place problems need the wide ones (aliasing contract of
 // gemm_f64.hpp).
 template <class V>
+bool gemm_in_place(const V& probs) {
+  for (const GemmProblem& p : probs)
+    for (int t = 0; t < p.nterms; ++t)
+      if (p.t[t].A == p.C || p.t[t].B == p.C) return true;
+  return false;
+}
+template <class V>
 int gemm_width(const V& probs) {
+  if (gemm_in_place(probs)) return 2;
   int64_t wide = 0;
   for (const GemmProblem& p : probs) {
-    for (int t = 0; t < p.nterms; ++t)
-      if (p.t[t].A == p.C || p.t[t].B == p.C) return 2;
     const int64_t tm = cdiv(p.M, 2 * GW), tn = cdiv(p.N, 2 * GW);
     wide += (p.uplo == TRI_NONE ? tm * tn : tm * (tn + 1) / 2) * p.batch1 * p.batch2;
   }
@@ -906,7 +912,7 @@ int pobtas_sweep(int64_t n, int64_t b, int64_t a, const double* D, const double*
 // A workgroup per row group and the rows of a phase in registers: the form
 // that loads a phase ahead and needs no transposes.
 bool bs_reg(int64_t b) {
-  return cdiv(b, bs_rw(1, 0)) <= std::min(BS_MAX_G, device_cus()) && b <= BS_KU * BS_THREADS;
+  return cdiv(b, BS_RW) <= std::min(BS_MAX_G, device_cus()) && b <= BS_KU * BS_THREADS;
 }
 
 struct BsLayout {
@@ -942,8 +948,7 @@ BsLayout bs_layout(int64_t n, int64_t b, int64_t a, int64_t r) {
 
 template <int CW>
 int launch_block_sweep(BlockSweepP P, hipStream_t s) {
-  const int rw = bs_rw(CW, P.trans);
-  P.G = std::min(std::min(cdiv(P.b, rw), BS_MAX_G), device_cus());
+  P.G = std::min(std::min(cdiv(P.b, BS_RW), BS_MAX_G), device_cus());
   const bool reg = bs_reg(P.b);
   if (reg && P.trans == 0)
     pobtas_block_reg_kernel<CW, 0><<<P.G, BS_THREADS, 0, s>>>(P);

@@ -43,9 +43,7 @@
 namespace rocbta {
 
 constexpr int BS_THREADS = 256;
-// Rows per row group (RW * CW partial sums per thread): four in both
-// directions.
-__host__ __device__ constexpr int bs_rw(int cw, int trans) { return 4 + 0 * cw * trans; }
+constexpr int BS_RW = 4;  // rows per row group (BS_RW * CW partial sums per thread)
 
 // Transposes of nb square b x b blocks, 64 x 64 tiles through LDS (pitch 65,
 // so that the column reads do not share banks).  Out of place: block z of
@@ -174,15 +172,14 @@ struct BsLds {
   double rv[BS_TIPMAX * RW];  // backward: R_i[m][k0 + q] at m * RW + q (a <= BS_TIPMAX)
 };
 
-// Rows of block i (k0 .. k0 + RW - 1) times the solution block `src`
-// (forward: M[k][j] row access, backward: M[j][k] column access), K range
+// Rows of block i (k0 .. k0 + RW - 1) times the solution block `src`, K range
 // [jlo, jhi), into acc[q][c].  src rows are polled from the buffer: a thread
 // first issues the matrix loads and the polled loads of BS_KU reduction
 // indices together, then re-polls only the values still marked empty, so
 // one round trip covers all of them.
 constexpr int BS_KU = 4;
 
-template <int CW, int RW, bool TR>
+template <int CW, int RW>
 __device__ __forceinline__ void bs_product(const BlockSweepP& P, const double* M, int k0,
                                            const double* src, int jlo, int jhi,
                                            double (&acc)[RW][CW]) {
@@ -196,7 +193,7 @@ __device__ __forceinline__ void bs_product(const BlockSweepP& P, const double* M
 #pragma unroll
       for (int q = 0; q < RW; ++q) {
         const int k = k0 + q;
-        m[u][q] = (j < jhi && k < b) ? (TR ? M[(int64_t)j * b + k] : M[(int64_t)k * b + j]) : 0.0;
+        m[u][q] = (j < jhi && k < b) ? M[(int64_t)k * b + j] : 0.0;
       }
     }
 #pragma unroll
@@ -336,7 +333,7 @@ __device__ __forceinline__ void bs_tip_back(const BlockSweepP& P, double* xt) {
 
 template <int CW, int TRANS>
 __global__ void __launch_bounds__(BS_THREADS) pobtas_block_kernel(BlockSweepP P) {
-  constexpr int RW = bs_rw(CW, TRANS);
+  constexpr int RW = BS_RW;
   __shared__ BsLds<CW, RW> S;
   const int tid = threadIdx.x;
   const int b = P.b, n = P.n, a = P.a;
@@ -354,7 +351,7 @@ __global__ void __launch_bounds__(BS_THREADS) pobtas_block_kernel(BlockSweepP P)
         // phase A: t = b_i - L_{i,i-1} y_{i-1}
         bs_zero(acc);
         if (i > 0)
-          bs_product<CW, RW, false>(P, P.L + (int64_t)(i - 1) * b * b, k0,
+          bs_product<CW, RW>(P, P.L + (int64_t)(i - 1) * b * b, k0,
                                 P.sbuf + (int64_t)(i - 1) * b * CW, 0, b, acc);
         double flat[RW * CW];
 #pragma unroll
@@ -377,7 +374,7 @@ __global__ void __launch_bounds__(BS_THREADS) pobtas_block_kernel(BlockSweepP P)
         const int k0 = g * RW;
         // phase B: y = Linv_i t (t rows 0 .. k0 + RW - 1)
         bs_zero(acc);
-        bs_product<CW, RW, false>(P, P.Linv + (int64_t)i * b * b, k0, P.tbuf + (int64_t)i * b * CW, 0,
+        bs_product<CW, RW>(P, P.Linv + (int64_t)i * b * b, k0, P.tbuf + (int64_t)i * b * CW, 0,
                               min(b, k0 + RW), acc);
         double flat[RW * CW];
 #pragma unroll
@@ -439,7 +436,7 @@ __global__ void __launch_bounds__(BS_THREADS) pobtas_block_kernel(BlockSweepP P)
       }
       bs_zero(acc);
       if (i + 1 < n)
-        bs_product<CW, RW, false>(P, P.L + (int64_t)i * b * b, k0, P.sbuf + (int64_t)(i + 1) * b * CW,
+        bs_product<CW, RW>(P, P.L + (int64_t)i * b * b, k0, P.sbuf + (int64_t)(i + 1) * b * CW,
                               0, b, acc);
       double flat[RW * CW];
 #pragma unroll
@@ -465,7 +462,7 @@ __global__ void __launch_bounds__(BS_THREADS) pobtas_block_kernel(BlockSweepP P)
       const int k0 = g * RW;
       // phase B: x = Linv_i^T s (s rows k0 .. b - 1)
       bs_zero(acc);
-      bs_product<CW, RW, false>(P, P.Linv + (int64_t)i * b * b, k0, P.tbuf + (int64_t)i * b * CW, k0,
+      bs_product<CW, RW>(P, P.Linv + (int64_t)i * b * b, k0, P.tbuf + (int64_t)i * b * CW, k0,
                             b, acc);
       double flat[RW * CW];
 #pragma unroll
@@ -540,7 +537,7 @@ typedef double bsdbl2u __attribute__((ext_vector_type(2), aligned(8)));  // any 
 
 template <int CW, int TRANS>
 __global__ void __launch_bounds__(BS_THREADS) pobtas_block_reg_kernel(BlockSweepP P) {
-  constexpr int RW = bs_rw(CW, TRANS), NV = RW * CW, TU = BS_TIPMAX / BS_THREADS;
+  constexpr int RW = BS_RW, NV = RW * CW, TU = BS_TIPMAX / BS_THREADS;
   __shared__ double red[2][4 * NV];
   __shared__ double ysh[NV];
   __shared__ double xt[BS_TIPMAX];
