@@ -1767,7 +1767,14 @@ int rocbta_dpobtas(int64_t n, int64_t b, int64_t a, const double* D, const doubl
   if (trans != 'N' && trans != 'T' && trans != 'C') return ROCBTA_ERR_ARG;
   if (r == 0) return ROCBTA_OK;
   hipStream_t s = (hipStream_t)stream;
-  const int algo = pobtas_algo(pobtas_forced(), n, b, a, r, partial);
+  const char* const forced = pobtas_forced();
+  int algo = pobtas_algo(forced, n, b, a, r, partial);
+  // below BS_MIN_B a smaller workspace, or for partial solves none, is enough for
+  // the forms that take over from the block and wide sweeps there
+  if (!forced && b < BS_MIN_B && (algo == SOLVE_BLOCK || algo == SOLVE_WIDE)) {
+    const size_t need = algo == SOLVE_BLOCK ? bs_layout(n, b, a, r).total : wd_layout(n, b, a).total;
+    if (!workspace || workspace_bytes < need) algo = partial ? SOLVE_LOOP : SOLVE_SWEEP;
+  }
   if (algo == SOLVE_BLOCK) {
     if (!workspace || workspace_bytes < bs_layout(n, b, a, r).total) return ROCBTA_ERR_WORKSPACE;
     return pobtas_block(n, b, a, D, L, R, T, B, r, ldb, trans == 'N' ? 0 : 1, partial,
