@@ -91,9 +91,15 @@ int rocbta_dpobtasi(int64_t n, int64_t b, int64_t a, double* D, double* L, doubl
  * Replaces serinv.algs.pobtas / _pobtas (src/serinv/algs/pobtas.py:10-62,
  * 65-161) and, with a == 0, serinv.algs.pobts / _pobts (pobts.py:10-118).
  * partial = 1 skips the last-block and tip solves (pobtas.py:99,129).
- * With partial = 0 the solve runs as one persistent kernel per call; the
- * first int32 of the workspace then holds 0, or -1 if that kernel hit its
- * internal scheduling time-out (the contents of B are then undefined). */
+ * The sweep is one persistent kernel per call (per group of columns where there
+ * are many), or, for partial solves of small blocks or of more than 8 columns,
+ * launches per tile.  The first int32 of the workspace, if there is one, then
+ * holds 0, or -1 if a persistent kernel hit its internal scheduling time-out
+ * (the contents of B are then undefined).  The workspace of
+ * rocbta_workspace_bytes(ROCBTA_OP_POBTAS, n, b, a, r) also serves fewer
+ * columns (for b >= 256 and r > 8: down to 9).  For b < 256 a call with a
+ * smaller one, or with none for a partial solve, runs in a slower form that
+ * fits it, if there is one. */
 int rocbta_dpobtas(int64_t n, int64_t b, int64_t a, const double* D, const double* L,
                    const double* R, const double* T, double* B, int64_t r, int64_t ldb,
                    char trans, int partial, void* workspace, size_t workspace_bytes,
@@ -174,8 +180,9 @@ int rocbta_dquad(int64_t rows, int64_t r, const double* y, const double* x, int6
  * ROCBTA_BATCHED_RC1 / _RC4 / _RC8 force the solve sweeps' column-chunk
  * width (right-hand-side columns per chain workgroup; default: 1 for r = 1,
  * 4 for r <= 4, else 8), ROCBTA_BATCHED_GEMM512 runs every selected-inversion
- * GEMM phase on 32x32 tiles (512 threads, the K range split over the eight
- * waves; default: phases of many tiles take 64x64 ones). */
+ * GEMM phase without in-place products on 32x32 tiles (512 threads, the K
+ * range split over the eight waves; default: phases of many tiles take 64x64
+ * ones, as in-place products always do). */
 #define ROCBTA_BATCHED_RC1 16
 #define ROCBTA_BATCHED_RC4 32
 #define ROCBTA_BATCHED_RC8 64

@@ -26,12 +26,14 @@
 // PD(g) (stage g-1) and PX(g) (stage g), so no wait can cycle.  Every wait is
 // bounded: an overrun sets info = -1 and makes all later waits return.
 //
-// Memory ordering: helpers publish a tile with an agent-scope release before
-// the flag store.  The chain's tiles are written through (agent-scope stores),
-// each wave adding its share to the flag once its own stores are complete: no
-// barrier and no cache write-back on the chain's path.  A tile is ready when
-// its flag holds CH_READY; waiters poll relaxed and issue one agent-scope
-// acquire.
+// Memory ordering: the helpers' TRSM, ARR, PX and PD tiles and the chain's
+// Linv(g) are written through (agent-scope stores), each wave adding its share
+// to the flag once its own stores are complete: no barrier and no cache
+// write-back between a tile and its readers.  The chain's L(g+1,g) uses plain
+// stores, whose issue does not hold a wave up, and one release by wave 3 at the
+// start of the next step; TIPP and TIP are published behind a barrier and one
+// release (chain_publish).  A tile is ready when its flag holds CH_READY;
+// waiters poll relaxed and issue one agent-scope acquire.
 #pragma once
 #include "common.hpp"
 #include "tile_f64.hpp"

@@ -1,5 +1,6 @@
 // Block-level persistent triangular sweep with the BTA block Cholesky factor
-// (pobtas) on gfx950, for large diagonal blocks.
+// (pobtas) on gfx950, for few right-hand sides: any large diagonal block, and
+// smaller ones where its inverses pay.
 //
 // Reference recurrence: src/serinv/algs/pobtas.py:80-126 (forward,
 // y = L^{-1} B) and :127-159 (backward, x = L^{-T} y).  With the inverses
