@@ -163,8 +163,9 @@ __device__ __forceinline__ void frag_load(const GStream& st, int k0, GFrag& f) {
 // Even lanes keep x and get y from the odd neighbour's x; odd lanes keep y and
 // get x from the even neighbour's y.  One select per 32 bits, which takes one of
 // its operands from the other lane (as a lane read and a select each, B
-// transposed took 600 us); the wait states in front of a DPP read are written
-// out, since the compiler does not track them into an asm statement.
+// transposed took 600 us); the wait states in front of a DPP read, and of an
+// MFMA that reads the result, are written out, since the compiler does not track
+// them into and out of an asm statement.
 #define ROCBTA_SEL(d, n, o, q) \
   "v_cndmask_b32_dpp " d ", " n ", " o ", vcc quad_perm:[" q "] row_mask:0xf bank_mask:0xf\n\t"
 __device__ __forceinline__ void pair_trade(double& x0, double& x1, double& y0, double& y1) {
@@ -179,14 +180,14 @@ __device__ __forceinline__ void pair_trade(double& x0, double& x1, double& y0, d
   }
   asm("s_mov_b64 vcc, %12\n\ts_nop 0\n\t" ROCBTA_SEL("%0", "%4", "%8", "0,0,2,2")
           ROCBTA_SEL("%1", "%5", "%9", "0,0,2,2") ROCBTA_SEL("%2", "%6", "%10", "0,0,2,2")
-              ROCBTA_SEL("%3", "%7", "%11", "0,0,2,2")
+              ROCBTA_SEL("%3", "%7", "%11", "0,0,2,2") "s_nop 1"
       : "=&v"(a[0]), "=&v"(a[1]), "=&v"(a[2]), "=&v"(a[3])
       : "v"(y[0]), "v"(y[1]), "v"(y[2]), "v"(y[3]), "v"(x[0]), "v"(x[1]), "v"(x[2]), "v"(x[3]),
         "s"(even)
       : "vcc");
   asm("s_mov_b64 vcc, %8\n\ts_nop 0\n\t" ROCBTA_SEL("%0", "%4", "%0", "1,1,3,3")
           ROCBTA_SEL("%1", "%5", "%1", "1,1,3,3") ROCBTA_SEL("%2", "%6", "%2", "1,1,3,3")
-              ROCBTA_SEL("%3", "%7", "%3", "1,1,3,3")
+              ROCBTA_SEL("%3", "%7", "%3", "1,1,3,3") "s_nop 1"
       : "+&v"(y[0]), "+&v"(y[1]), "+&v"(y[2]), "+&v"(y[3])
       : "v"(x[0]), "v"(x[1]), "v"(x[2]), "v"(x[3]), "s"(~even)
       : "vcc");
